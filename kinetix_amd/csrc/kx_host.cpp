@@ -47,6 +47,8 @@ struct Mech {
   std::map<std::string, hipFunction_t> fn;
   std::map<std::string, unsigned> block;     // each kernel's launch bound (threads per block)
   std::map<std::string, int> lanes;          // lanes per state of kernels that share a state
+  std::map<std::string, int> wave_states;    // states per wavefront of the kernels that loop over
+  std::map<std::string, long long> resident;  // state groups, and their workgroups resident at once
   int queue_lanes = 1;                        // lanes per queued state of kx_bk2_fp64_queue
   long long queue_grid_cap = 0;               // its workgroups resident at once (strided form)
   int n_species = 0, n_active = 0, n_reactions = 0;
@@ -133,6 +135,14 @@ int launch(Mech* m, const char* name, long long n_lanes, void* stream, void** ar
   const unsigned block = m->block.at(name);
   auto l = m->lanes.find(name);
   if (l != m->lanes.end()) n_lanes *= l->second;
+  auto ws = m->wave_states.find(name);
+  if (ws != m->wave_states.end()) {
+    // a workgroup per group of states up to those resident at once; the kernel loops
+    const long long groups = (n_lanes + ws->second - 1) / ws->second;
+    KX_HIP(hipModuleLaunchKernel(it->second, (unsigned)std::min(groups, m->resident.at(name)), 1, 1,
+                                 block, 1, 1, 0, (hipStream_t)stream, args, nullptr));
+    return KX_OK;
+  }
   const long long g = (n_lanes + (long long)block - 1) / block;
   if (g > 0x7fffffffLL) return fail(KX_ERR_INVALID_ARG, "grid too large");
   const unsigned grid = (unsigned)g;
@@ -171,6 +181,20 @@ int check_layout(Mech* m, int n, int offsetT, int offset, const void* a, const v
 extern "C" {
 
 const char* kx_last_error(void) { return g_err.c_str(); }
+
+// Workgroups of f (block threads, static LDS) that the device holds at once.
+static long long resident_workgroups(Mech* m, hipFunction_t f, int block)
+{
+  int ncu = 0, per_cu = 0;
+  if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, m->device) != hipSuccess ||
+      ncu <= 0)
+    ncu = 1;
+  if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, f, block, 0) != hipSuccess ||
+      per_cu <= 0)
+    per_cu = 1;
+  (void)hipGetLastError();
+  return (long long)ncu * per_cu;
+}
 
 // Registers the module's kernels with their launch bounds and publishes the handle; takes
 // ownership of m (deleted on failure).
@@ -213,6 +237,22 @@ static int finish_init(Mech* m, kx_mech_t* out)
     } else {
       (void)hipGetLastError();
     }
+    // a kernel whose wavefronts loop over groups of states exports the group's size
+    if (hipModuleGetGlobal(&lp, &lbytes, m->module, (std::string(k) + "_states_per_wave").c_str()) ==
+            hipSuccess &&
+        lbytes == sizeof(int)) {
+      int ws = 0;
+      if (hipMemcpyDtoH(&ws, lp, sizeof(int)) != hipSuccess || ws < 1) {
+        (void)hipGetLastError();
+        (void)hipModuleUnload(m->module);
+        delete m;
+        return fail(KX_ERR_HIP, std::string("unusable states per wave for ") + k);
+      }
+      m->wave_states[k] = ws;
+      m->resident[k] = resident_workgroups(m, f, bound);
+    } else {
+      (void)hipGetLastError();
+    }
   }
   // the queue kernel may share each state among several lanes; it then exports how many
   {
@@ -230,16 +270,8 @@ static int finish_init(Mech* m, kx_mech_t* out)
       }
       m->queue_lanes = lanes;
       // the strided queue kernel runs on a grid capped at the workgroups resident at once
-      int ncu = 0, per_cu = 0;
-      if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, m->device) !=
-              hipSuccess || ncu <= 0)
-        ncu = 1;
-      if (hipModuleOccupancyMaxActiveBlocksPerMultiprocessor(
-              &per_cu, m->fn["kx_bk2_fp64_queue"], (int)m->block["kx_bk2_fp64_queue"], 0) !=
-              hipSuccess || per_cu <= 0)
-        per_cu = 1;
-      (void)hipGetLastError();
-      m->queue_grid_cap = (long long)ncu * per_cu;
+      m->queue_grid_cap = resident_workgroups(m, m->fn["kx_bk2_fp64_queue"],
+                                              (int)m->block["kx_bk2_fp64_queue"]);
     } else {
       (void)hipGetLastError();
     }
@@ -619,7 +651,7 @@ int kx_sur_transport(kx_mech_t h, int n, int offsetT, int offset, const double* 
                     (void*)&d_p,
                     (void*)&d_state, &d_cond, &d_visc, &d_rhoD, &d_Dkm, &Tref};
     const long long longest = (long long)n_audit + n;
-    if (m->queue_lanes > 1) {
+    if (m->queue_lanes > 1 && !m->wave_states.count("kx_bk2_fp64_queue")) {
       // the cooperative form strides over the queue: a grid of the workgroups resident at
       // once, or fewer when even the longest possible queue needs fewer
       const long long per_wg = m->block.at("kx_bk2_fp64_queue") / m->queue_lanes;

@@ -1,10 +1,13 @@
-"""The surrogate's plain pass, cooperative: kx_bk2_fp64_queue with several lanes per state.
+"""The surrogate's plain pass, cooperative: kx_bk2_fp64_queue with several lanes per state, for
+mechanisms whose plain transport kernel runs one state per lane (emit_bk2_quad.fits says which
+do not): the pass evaluates the same polynomials in ln T as that kernel, so that the states it
+recomputes equal the plain kernel's to rounding.
 
 kx_sur_transport runs the plain FP64 transport kernel over a queue of state ids -- the 1 %
 audit samples, then the out-of-hull states -- reading each state in place and writing its
 results over the surrogate's. A few 10^4 states cannot fill the GPU one state per lane: that
 pass lasts one full BK2 lane program (~47k instructions) at one wavefront per SIMD, ~0.37 ms
-with the rho*D audit, whatever the count. Here LPS = 16 lanes share a state, each taking the
+with the rho*D audit, whatever the count. Here 16 lanes share a state, each taking the
 species rows k = q, q + 16, ... of every row-wise sum:
 
   * mole fractions and eta_k (species-parallel, group sums by xor shuffles), x_k and 1/eta_k
@@ -37,10 +40,12 @@ from __future__ import annotations
 
 import numpy as np
 
+from . import emit_bk2_quad
 from . import emit_hip as E
 from . import emit_rolled as RL
 
-LPS = 16
+LPS = emit_bk2_quad.LPS      # of the mechanisms whose transport runs four lanes per state
+COOP_LPS = 16                # of this module's kernel
 BLOCK = 1024
 
 
@@ -58,12 +63,12 @@ def tables(t):
     return tri, np.asarray(t['C1'], np.float64), np.asarray(t['C2'], np.float64), sp
 
 
-def lds_bytes(t, lps=LPS, block=BLOCK):
+def lds_bytes(t, lps=COOP_LPS, block=BLOCK):
     N = int(t['n_species'])
     return 8 * (5 * N * (N - 1) // 2 + 2 * N * N + 12 * N + 2 * N * (block // lps))
 
 
-def emit(t, info, lps=LPS, block=BLOCK, unroll=8):
+def emit(t, info, lps=COOP_LPS, block=BLOCK, unroll=8):
     N = int(t['n_species'])
     if block % lps or 64 % lps:
         raise ValueError('lanes per state must divide the wavefront and the workgroup')

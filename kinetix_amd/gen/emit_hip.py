@@ -1119,7 +1119,10 @@ def generate(tables, info, opts=None):
     else:
         parts.append(_with_pool('kx_bk1_fp64_k', _emit_bk1_fp64, tables, info, o['bk1_sched_window'],
                                 o['bk1_wform'], lds=o['lds_pool']))
-    if 'cond' in tables:
+    from . import emit_bk2_quad as QD
+    if 'cond' in tables and QD.fits(tables):
+        parts.append(QD.emit(tables, info))
+    elif 'cond' in tables:
         parts.append(_with_pool('kx_bk2_fp64_k', _emit_bk2_fp64, tables, info, False, o['bk2_block'],
                                 lds=o['lds_pool'], block=o['bk2_block']))
         parts.append(_with_pool('kx_bk2_fp64_pstate_k', _emit_bk2_fp64, tables, info, True, o['bk2_block'],
