@@ -54,66 +54,219 @@ __device__ __forceinline__ uint16_t to_bf16(float f)
   return (uint16_t)(u >> 16);
 }
 
-// C[MxN] = alpha * op(A) op(B) + beta * C, row-major; op(A) is MxK (A or A^T stored KxM),
-// op(B) is KxN (B or B^T stored NxK). M, N multiples of 64, K multiple of 16.
-template <bool TA, bool TB>
-__global__ void __launch_bounds__(256) gemm_f32(int M, int N, int K, float alpha,
-                                                const float* __restrict__ A, int lda,
-                                                const float* __restrict__ B, int ldb, float beta,
-                                                float* __restrict__ C, int ldc)
+// ---- training GEMMs on FP32 MFMA (v_mfma_f32_32x32x2_f32, 16x16x4): full FP32 products and sums
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4t __attribute__((ext_vector_type(4)));
+typedef float f32x2t __attribute__((ext_vector_type(2)));
+
+// What a GEMM tile does with its result c at (row, col):
+//   BIAS_GELU  Z = c + bias[col], H = gelu(Z)          (hidden layer forward)
+//   BIAS       Z = c + bias[col]                       (output layer forward)
+//   GELU_BACK  Z = c * gelu'(Zin)                      (gradient before the activation)
+enum Epilogue { BIAS_GELU, BIAS, GELU_BACK };
+
+struct GemmArgs {
+  const float* A;      // M x K row-major
+  const float* B;      // N x K (forward: W) or, transposed, K x N (backward: W again)
+  int N, K;
+  const float* bias;   // N, or null
+  const float* Zin;    // M x N, GELU_BACK
+  float* Z;            // M x N
+  float* H;            // M x N, BIAS_GELU
+};
+
+// One (32 WM) x (32 WN) tile of C = A op(B)^T: WM x WN wavefronts of 32 x 32. K runs in chunks of 32
+// staged in LDS as [row][k] (rows padded to 36 floats: 16 B reads without bank conflicts),
+// the next chunk's global loads in flight during the products. A lane's 16 B hold k = 8 q + 4 h
+// .. + 3 (h = lane / 32), so product e of the four takes k = 8 q + e and 8 q + 4 + e from the
+// two halves: the same permutation of k in A and B.
+constexpr int kBK = 32, kLd = kBK + 4;
+template <int WM, int WN>
+constexpr int gemm_lds() { return 32 * (WM + WN) * kLd; }
+
+template <int WM, int WN, bool TB, Epilogue EPI>
+__device__ __forceinline__ void gemm_tile(const GemmArgs& g, int tm, int tn, float* lds)
 {
-  __shared__ float As[16][68];
-  __shared__ float Bs[16][68];
-  const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-  const int m0 = blockIdx.y * 64, n0 = blockIdx.x * 64;
-  float acc[4][4] = {};
-  for (int k0 = 0; k0 < K; k0 += 16) {
-    for (int e = threadIdx.x; e < 1024; e += 256) {
-      if (!TA) { const int mm = e >> 4, kk = e & 15; As[kk][mm] = A[(size_t)(m0 + mm) * lda + k0 + kk]; }
-      else     { const int kk = e >> 6, mm = e & 63; As[kk][mm] = A[(size_t)(k0 + kk) * lda + m0 + mm]; }
-      if (!TB) { const int kk = e >> 6, nn = e & 63; Bs[kk][nn] = B[(size_t)(k0 + kk) * ldb + n0 + nn]; }
-      else     { const int nn = e >> 4, kk = e & 15; Bs[kk][nn] = B[(size_t)(n0 + nn) * ldb + k0 + kk]; }
+  constexpr int TH = 64 * WM * WN, MT = 32 * WM, NT = 32 * WN;
+  constexpr int LA = MT * kBK / 4 / TH, LB = NT * kBK / 4 / TH;
+  static_assert(LA >= 1 && LB >= 1 && MT * kBK / 4 % TH == 0 && NT * kBK / 4 % TH == 0, "whole loads");
+  float* As = lds;                 // [MT][kLd]
+  float* Bs = lds + MT * kLd;      // [NT][kLd]
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane & 31, h = lane >> 5;
+  const int wm = w / WN, wn = w % WN, m0 = tm * MT, n0 = tn * NT;
+  f32x4t ra[LA], rb[LB];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int r = 0; r < LA; ++r) {
+      const int e = threadIdx.x + r * TH;
+      ra[r] = *(const f32x4t*)(g.A + (size_t)(m0 + e / (kBK / 4)) * g.K + k0 + 4 * (e % (kBK / 4)));
     }
-    __syncthreads();
 #pragma unroll
-    for (int kk = 0; kk < 16; ++kk) {
-      float a[4], b[4];
-#pragma unroll
-      for (int i = 0; i < 4; ++i) { a[i] = As[kk][ty * 4 + i]; b[i] = Bs[kk][tx * 4 + i]; }
-#pragma unroll
-      for (int i = 0; i < 4; ++i)
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[i][j] = fmaf(a[i], b[j], acc[i][j]);
+    for (int r = 0; r < LB; ++r) {
+      const int e = threadIdx.x + r * TH;
+      if (TB) rb[r] = *(const f32x4t*)(g.B + (size_t)(k0 + e / (NT / 4)) * g.N + n0 + 4 * (e % (NT / 4)));
+      else rb[r] = *(const f32x4t*)(g.B + (size_t)(n0 + e / (kBK / 4)) * g.K + k0 + 4 * (e % (kBK / 4)));
     }
+  };
+  auto store = [&]() {
+#pragma unroll
+    for (int r = 0; r < LA; ++r) {
+      const int e = threadIdx.x + r * TH;
+      *(f32x4t*)(As + (e / (kBK / 4)) * kLd + 4 * (e % (kBK / 4))) = ra[r];
+    }
+#pragma unroll
+    for (int r = 0; r < LB; ++r) {
+      const int e = threadIdx.x + r * TH;
+      if (TB) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) Bs[(4 * (e % (NT / 4)) + q) * kLd + e / (NT / 4)] = rb[r][q];
+      } else {
+        *(f32x4t*)(Bs + (e / (kBK / 4)) * kLd + 4 * (e % (kBK / 4))) = rb[r];
+      }
+    }
+  };
+  f32x16 acc = {};
+  load(0);
+  for (int k0 = 0; k0 < g.K; k0 += kBK) {
     __syncthreads();
+    store();
+    __syncthreads();
+    if (k0 + kBK < g.K) load(k0 + kBK);
+#pragma unroll
+    for (int q = 0; q < kBK / 8; ++q) {
+      const f32x4t a = *(const f32x4t*)(As + (32 * wm + i) * kLd + 8 * q + 4 * h);
+      const f32x4t b = *(const f32x4t*)(Bs + (32 * wn + i) * kLd + 8 * q + 4 * h);
+#pragma unroll
+      for (int e = 0; e < 4; ++e) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], acc, 0, 0, 0);
+    }
   }
+  // element r of a lane: row 8 (r / 4) + 4 h + r % 4, column i
+  const int col = n0 + 32 * wn + i;
+  const float bias = EPI != GELU_BACK ? g.bias[col] : 0.0f;
 #pragma unroll
-  for (int i = 0; i < 4; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-      float* c = &C[(size_t)(m0 + ty * 4 + i) * ldc + n0 + tx * 4 + j];
-      *c = alpha * acc[i][j] + (beta != 0.0f ? beta * *c : 0.0f);
+  for (int r = 0; r < 16; ++r) {
+    const size_t o = (size_t)(m0 + 32 * wm + 8 * (r >> 2) + 4 * h + (r & 3)) * g.N + col;
+    if (EPI == GELU_BACK) {
+      g.Z[o] = acc[r] * gelu_grad(g.Zin[o]);
+    } else {
+      const float z = acc[r] + bias;
+      g.Z[o] = z;
+      if (EPI == BIAS_GELU) g.H[o] = gelu(z);
     }
+  }
 }
 
-// Z[M][N] += b[N]; H = gelu(Z) if H != nullptr
-__global__ void __launch_bounds__(256) bias_act(int M, int N, float* __restrict__ Z,
-                                                const float* __restrict__ b, float* __restrict__ H)
+template <int WM, int WN, Epilogue EPI>
+__global__ void __launch_bounds__(64 * WM * WN) gemm_forward(GemmArgs g)
 {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)M * N) return;
-  const float z = Z[i] + b[i % N];
-  Z[i] = z;
-  if (H) H[i] = gelu(z);
+  __shared__ __attribute__((aligned(16))) float lds[gemm_lds<WM, WN>()];
+  gemm_tile<WM, WN, false, EPI>(g, blockIdx.y, blockIdx.x, lds);
 }
 
-// dZ = dH * gelu'(Z)
-__global__ void __launch_bounds__(256) gelu_back(int M, int N, const float* __restrict__ dH,
-                                                 const float* __restrict__ Z, float* __restrict__ dZ)
+// Weight gradient of one layer, dW[m][n] = sum_b dZ[b][m] X[b][n], db[m] = sum_b dZ[b][m].
+struct GradArgs {
+  const float* dZ;     // batch x M
+  const float* X;      // batch x N
+  int batch, M, N;
+  float* dW;           // M x N
+  float* db;           // M
+};
+
+// A (16 RM) x 16 tile of dW per workgroup, the batch split over its WAVES wavefronts and summed in
+// wavefront order through LDS: deterministic, and no workspace beyond the caller's. The
+// operands are read in MFMA layout straight from memory (lane l: row l / 16 of four, RM
+// consecutive columns from RM (l % 16)), 8 steps of 4 rows in flight. Tiles of column 0 add up db.
+template <int RM, int WAVES>
+constexpr int grad_lds() { return WAVES * 64 * (4 * RM + RM); }
+
+template <int RM, int WAVES>
+__device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* lds)
 {
-  const size_t i = (size_t)blockIdx.x * 256 + threadIdx.x;
-  if (i >= (size_t)M * N) return;
-  dZ[i] = dH[i] * gelu_grad(Z[i]);
+  typedef float vec __attribute__((ext_vector_type(RM)));
+  constexpr int U = 8;
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane & 15, q = lane >> 4;
+  const int tn = g.N / 16, m0 = (tile / tn) * 16 * RM, n0 = (tile % tn) * 16;
+  const int steps = g.batch / (4 * WAVES);                      // per wavefront
+  const float* a = g.dZ + (size_t)(4 * steps * w + q) * g.M + m0 + RM * i;
+  const float* b = g.X + (size_t)(4 * steps * w + q) * g.N + n0 + i;
+  f32x4t acc[RM];
+  vec bs;
+#pragma unroll
+  for (int e = 0; e < RM; ++e) { acc[e] = (f32x4t){0.f, 0.f, 0.f, 0.f}; bs[e] = 0.f; }
+  int s = 0;
+  vec va[U];
+  float vb[U];
+  auto load = [&](int at) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      va[u] = *(const vec*)(a + (size_t)4 * (at + u) * g.M);
+      vb[u] = b[(size_t)4 * (at + u) * g.N];
+    }
+  };
+  auto products = [&]() {
+#pragma unroll
+    for (int u = 0; u < U; ++u)
+#pragma unroll
+      for (int e = 0; e < RM; ++e) {
+        acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u][e], vb[u], acc[e], 0, 0, 0);
+        bs[e] += va[u][e];
+      }
+  };
+  for (; s + U <= steps; s += U) { load(s); products(); }
+  for (; s < steps; ++s) {
+    const vec ta = *(const vec*)(a + (size_t)4 * s * g.M);
+    const float tb = b[(size_t)4 * s * g.N];
+#pragma unroll
+    for (int e = 0; e < RM; ++e) {
+      acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[e], tb, acc[e], 0, 0, 0);
+      bs[e] += ta[e];
+    }
+  }
+  float* red = lds;                               // [wave][RM * 4][64]
+  float* redb = lds + WAVES * 64 * 4 * RM;        // [wave][RM][64]
+#pragma unroll
+  for (int e = 0; e < RM; ++e) {
+#pragma unroll
+    for (int r = 0; r < 4; ++r) red[(w * 4 * RM + 4 * e + r) * 64 + lane] = acc[e][r];
+    redb[(w * RM + e) * 64 + lane] = bs[e];
+  }
+  __syncthreads();
+  for (int t = threadIdx.x; t < 256 * RM; t += 64 * WAVES) {
+    float v = 0.0f;
+    for (int k = 0; k < WAVES; ++k) v += red[k * 256 * RM + t];
+    const int l = t & 63, e = t >> 8, r = (t >> 6) & 3;        // element r of lane l, block e
+    g.dW[(size_t)(m0 + RM * (4 * (l >> 4) + r) + e) * g.N + n0 + (l & 15)] = v;
+  }
+  if (n0 == 0 && threadIdx.x < 16 * RM) {
+    const int e = threadIdx.x >> 4, c = threadIdx.x & 15;
+    float v = 0.0f;
+    for (int k = 0; k < WAVES; ++k)
+      for (int r = 0; r < 4; ++r) v += redb[(k * RM + e) * 64 + 16 * r + c];
+    g.db[m0 + RM * c + e] = v;
+  }
+}
+
+// One layer backwards in one launch: the first n_grad workgroups take tiles of its weight
+// gradient, the others tiles of the gradient handed to the layer below (dZ W * gelu'). The
+// long batch sums start first and share the chip with the other product.
+constexpr int kWN = kH % 128 ? 2 : 4;            // hidden-layer tiles: 64 rows x 32 kWN columns
+constexpr int kTileWaves = 2 * kWN;
+
+template <int RM>
+__global__ void __launch_bounds__(64 * kTileWaves) layer_backward(GradArgs gr, GemmArgs ge, int n_grad, int tiles_n)
+{
+  constexpr int L0 = grad_lds<RM, kTileWaves>(), L1 = gemm_lds<2, kWN>();
+  __shared__ __attribute__((aligned(16))) float lds[L0 > L1 ? L0 : L1];
+  const int b = blockIdx.x;
+  if (b < n_grad) grad_tile<RM, kTileWaves>(gr, b, lds);
+  else gemm_tile<2, kWN, true, GELU_BACK>(ge, (b - n_grad) / tiles_n, (b - n_grad) % tiles_n, lds);
+}
+
+template <int RM, int WAVES>
+__global__ void __launch_bounds__(64 * WAVES) layer_grad(GradArgs gr)
+{
+  __shared__ float lds[grad_lds<RM, WAVES>()];
+  grad_tile<RM, WAVES>(gr, blockIdx.x, lds);
 }
 
 // dY = 2 (Y - T) / (M * valid) on the first `valid` columns, 0 on the padding; per-block
@@ -138,23 +291,6 @@ __global__ void __launch_bounds__(256) mse_grad(int M, int N, int valid, const f
     __syncthreads();
   }
   if (threadIdx.x == 0) part[blockIdx.x] = red[0];
-}
-
-// db[j] = sum_i dZ[i][j]  (one workgroup per column, fixed summation order)
-__global__ void __launch_bounds__(256) bias_grad(int M, int N, const float* __restrict__ dZ,
-                                                 float* __restrict__ db)
-{
-  __shared__ float red[256];
-  const int j = blockIdx.x;
-  float s = 0.0f;
-  for (int i = threadIdx.x; i < M; i += 256) s += dZ[(size_t)i * N + j];
-  red[threadIdx.x] = s;
-  __syncthreads();
-  for (int w = 128; w > 0; w >>= 1) {
-    if (threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
-    __syncthreads();
-  }
-  if (threadIdx.x == 0) db[j] = red[0];
 }
 
 __global__ void __launch_bounds__(256) adam(int n, float* __restrict__ w, const float* __restrict__ g,
@@ -293,15 +429,13 @@ int kx_mlp_forward(const float* p, int B, const float* X, float* acts, void* str
   hipStream_t s = (hipStream_t)stream;
   const size_t L = (size_t)B * kH;
   float *Z1 = acts, *H1 = Z1 + L, *Z2 = H1 + L, *H2 = Z2 + L, *Z3 = H2 + L, *H3 = Z3 + L, *Yo = H3 + L;
-  const dim3 gH(kH / 64, B / 64), gO(kOut / 64, B / 64);
-  hipLaunchKernelGGL((gemm_f32<false, true>), gH, dim3(256), 0, s, B, kH, kIn, 1.f, X, kIn, p + kW1, kIn, 0.f, Z1, kH);
-  hipLaunchKernelGGL(bias_act, dim3(grid1(L)), dim3(256), 0, s, B, kH, Z1, p + kB1, H1);
-  hipLaunchKernelGGL((gemm_f32<false, true>), gH, dim3(256), 0, s, B, kH, kH, 1.f, H1, kH, p + kW2, kH, 0.f, Z2, kH);
-  hipLaunchKernelGGL(bias_act, dim3(grid1(L)), dim3(256), 0, s, B, kH, Z2, p + kB2, H2);
-  hipLaunchKernelGGL((gemm_f32<false, true>), gH, dim3(256), 0, s, B, kH, kH, 1.f, H2, kH, p + kW3, kH, 0.f, Z3, kH);
-  hipLaunchKernelGGL(bias_act, dim3(grid1(L)), dim3(256), 0, s, B, kH, Z3, p + kB3, H3);
-  hipLaunchKernelGGL((gemm_f32<false, true>), gO, dim3(256), 0, s, B, kOut, kH, 1.f, H3, kH, p + kW4, kH, 0.f, Yo, kOut);
-  hipLaunchKernelGGL(bias_act, dim3(grid1((size_t)B * kOut)), dim3(256), 0, s, B, kOut, Yo, p + kB4, (float*)nullptr);
+  const dim3 gH(kH / (32 * kWN), B / 64), bH(64 * kTileWaves), gO(kOut / 64, B / 64);
+  const GemmArgs l1{X, p + kW1, kH, kIn, p + kB1, nullptr, Z1, H1}, l2{H1, p + kW2, kH, kH, p + kB2, nullptr, Z2, H2};
+  const GemmArgs l3{H2, p + kW3, kH, kH, p + kB3, nullptr, Z3, H3}, l4{H3, p + kW4, kOut, kH, p + kB4, nullptr, Yo, nullptr};
+  hipLaunchKernelGGL((gemm_forward<2, kWN, BIAS_GELU>), gH, bH, 0, s, l1);
+  hipLaunchKernelGGL((gemm_forward<2, kWN, BIAS_GELU>), gH, bH, 0, s, l2);
+  hipLaunchKernelGGL((gemm_forward<2, kWN, BIAS_GELU>), gH, bH, 0, s, l3);
+  hipLaunchKernelGGL((gemm_forward<2, 2, BIAS>), gO, dim3(256), 0, s, l4);
   return hip_status();
 }
 
@@ -315,27 +449,22 @@ int kx_mlp_backward(const float* p, int B, const float* X, const float* acts, co
   hipStream_t s = (hipStream_t)stream;
   const size_t L = (size_t)B * kH;
   const float *Z1 = acts, *H1 = Z1 + L, *Z2 = H1 + L, *H2 = Z2 + L, *Z3 = H2 + L, *H3 = Z3 + L, *Yo = H3 + L;
-  float *dA = work, *dB = work + L;       // dH / dZ scratch (B x kH each)
+  float *dA = work, *dB = work + L;       // dZ of alternate layers (B x kH each)
   float* dY = dB;                          // B x 64 fits in dB
   hipLaunchKernelGGL(mse_grad, dim3(grid1((size_t)B * kOut)), dim3(256), 0, s, B, kOut, kValidOut, Yo, T, dY, loss_part);
-  // layer 4: dW4 = dY^T H3, db4, dH3 = dY W4
-  hipLaunchKernelGGL((gemm_f32<true, false>), dim3(kH / 64, kOut / 64), dim3(256), 0, s, kOut, kH, B, 1.f, dY, kOut, H3, kH, 0.f, g + kW4, kH);
-  hipLaunchKernelGGL(bias_grad, dim3(kOut), dim3(256), 0, s, B, kOut, dY, g + kB4);
-  hipLaunchKernelGGL((gemm_f32<false, false>), dim3(kH / 64, B / 64), dim3(256), 0, s, B, kH, kOut, 1.f, dY, kOut, p + kW4, kH, 0.f, dA, kH);
-  // layer 3
-  hipLaunchKernelGGL(gelu_back, dim3(grid1(L)), dim3(256), 0, s, B, kH, dA, Z3, dA);
-  hipLaunchKernelGGL((gemm_f32<true, false>), dim3(kH / 64, kH / 64), dim3(256), 0, s, kH, kH, B, 1.f, dA, kH, H2, kH, 0.f, g + kW3, kH);
-  hipLaunchKernelGGL(bias_grad, dim3(kH), dim3(256), 0, s, B, kH, dA, g + kB3);
-  hipLaunchKernelGGL((gemm_f32<false, false>), dim3(kH / 64, B / 64), dim3(256), 0, s, B, kH, kH, 1.f, dA, kH, p + kW3, kH, 0.f, dB, kH);
-  // layer 2
-  hipLaunchKernelGGL(gelu_back, dim3(grid1(L)), dim3(256), 0, s, B, kH, dB, Z2, dB);
-  hipLaunchKernelGGL((gemm_f32<true, false>), dim3(kH / 64, kH / 64), dim3(256), 0, s, kH, kH, B, 1.f, dB, kH, H1, kH, 0.f, g + kW2, kH);
-  hipLaunchKernelGGL(bias_grad, dim3(kH), dim3(256), 0, s, B, kH, dB, g + kB2);
-  hipLaunchKernelGGL((gemm_f32<false, false>), dim3(kH / 64, B / 64), dim3(256), 0, s, B, kH, kH, 1.f, dB, kH, p + kW2, kH, 0.f, dA, kH);
+  // layers 4, 3, 2: the weight gradient and the gradient before the next activation down
+  const GradArgs w4{dY, H3, B, kOut, kH, g + kW4, g + kB4}, w3{dA, H2, B, kH, kH, g + kW3, g + kB3};
+  const GradArgs w2{dB, H1, B, kH, kH, g + kW2, g + kB2}, w1{dA, X, B, kH, kIn, g + kW1, g + kB1};
+  const GemmArgs x3{dY, p + kW4, kH, kOut, nullptr, Z3, dA, nullptr}, x2{dA, p + kW3, kH, kH, nullptr, Z2, dB, nullptr};
+  const GemmArgs x1{dB, p + kW2, kH, kH, nullptr, Z1, dA, nullptr};
+  constexpr int tn = kH / (32 * kWN);
+  const dim3 bH(64 * kTileWaves);
+  const int nx = (B / 64) * tn, n4 = (kOut / 16) * (kH / 16), nh = (kH / 32) * (kH / 16);
+  hipLaunchKernelGGL(layer_backward<1>, dim3(n4 + nx), bH, 0, s, w4, x3, n4, tn);
+  hipLaunchKernelGGL(layer_backward<2>, dim3(nh + nx), bH, 0, s, w3, x2, nh, tn);
+  hipLaunchKernelGGL(layer_backward<2>, dim3(nh + nx), bH, 0, s, w2, x1, nh, tn);
   // layer 1
-  hipLaunchKernelGGL(gelu_back, dim3(grid1(L)), dim3(256), 0, s, B, kH, dA, Z1, dA);
-  hipLaunchKernelGGL((gemm_f32<true, false>), dim3(kIn / 64, kH / 64), dim3(256), 0, s, kH, kIn, B, 1.f, dA, kH, X, kIn, 0.f, g + kW1, kIn);
-  hipLaunchKernelGGL(bias_grad, dim3(kH), dim3(256), 0, s, B, kH, dA, g + kB1);
+  hipLaunchKernelGGL((layer_grad<1, 16>), dim3((kH / 16) * (kIn / 16)), dim3(1024), 0, s, w1);
   return hip_status();
 }
 
