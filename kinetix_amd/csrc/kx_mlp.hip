@@ -175,7 +175,9 @@ struct GradArgs {
 // A (16 RM) x 16 tile of dW per workgroup, the batch split over its WAVES wavefronts and summed in
 // wavefront order through LDS: deterministic, and no workspace beyond the caller's. The
 // operands are read in MFMA layout straight from memory (lane l: row l / 16 of four, RM
-// consecutive columns from RM (l % 16)), 8 steps of 4 rows in flight. Tiles of column 0 add up db.
+// consecutive columns from RM (l % 16)), two batches of U steps of 4 rows in flight: the operands
+// come from other XCDs' L2s, ~2 us away (one batch of 8: 78 us for a hidden layer's launch at
+// batch 8,192, two of 16: 49). Tiles of column 0 add up db.
 template <int RM, int WAVES>
 constexpr int grad_lds() { return WAVES * 64 * (4 * RM + RM); }
 
@@ -183,7 +185,7 @@ template <int RM, int WAVES>
 __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* lds)
 {
   typedef float vec __attribute__((ext_vector_type(RM)));
-  constexpr int U = 8;
+  constexpr int U = WAVES > 8 ? 8 : 16;        // rows of 4 per batch of loads; two batches in flight
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane & 15, q = lane >> 4;
   const int tn = g.N / 16, m0 = (tile / tn) * 16 * RM, n0 = (tile % tn) * 16;
   const int steps = g.batch / (4 * WAVES);                      // per wavefront
@@ -194,16 +196,16 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
 #pragma unroll
   for (int e = 0; e < RM; ++e) { acc[e] = (f32x4t){0.f, 0.f, 0.f, 0.f}; bs[e] = 0.f; }
   int s = 0;
-  vec va[U];
-  float vb[U];
-  auto load = [&](int at) {
+  vec va[2][U];
+  float vb[2][U];
+  auto load = [&](vec (&va)[U], float (&vb)[U], int at) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       va[u] = *(const vec*)(a + (size_t)4 * (at + u) * g.M);
       vb[u] = b[(size_t)4 * (at + u) * g.N];
     }
   };
-  auto products = [&]() {
+  auto products = [&](const vec (&va)[U], const float (&vb)[U]) {
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
@@ -212,7 +214,16 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
         bs[e] += va[u][e];
       }
   };
-  for (; s + U <= steps; s += U) { load(s); products(); }
+  if (U <= steps) load(va[0], vb[0], 0);
+  for (; s + 2 * U <= steps; s += 2 * U) {
+    load(va[1], vb[1], s + U);
+    products(va[0], vb[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    if (s + 3 * U <= steps) load(va[0], vb[0], s + 2 * U);
+    products(va[1], vb[1]);
+    __builtin_amdgcn_sched_barrier(0);
+  }
+  if (s + U <= steps) { products(va[0], vb[0]); s += U; }
   for (; s < steps; ++s) {
     const vec ta = *(const vec*)(a + (size_t)4 * s * g.M);
     const float tb = b[(size_t)4 * s * g.N];
@@ -248,7 +259,9 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
 
 // One layer backwards in one launch: the first n_grad workgroups take tiles of its weight
 // gradient, the others tiles of the gradient handed to the layer below (dZ W * gelu'). The
-// long batch sums start first and share the chip with the other product.
+// long batch sums start first and share the chip with the other product. Bound: the weight
+// gradient's reads (each 32 x 16 tile reads both operands' columns over the whole batch); the
+// two products' FP32 MFMA time is 14 us of the 49.
 constexpr int kWN = kH % 128 ? 2 : 4;            // hidden-layer tiles: 64 rows x 32 kWN columns
 constexpr int kTileWaves = 2 * kWN;
 
