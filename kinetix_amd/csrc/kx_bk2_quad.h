@@ -28,9 +28,10 @@
 // (per block 68 for the MFMA, 110 for the reciprocals and sums) and ~12k of the rest are the
 // floor of this form; eight wavefronts per CU reach it. Measured against one state per lane
 // (pair constants broadcast from LDS by every wavefront): GRI-3.0, 4,194,304 states 7.30 ->
-// 3.66 ms, 1,000 states 222 -> 18.6 us; NH3Konnov_edit, 100,003 states 97 -> 61 us. At 12 and
+// 3.62 ms, 1,000 states 222 -> 18.6 us; NH3Konnov_edit, 100,003 states 97 -> 61 us. At 12 and
 // 16 wavefronts per workgroup the registers spill: 0.97 and 1.13 ms for 1,048,576 states
-// against 0.91.
+// against 0.91. With the pair rows streamed (160 species, 524,288 states): 3.07 ms against 9.14 for
+// 64-state tiles with a row per wavefront and LDS atomics; 162 registers spill, most of them once.
 //
 // The table (gen/emit_bk2_quad.py) holds the fits about t0, the middle of the fit window: the
 // same polynomials with far smaller cancelling terms than in powers of ln T.
@@ -123,20 +124,37 @@ __device__ __forceinline__ void pin(double (&S)[NB], int m)
     if (j <= m) asm volatile("" : "+v"(S[j]));
 }
 
+// f(0), f(1) .. f(N - 1) with compile-time arguments: the pair rows index register arrays, and
+// the unroller gives up on 40 of them
+template <int... I>
+struct Seq {};
+template <int N, int... I>
+struct MakeSeq : MakeSeq<N - 1, N - 1, I...> {};
+template <int... I>
+struct MakeSeq<0, I...> { typedef Seq<I...> type; };
+template <int V>
+struct Int { static constexpr int value = V; };
+template <class F, int... I>
+__device__ __forceinline__ void each(Seq<I...>, F&& f) { (f(Int<I>()), ...); }
+
 // Table offsets (doubles) for N species and Wilke factors of KR groups of four ranks; see
-// gen/emit_bk2_quad.py for the contents.
+// gen/emit_bk2_quad.py for the contents. Rows of pair blocks first (row m: 64 (m + 1) doubles of
+// A operands, 16 (m + 1) of constants), then the species part.
 template <int N, int KR>
 struct Layout {
-  static constexpr int NB = (N + 3) / 4, SG = (NB + 3) / 4, BLK = NB * (NB + 1) / 2;
-  static constexpr int kFitA = 0, kFitC = kFitA + 64 * BLK, kWilT = kFitC + 16 * BLK;
-  static constexpr int kWil = kWilT + 64 * NB * ((KR + 3) / 4), kViscA = kWil + 64 * SG * KR;
+  static constexpr int NB = (N + 3) / 4, SG = (NB + 3) / 4, RB = (KR + 3) / 4;
+  static constexpr int row(int m) { return 40 * m * (m + 1); }
+  static constexpr int kSpecies = row(NB);
+  static constexpr int kWilT = 0, kWil = kWilT + 64 * NB * RB, kViscA = kWil + 64 * SG * KR;
   static constexpr int kViscC = kViscA + 64 * SG, kCondA = kViscC + 16 * SG;
   static constexpr int kCondC = kCondA + 64 * SG, kRcpW = kCondC + 16 * SG;
   static constexpr int kW = kRcpW + 4 * NB, kSqW = kW + 4 * NB;
-  static constexpr int kSize = (kSqW + 4 * NB + 1) & ~1;
+  static constexpr int kSpeciesSize = (kSqW + 4 * NB + 1) & ~1;
+  static constexpr int kSize = kSpecies + kSpeciesSize;
+  static constexpr int kRowMax = 80 * NB;                    // the last row
 };
 
-// copy of the table to LDS by the whole workgroup, 16 B per lane, 8 loads in flight
+// copy of (part of) the table to LDS by the whole workgroup, 16 B per lane, 8 loads in flight
 template <int SIZE, int THREADS>
 __device__ __forceinline__ void stage(double* dst, const double* __restrict__ src)
 {
@@ -156,8 +174,16 @@ __device__ __forceinline__ void stage(double* dst, const double* __restrict__ sr
 // Transport of the wavefront's 16 states; lane l: state l % 16 (index id), species group
 // l / 16. store(D, rho) is called once with D_km of the lane's species 4 m + g in D[m] (all lanes;
 // the caller masks lanes without a state). Returns mu and lambda in all four lanes of a state.
-template <int N, int KR, bool RCP, class Store>
-__device__ __forceinline__ void states16(const double* tab, const double* __restrict__ state,
+//
+// STAGE > 0 (the workgroup's threads): the pair rows do not fit the LDS and are streamed through
+// two row buffers, the next row's global loads in flight during a row; every wavefront of the
+// workgroup makes the call together (one barrier per row), those without states with busy =
+// false. `rows` is then the two buffers and `grows` the table in global memory; else `rows` holds
+// every row.
+template <int N, int KR, bool RCP, int STAGE, class Store>
+__device__ __forceinline__ void states16(const double* tab, double* rows,
+                                         const double* __restrict__ grows, bool busy,
+                                         const double* __restrict__ state,
                                          long long id, long long offsetT, long long offset,
                                          double Tref, double p, double t0, double rcpR, int lane,
                                          double& mu, double& lambda, Store&& store)
@@ -170,10 +196,10 @@ __device__ __forceinline__ void states16(const double* tab, const double* __rest
   const int g = lane >> 4;
   const double T = Tref * state[id];
   double X[NB], S[NB];
-  const double* row = state + id + offsetT + g * offset;      // species 4 m + g at row + 4 m offset
+  const double* y = state + id + offsetT + g * offset;        // species 4 m + g at y + 4 m offset
 #pragma unroll
   for (int m = 0; m < NB; ++m)
-    X[m] = 4 * m + 3 < N || 4 * m + g < N ? row[4 * m * offset] : 0.0;
+    X[m] = 4 * m + 3 < N || 4 * m + g < N ? y[4 * m * offset] : 0.0;
   const double rcpT = 1.0 / T, sqrT = sqrt(T);
   const double t = log(T) - t0, tt = t * t;
   const double B = (g & 1 ? tt : t) * (g & 2 ? tt : 1.0);     // t^(g + 1)
@@ -188,20 +214,34 @@ __device__ __forceinline__ void states16(const double* tab, const double* __rest
   for (int m = 0; m < NB; ++m) { X[m] *= Mbar; S[m] = 0.0; }
 
   // ---- diffusion: S_k = sum_{j != k} x_j / D'_kj
-#pragma unroll
-  for (int m = 0; m < NB; ++m) {
+  each(typename MakeSeq<NB>::type(), [&](auto mc) __attribute__((always_inline)) {
+    constexpr int m = decltype(mc)::value;
     __builtin_amdgcn_sched_barrier(0);
+    const double* row = rows + (STAGE ? (m & 1) * L::kRowMax : L::row(m));
+    constexpr int PF = STAGE ? (L::kRowMax / 2 + STAGE - 1) / STAGE : 1;
+    f64x2 ahead[PF];
+    constexpr int n_ahead = 40 * (m + 2);                        // 16 B pieces of row m + 1
+    if (STAGE) {
+      __syncthreads();                   // row m written; the other buffer's row read by all
+      if (m + 1 < NB) {
+#pragma unroll
+        for (int r = 0; r < PF; ++r)
+          if (r * STAGE < n_ahead)
+            ahead[r] = ((const f64x2*)(grows + L::row(m + 1)))[min((int)threadIdx.x + r * STAGE, n_ahead - 1)];
+      }
+    }
+    if (!STAGE || busy) {
     double xk[4], q[4] = {0.0, 0.0, 0.0, 0.0};
     bcast4(X[m], xk);
 #pragma unroll
     for (int j = 0; j <= m; j += 2) {
-      const int b = m * (m + 1) / 2 + j;
+      if (STAGE) __builtin_amdgcn_sched_barrier(0);            // 160 registers hold X and S
       const bool two = j < m;                                  // blocks (m, j) and (m, j + 1)
-      f64x4 d0 = *(const f64x4*)(tab + L::kFitC + 16 * b + 4 * g), d1 = {1.0, 1.0, 1.0, 1.0};
-      d0 = mfma(tab[L::kFitA + 64 * b + lane], B, d0);
+      f64x4 d0 = *(const f64x4*)(row + 64 * (m + 1) + 16 * j + 4 * g), d1 = {1.0, 1.0, 1.0, 1.0};
+      d0 = mfma(row[64 * j + lane], B, d0);
       if (two) {
-        d1 = *(const f64x4*)(tab + L::kFitC + 16 * (b + 1) + 4 * g);
-        d1 = mfma(tab[L::kFitA + 64 * (b + 1) + lane], B, d1);
+        d1 = *(const f64x4*)(row + 64 * (m + 1) + 16 * (j + 1) + 4 * g);
+        d1 = mfma(row[64 * (j + 1) + lane], B, d1);
       }
       double r0[4] = {d0[0], d0[1], d0[2], d0[3]}, r1[4] = {d1[0], d1[1], d1[2], d1[3]};
       if (!RCP) {
@@ -229,7 +269,15 @@ __device__ __forceinline__ void states16(const double* tab, const double* __rest
     }
     if (m) S[m] += reduce_scatter4(q);
     pin<NB>(S, m);
-  }
+    }
+    if (STAGE && m + 1 < NB) {
+      f64x2* next = (f64x2*)(rows + ((m + 1) & 1) * L::kRowMax);
+#pragma unroll
+      for (int r = 0; r < PF; ++r)
+        if (r * STAGE < n_ahead && (int)threadIdx.x + r * STAGE < n_ahead) next[threadIdx.x + r * STAGE] = ahead[r];
+    }
+  });
+  if (STAGE && !busy) return;
   __builtin_amdgcn_sched_barrier(0);
   const double TsqrT = T * sqrT, rho = p * rcpR * rcpT * Mbar, pMbar = p * Mbar;
 #pragma unroll
@@ -262,7 +310,7 @@ __device__ __forceinline__ void states16(const double* tab, const double* __rest
   lambda = sqrT * (0.5 * (s1 + 1.0 / s2));
 
   // ---- viscosity (Wilke): z = L^T (a, a u, a u^2), element e of a lane: rank 16 h + 4 e + g
-  constexpr int RB = (KR + 3) / 4;
+  constexpr int RB = L::RB;
   f64x4 z[3][RB];
 #pragma unroll
   for (int h = 0; h < RB; ++h) {
@@ -312,9 +360,10 @@ __device__ __forceinline__ long long unit_of(long long units, int it, int waves,
   return units - base >= G * waves ? base + b * waves + w : base + b + G * w;
 }
 
-// The plain kernel over states [0, n_eff).
-template <int N, int KR, bool RCP, int WAVES, bool PSTATE>
-__device__ __forceinline__ void plain(const double* tab, long long n_eff, long long offsetT,
+// The plain kernel over states [0, n_eff); STAGED: `rows` is two row buffers (states16).
+template <int N, int KR, bool RCP, int WAVES, bool PSTATE, bool STAGED>
+__device__ __forceinline__ void plain(const double* tab, double* rows, const double* __restrict__ grows,
+                                      long long n_eff, long long offsetT,
                                       long long offset, const double* __restrict__ p_state,
                                       double pressure, const double* __restrict__ state,
                                       double* __restrict__ conductivity,
@@ -327,16 +376,22 @@ __device__ __forceinline__ void plain(const double* tab, long long n_eff, long l
   const long long units = (n_eff + 15) / 16;
 #pragma unroll 1
   for (int it = 0;; ++it) {
-    const long long u = unit_of(units, it, WAVES, w);
-    if (u >= units) break;
+    const long long u0 = unit_of(units, it, WAVES, w);
+    const bool busy = u0 < units;
+    if (STAGED ? unit_of(units, it, WAVES, 0) >= units : !busy) break;   // staged: whole workgroups
+    const long long u = busy ? u0 : 0;
     const long long id0 = 16 * u + (lane & 15);
-    const bool live = id0 < n_eff;
-    const long long id = live ? id0 : 16 * u;     // lanes past the end redo the first state, store nothing
+    const bool live = busy && id0 < n_eff;
+    const long long id = id0 < n_eff ? id0 : 16 * u;   // lanes past the end redo the first state, store nothing
+    if (STAGED) {
+      __syncthreads();                                 // the last call's rows read by all
+      for (int e = threadIdx.x; e < 80; e += 64 * WAVES) rows[e] = grows[e];
+    }
     const double p = PSTATE ? p_state[id] : pressure;
     double mu, lambda;
     const long long own = id + (lane >> 4) * offset;       // species 4 m + g at own + 4 m offset
-    states16<N, KR, RCP>(tab, state, id, offsetT, offset, Tref, p, t0, rcpR, lane, mu, lambda,
-                     [&](const double (&D)[NB], double rho) {
+    states16<N, KR, RCP, STAGED ? 64 * WAVES : 0>(tab, rows, grows, busy, state, id, offsetT, offset,
+                     Tref, p, t0, rcpR, lane, mu, lambda, [&](const double (&D)[NB], double rho) {
                        if (!live) return;
 #pragma unroll
                        for (int m = 0; m < NB; ++m)
@@ -357,7 +412,7 @@ __device__ __forceinline__ void plain(const double* tab, long long n_eff, long l
 // audit entry the surrogate answered (flag 0) first compares mu, lambda and rho*D_k with its
 // values, and counts in counters[1] if any is off (or NaN).
 template <int N, int KR, bool RCP, int WAVES>
-__device__ __forceinline__ void queued(const double* tab, long long valid, int n_audit,
+__device__ __forceinline__ void queued(const double* tab, double* rows, long long valid, int n_audit,
                                        const int* __restrict__ queue, int* __restrict__ counters,
                                        const int* __restrict__ flags, double tol, double tol_rhoD,
                                        long long offsetT, long long offset,
@@ -381,8 +436,8 @@ __device__ __forceinline__ void queued(const double* tab, long long valid, int n
     const bool audit = live && slot < n_audit && flags[id] == 0;
     const long long own = id + (lane >> 4) * offset;
     double mu, lambda, bad = 0.0;
-    states16<N, KR, RCP>(tab, state, id, offsetT, offset, Tref, p_state[id], t0, rcpR, lane, mu, lambda,
-                         [&](const double (&D)[NB], double rho) {
+    states16<N, KR, RCP, 0>(tab, rows, nullptr, true, state, id, offsetT, offset, Tref, p_state[id], t0,
+                         rcpR, lane, mu, lambda, [&](const double (&D)[NB], double rho) {
                            if (!live) return;
 #pragma unroll
                            for (int m = 0; m < NB; ++m)

@@ -3,9 +3,9 @@ surrogate's kx_bk2_fp64_queue on the wave-level routine of csrc/kx_bk2_quad.h.
 
 This module builds the routine's table (one FP64 __device__ array per mechanism, staged in
 LDS by each workgroup) and emits the kernels around it. With NB = ceil(N / 4) slots of four
-species and one block (m, j) per slot pair j <= m, at m (m + 1) / 2 + j, the table holds, in
-this order:
+species and one block (m, j) per slot pair j <= m, the table holds, in this order:
 
+  rows m = 0 .. NB - 1, each fitA then fitC of its m + 1 blocks:
   fitA [block][64]   the diffusion fits' A operand of v_mfma_f64_16x16x4_f64: lane l holds the
                      coefficient of t^(l / 16 + 1) of the pair in row l % 16; row 4 c + g is
                      the pair (4 m + c, 4 j + g)
@@ -78,8 +78,17 @@ def table_doubles(N, kr):
     return (n + 1) & ~1
 
 
-def lds_bytes(t):
-    return 8 * table_doubles(int(t['n_species']), rank_groups(t))
+def row_doubles(N):
+    """The pair rows, and the longest of them."""
+    nb = slots(N)
+    return 40 * nb * (nb + 1), 80 * nb
+
+
+def lds_bytes(t, staged=False):
+    N = int(t['n_species'])
+    rows, longest = row_doubles(N)
+    n = table_doubles(N, rank_groups(t))
+    return 8 * (n - rows + 2 * longest if staged else n)
 
 
 def center(t):
@@ -144,7 +153,8 @@ def table(t):
                             A[h, 16 * q + 4 * c + g] = f[q + 1]
         return [A, C]
     pad = lambda v: np.concatenate([v, np.zeros(4 * nb - N)])
-    parts = [fitA, fitC, wilT, wil] + species(t['visc'], [1.0 / math.sqrt(math.sqrt(w)) for w in W]) \
+    rows = [v[m * (m + 1) // 2:(m + 1) * (m + 2) // 2] for m in range(nb) for v in (fitA, fitC)]
+    parts = rows + [wilT, wil] + species(t['visc'], [1.0 / math.sqrt(math.sqrt(w)) for w in W]) \
         + species(t['cond'], np.ones(N)) \
         + [pad(np.asarray(t['rcpW'], dtype=np.float64)), pad(W), pad(np.sqrt(W))]
     flat = np.concatenate([p.reshape(-1) for p in parts])
@@ -152,29 +162,44 @@ def table(t):
 
 
 def fits(t):
-    """Whether a mechanism takes this family. N >= 20: below, the 4-fold repeated per-state work
-    (T powers, divides) outweighs the shared pairs -- 1,048,576 states of 9 species: 144 us
-    against 69 for one state per lane, of 31 species: 422 against 598, of 53: 910 against
-    1,861; the two cost curves in N cross near 18. At the other end the table has to fit the
-    160 KB of a CU's LDS (N <= 72)."""
+    """Whether a mechanism takes this family, with its whole table in LDS. N >= 20: below, the
+    4-fold repeated per-state work (T powers, divides) outweighs the shared pairs -- 1,048,576
+    states of 9 species: 144 us against 69 for one state per lane, of 31 species: 422 against
+    598, of 53: 910 against 1,861; the two cost curves in N cross near 18. At the other end the
+    table has to fit the 160 KB of a CU's LDS (N <= 72)."""
     return int(t['n_species']) >= 20 and lds_bytes(t) <= LDS_MAX
 
 
-def emit(t, info, waves=WAVES):
-    """kx_bk2_fp64, kx_bk2_fp64_pstate, kx_bk2_fp64_queue, and kx_bk2_fp64_mfma (the transport
-    entry point that asks for the Wilke sum on FP64 MFMA: the same kernel here)."""
+def fits_staged(t):
+    """Whether it does with the pair rows streamed through LDS: up to 160 species, whose 40 slots
+    of x and of the sums take 160 of a wavefront's 256 VGPRs."""
+    return 20 <= int(t['n_species']) <= 160 and lds_bytes(t, True) <= LDS_MAX
+
+
+def emit(t, info, waves=WAVES, staged=False, mfma=True):
+    """kx_bk2_fp64, kx_bk2_fp64_pstate, beside straight-line kernels also kx_bk2_fp64_mfma (the
+    transport entry point that asks for the Wilke sum on FP64 MFMA: the same kernel here), and
+    with the table resident (every mechanism a surrogate can have) kx_bk2_fp64_queue."""
     N = int(t['n_species'])
     rcp = 'true' if int(t.get('rcp_diff', 0)) else 'false'
     kr = rank_groups(t)
     n = table_doubles(N, kr)
+    rows, longest = row_doubles(N)
     t0, rcpR = repr(center(t)), E._literal(1.0 / float(t['R']))
     S = E._Src()
     S('#include "kx_bk2_quad.h"   // four lanes per state (kinetix_amd/csrc)', 0)
     S(f'__device__ const double kx_bk2_tab[{n}] __attribute__((aligned(16))) = {{' +
       ', '.join(E._literal(v) for v in table(t)) + '};', 0)
-    tab = [f'__shared__ __attribute__((aligned(16))) double tab[{n}];',
-           f'kxquad::stage<{n}, {64 * waves}>(tab, kx_bk2_tab);']
-    for name, ps in (('kx_bk2_fp64', False), ('kx_bk2_fp64_mfma', False), ('kx_bk2_fp64_pstate', True)):
+    if staged:
+        tab = [f'__shared__ __attribute__((aligned(16))) double tab[{n - rows}], rows[{2 * longest}];',
+               f'kxquad::stage<{n - rows}, {64 * waves}>(tab, kx_bk2_tab + {rows});']
+        args = 'tab, rows, kx_bk2_tab'
+    else:
+        tab = [f'__shared__ __attribute__((aligned(16))) double rows[{n}];',
+               f'kxquad::stage<{n}, {64 * waves}>(rows, kx_bk2_tab);']
+        args = f'rows + {rows}, rows, nullptr'
+    forms = [('kx_bk2_fp64', False), ('kx_bk2_fp64_mfma', False), ('kx_bk2_fp64_pstate', True)]
+    for name, ps in forms if mfma else forms[::2]:
         S(f'extern "C" __device__ const int {name}_states_per_wave = 16;', 0)
         S(f'extern "C" __global__ void __launch_bounds__({64 * waves})', 0)
         S(f'{name}(const int n_states, const long long offsetT, const long long offset,', 0)
@@ -189,10 +214,13 @@ def emit(t, info, waves=WAVES):
         S('if (16ll * blockIdx.x >= n_eff) return;        // whole workgroup past the end')
         for line in tab:
             S(line)
-        S(f'kxquad::plain<{N}, {kr}, {rcp}, {waves}, {"true" if ps else "false"}>(tab, n_eff, offsetT, offset,')
-        S('    ' + ('p_state, 0.0' if ps else 'nullptr, pressure') + ', state, conductivity, viscosity, rhoD, '
-          + ('Dkm' if ps else 'nullptr') + f', Tref, {t0}, {rcpR});')
+        S(f'kxquad::plain<{N}, {kr}, {rcp}, {waves}, {"true" if ps else "false"}, {"true" if staged else "false"}>(')
+        S(f'    {args}, n_eff, offsetT, offset, ' + ('p_state, 0.0' if ps else 'nullptr, pressure') +
+          ', state, conductivity, viscosity, rhoD,')
+        S('    ' + ('Dkm' if ps else 'nullptr') + f', Tref, {t0}, {rcpR});')
         S('}', 0)
+    if staged:
+        return S.text()
     S('// the surrogate\'s plain pass over a device queue of state ids (kxquad::queued)', 0)
     S(f'extern "C" __device__ const int kx_bk2q_lanes = {LPS};', 0)
     S('extern "C" __device__ const int kx_bk2_fp64_queue_states_per_wave = 16;', 0)
@@ -210,7 +238,7 @@ def emit(t, info, waves=WAVES):
     S('if (16ll * blockIdx.x >= valid) return;           // whole workgroup past the queue')
     for line in tab:
         S(line)
-    S(f'kxquad::queued<{N}, {kr}, {rcp}, {waves}>(tab, valid, n_audit, queue, counters, flags, tol, tol_rhoD,')
-    S(f'    offsetT, offset, p_state, state, conductivity, viscosity, rhoD, Dkm, Tref, {t0}, {rcpR});')
+    S(f'kxquad::queued<{N}, {kr}, {rcp}, {waves}>(rows + {rows}, rows, valid, n_audit, queue, counters, flags,')
+    S(f'    tol, tol_rhoD, offsetT, offset, p_state, state, conductivity, viscosity, rhoD, Dkm, Tref, {t0}, {rcpR});')
     S('}', 0)
     return S.text()

@@ -1,4 +1,5 @@
-"""Transport (BK2) for large mechanisms: kx_bk2_fp64 / kx_bk2_fp64_pstate over state tiles.
+"""Transport (BK2) in loop form: kx_bk2_fp64 / kx_bk2_fp64_pstate over state tiles, for small
+mechanisms asked for in loop form (large ones take emit_bk2_quad, 3x faster at 160 species).
 
 The loop form with one state per lane (one lane's x, 1/eta and pair-sum arrays of N doubles
 each) keeps ~5 KB per lane at 160 species in scratch; with ~10^4 lanes per XCD that working set

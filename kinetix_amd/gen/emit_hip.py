@@ -1102,12 +1102,20 @@ def generate(tables, info, opts=None):
         parts.append(emit_coop.emit_bk1(tables, info, 'fp64', o['coop_lps']))
         parts.append(emit_coop.emit_bk1(tables, info, 'mixed_valu', o['coop_lps']))
         if 'cond' in tables:
-            # transport over 64-state tiles (species rows across wavefronts, x and 1/eta in
-            # LDS) up to 160 species; beyond that, or asked for (bk2_loop), the one-lane loop form
+            # transport: four lanes per state with the pair rows streamed through LDS up to 160
+            # species (160 species, 2,097,152 states: 12.1 ms against 36.7 in 64-state tiles);
+            # beyond that, or asked for (bk2_loop), the one-lane loop form. A mechanism small
+            # enough for straight-line code that is asked for in loop form takes the tiles:
+            # its transport does not unroll the pairs either
+            from . import emit_bk2_quad as QD
             from . import emit_bk2_tile as BT
-            tile = BT.lds_bytes(tables) <= 160 * 1024 and not o.get('bk2_loop')
-            for ps in (False, True):
-                parts.append(BT.emit(tables, info, ps) if tile else emit_rolled.emit_bk2(tables, info, ps))
+            small = int(tables['n_species']) <= emit_rolled.ROLL_N
+            if not small and QD.fits_staged(tables) and not o.get('bk2_loop'):
+                parts.append(QD.emit(tables, info, staged=True, mfma=False))
+            else:
+                tile = BT.lds_bytes(tables) <= 160 * 1024 and not o.get('bk2_loop')
+                for ps in (False, True):
+                    parts.append(BT.emit(tables, info, ps) if tile else emit_rolled.emit_bk2(tables, info, ps))
         parts.append(_with_pool('kx_thermo_fp64_k', _emit_thermo_fp64, tables, info))
         return '\n\n'.join(parts) + '\n'
     order = None
@@ -1120,8 +1128,8 @@ def generate(tables, info, opts=None):
         parts.append(_with_pool('kx_bk1_fp64_k', _emit_bk1_fp64, tables, info, o['bk1_sched_window'],
                                 o['bk1_wform'], lds=o['lds_pool']))
     from . import emit_bk2_quad as QD
-    if 'cond' in tables and QD.fits(tables):
-        parts.append(QD.emit(tables, info))
+    if 'cond' in tables and (QD.fits(tables) or QD.fits_staged(tables)):
+        parts.append(QD.emit(tables, info, staged=not QD.fits(tables)))
     elif 'cond' in tables:
         parts.append(_with_pool('kx_bk2_fp64_k', _emit_bk2_fp64, tables, info, False, o['bk2_block'],
                                 lds=o['lds_pool'], block=o['bk2_block']))

@@ -38,9 +38,9 @@ def quad_numpy(t, s, p):
     tab = Q.table(t)
     kr = Q.rank_groups(t)
     rb = (kr + 3) // 4
-    o = np.cumsum([0, 64 * blk, 16 * blk, 64 * nb * rb, 64 * sg * kr, 64 * sg, 16 * sg, 64 * sg, 16 * sg,
+    o = np.cumsum([80 * blk, 64 * nb * rb, 64 * sg * kr, 64 * sg, 16 * sg, 64 * sg, 16 * sg,
                    4 * nb, 4 * nb, 4 * nb])
-    fitA, fitC, wilT, wil, vA, vC, lA, lC, rW, Wt, sW = (tab[a:b] for a, b in zip(o[:-1], o[1:]))
+    wilT, wil, vA, vC, lA, lC, rW, Wt, sW = (tab[a:b] for a, b in zip(o[:-1], o[1:]))
     lane = np.arange(64)
     st, g = lane % 16, lane // 16
     T = s[0][st]
@@ -60,8 +60,8 @@ def quad_numpy(t, s, p):
     for m in range(nb):
         xk, q = bc(x[m]), np.zeros((4, 64))
         for j in range(m + 1):
-            b = m * (m + 1) // 2 + j
-            d = _mfma(fitA[64 * b:64 * b + 64], B, acc(fitC, b))
+            row = tab[40 * m * (m + 1):]
+            d = _mfma(row[64 * j:64 * j + 64], B, acc(row[64 * (m + 1):], j))
             r = (d if int(t['rcp_diff']) else 1.0 / d).T
             if j < m:
                 S[j] += (xk * r).sum(0)
@@ -124,10 +124,11 @@ def test_quad_routine_vs_oracle(mech):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize('mech,n', [('gri30', 1), ('gri30', 15), ('gri30', 2049), ('gri30', 33000),
-                                    ('chempolimi_edit', 17), ('synth40cov', 4097)])
+                                    ('chempolimi_edit', 17), ('synth40cov', 4097),
+                                    ('EtOHKonnov', 1), ('EtOHKonnov', 2065), ('synth160', 33000)])
 def test_quad_kernels_at_group_edges(mech, n):
-    """Scalar, per-state-pressure and MFMA entry points at state counts that end inside a
-    16-state group, fill every wavefront of the grid (256 x 8 x 16 states on a 256-CU GPU) and
+    """Scalar, per-state-pressure and (straight-line mechanisms) MFMA entry points, the table
+    resident in LDS and streamed (129 and 160 species), at state counts that end inside a 16-state group, fill every wavefront of the grid (256 x 8 x 16 states on a 256-CU GPU) and
     run past it, on a strided view: against the oracle, nothing written outside the view, and
     the same bits whatever the group a state lands in."""
     import torch
@@ -145,7 +146,7 @@ def test_quad_kernels_at_group_edges(mech, n):
         kx.build(101325.0, 1.0, states.reference_mass_fractions(info['species'], t['W']))
         ds, dp = d(s).reshape(-1)[lo:], d(p)[lo:]
         out = {}
-        for form in ('plain', 'mfma', 'pstate'):
+        for form in ('plain', 'mfma', 'pstate') if N <= 96 else ('plain', 'pstate'):
             v, c, r, D = z(n), z(n), z(N, ld), z(N, ld)
             R, DD = r.reshape(-1)[lo:], D.reshape(-1)[lo:]
             if form == 'pstate':
@@ -175,5 +176,6 @@ def test_quad_kernels_at_group_edges(mech, n):
         for a in (r, D) if form == 'pstate' else (r,):
             assert np.all(np.isfinite(a[:, lo:lo + n]))
             assert np.all(np.isnan(a[:, :lo])) and np.all(np.isnan(a[:, lo + n:]))
-    assert all(np.array_equal(a, b, equal_nan=True) for a, b in zip(out['plain'][:3], out['mfma'][:3]))
+    if 'mfma' in out:
+        assert all(np.array_equal(a, b, equal_nan=True) for a, b in zip(out['plain'][:3], out['mfma'][:3]))
     assert all(np.array_equal(a, b) for a, b in zip(out['plain'][:2], out['pstate'][:2]))
