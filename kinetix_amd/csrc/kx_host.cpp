@@ -47,8 +47,8 @@ struct Mech {
   std::map<std::string, hipFunction_t> fn;
   std::map<std::string, unsigned> block;     // each kernel's launch bound (threads per block)
   std::map<std::string, int> lanes;          // lanes per state of kernels that share a state
-  std::map<std::string, int> wave_states;    // states per wavefront of the kernels that loop over
-  std::map<std::string, long long> resident;  // state groups, and their workgroups resident at once
+  std::map<std::string, int> group_states;    // kernels that loop over groups of states: the group's
+  std::map<std::string, long long> resident;  // size, and their workgroups resident at once
   int queue_lanes = 1;                        // lanes per queued state of kx_bk2_fp64_queue
   long long queue_grid_cap = 0;               // its workgroups resident at once (strided form)
   int n_species = 0, n_active = 0, n_reactions = 0;
@@ -135,8 +135,8 @@ int launch(Mech* m, const char* name, long long n_lanes, void* stream, void** ar
   const unsigned block = m->block.at(name);
   auto l = m->lanes.find(name);
   if (l != m->lanes.end()) n_lanes *= l->second;
-  auto ws = m->wave_states.find(name);
-  if (ws != m->wave_states.end()) {
+  auto ws = m->group_states.find(name);
+  if (ws != m->group_states.end()) {
     // a workgroup per group of states up to those resident at once; the kernel loops
     const long long groups = (n_lanes + ws->second - 1) / ws->second;
     KX_HIP(hipModuleLaunchKernel(it->second, (unsigned)std::min(groups, m->resident.at(name)), 1, 1,
@@ -237,8 +237,8 @@ static int finish_init(Mech* m, kx_mech_t* out)
     } else {
       (void)hipGetLastError();
     }
-    // a kernel whose wavefronts loop over groups of states exports the group's size
-    if (hipModuleGetGlobal(&lp, &lbytes, m->module, (std::string(k) + "_states_per_wave").c_str()) ==
+    // a kernel that loops over groups of states exports the group's size
+    if (hipModuleGetGlobal(&lp, &lbytes, m->module, (std::string(k) + "_states_per_group").c_str()) ==
             hipSuccess &&
         lbytes == sizeof(int)) {
       int ws = 0;
@@ -246,9 +246,9 @@ static int finish_init(Mech* m, kx_mech_t* out)
         (void)hipGetLastError();
         (void)hipModuleUnload(m->module);
         delete m;
-        return fail(KX_ERR_HIP, std::string("unusable states per wave for ") + k);
+        return fail(KX_ERR_HIP, std::string("unusable states per group for ") + k);
       }
-      m->wave_states[k] = ws;
+      m->group_states[k] = ws;
       m->resident[k] = resident_workgroups(m, f, bound);
     } else {
       (void)hipGetLastError();
@@ -651,7 +651,7 @@ int kx_sur_transport(kx_mech_t h, int n, int offsetT, int offset, const double* 
                     (void*)&d_p,
                     (void*)&d_state, &d_cond, &d_visc, &d_rhoD, &d_Dkm, &Tref};
     const long long longest = (long long)n_audit + n;
-    if (m->queue_lanes > 1 && !m->wave_states.count("kx_bk2_fp64_queue")) {
+    if (m->queue_lanes > 1 && !m->group_states.count("kx_bk2_fp64_queue")) {
       // the cooperative form strides over the queue: a grid of the workgroups resident at
       // once, or fewer when even the longest possible queue needs fewer
       const long long per_wg = m->block.at("kx_bk2_fp64_queue") / m->queue_lanes;

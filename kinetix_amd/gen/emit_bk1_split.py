@@ -1,0 +1,400 @@
+"""Production rates (BK1) with the reactions split over the wavefronts of a workgroup: kx_bk1_fp64
+and kx_bk1_mixed_valu for straight-line mechanisms (benchmark/okl/productionRates.okl:10-62,
+kinetix/core/reaction_rates.py:616-1333).
+
+One lane still works on one state, but a workgroup's WAVES wavefronts share the same 64 states:
+
+  species    wavefront v takes the species k = v, v + WAVES, ...: Y, the Gibbs term g_k from the
+             LDS NASA-7 table, e = exp(g_k), and puts w_k = C_k e and rg_k = 1 / e into LDS rows of 64
+             states (512 B: every access is conflict-free);
+  reactions  each wavefront runs its own part of the reactions as straight-line code (product
+             form: q = k_f prod rg_reactants (prod w_reactants - C0^-dnu prod w_products)),
+             reading w and rg from LDS where they are used and adding nu q to its own sums;
+  sums       the wavefronts' sums meet in LDS rows (over the dead w and rg rows) and the
+             species' owners add them in a fixed order, store W_k omega_k and add up the heat
+             release.
+
+Why: one wavefront that runs all of a state's reactions keeps three FP64 values per species alive
+(474 registers for GRI-3.0: one wave per SIMD, which issues at most every fifth cycle, or, at two
+waves, spills that double the HBM traffic). In LDS the values are shared, a wavefront needs
+under 128 registers, and four waves per SIMD hide each other's latencies; a small call's latency
+falls with the length of one wavefront's program.
+
+Measured (before: one wavefront per 64 states, product form): GRI-3.0, 1,048,576 states FP64 762
+-> 617 us, mixed 517 -> 440, 1,000 states FP64 41 -> 13.0 us; NH3Konnov_edit 2,510 -> 518 and
+2,236 -> 378 us. Bound: FP64 issue and its power (75 % of the issue slots at 2.06 GHz). 4
+wavefronts of 256 registers: 625 / 478 us, 15.4 us; 16: 949 / 774; two groups of 64 states per
+workgroup in step: 715 / 566; a loop over groups instead of one per workgroup: 826 / 618 (the
+compiler hoists the constants and spills).
+
+The reactions are dealt to the wavefronts by modelled cost with as few (wavefront, species) sums
+as possible (assign), and the values read from LDS are cached for SEGMENT reactions at a time.
+"""
+from __future__ import annotations
+
+import random
+
+import numpy as np
+
+from . import emit_hip as E
+from . import emit_rolled as RL
+from . import mechanism as M
+
+WAVES = 8                # wavefronts that share 64 states' reactions
+SEGMENT = 6              # reactions between points where values read from LDS are dropped
+ROW = 64                 # states per workgroup
+
+
+def reaction_cost(em, r):
+    """Issue cycles of one reaction (FP64), roughly: exponentials dominate."""
+    t = em.t
+    kind = em.kind[r]
+    c = 30 + 8 * int(em.nu_f[r].sum() + em.nu_r[r].sum()) + 5 * int((em.net[r] != 0).sum())
+    if kind == M.PLOG:
+        return c + 300
+    if em.arrh_key(t['beta'][r], t['Ta'][r]) is not None:
+        c += 95
+    if kind in (M.LINDEMANN, M.TROE, M.SRI):
+        c += 140
+    if kind in (M.TROE, M.SRI):
+        c += 640
+    return c
+
+
+def assign(em, waves=WAVES, iters=40000, seed=7):
+    """Wavefront of every reaction: greedy by cost, then a seeded local search over moves and
+    swaps, minimising the largest load (in cycles) plus 12 cycles per (wavefront, species) sum
+    and 40 per (wavefront, third-body set)."""
+    R = em.R
+    cost = np.array([reaction_cost(em, r) for r in range(R)], dtype=float)
+    net = [np.flatnonzero(em.net[r]).tolist() for r in range(R)]
+
+    def third(r):
+        if em.kind[r] in (M.ELEMENTARY, M.PLOG) or not em.has_eff[r]:
+            return None
+        return tuple(em.t['eff'][r])
+    sets = [third(r) for r in range(R)]
+    load = np.zeros(waves)
+    cnt = [dict() for _ in range(waves)]
+    scnt = [dict() for _ in range(waves)]
+    where = [0] * R
+
+    def put(r, w, s):
+        load[w] += s * cost[r]
+        for k in net[r]:
+            cnt[w][k] = cnt[w].get(k, 0) + s
+            if not cnt[w][k]:
+                del cnt[w][k]
+        if sets[r] is not None:
+            scnt[w][sets[r]] = scnt[w].get(sets[r], 0) + s
+            if not scnt[w][sets[r]]:
+                del scnt[w][sets[r]]
+    target = cost.sum() / waves
+    for r in sorted(range(R), key=lambda r: (-cost[r], r)):
+        key = [(load[w] + cost[r] > 1.02 * target,
+                12 * sum(k not in cnt[w] for k in net[r]) + 40 * (sets[r] is not None and sets[r] not in scnt[w])
+                + 60 * load[w] / target, w) for w in range(waves)]
+        w = min(key)[2]
+        where[r] = w
+        put(r, w, 1)
+
+    def score():
+        per = [load[w] + 12 * len(cnt[w]) + 40 * len(scnt[w]) for w in range(waves)]
+        return waves * max(per) + sum(12 * len(c) for c in cnt) * 3
+    rng = random.Random(seed)
+    cur = score()
+    for _ in range(iters):
+        r = rng.randrange(R)
+        a = where[r]
+        if rng.random() < 0.5:
+            b, s = rng.randrange(waves), None
+            if b == a:
+                continue
+        else:
+            s = rng.randrange(R)
+            b = where[s]
+            if b == a:
+                continue
+        put(r, a, -1); put(r, b, 1)
+        if s is not None:
+            put(s, b, -1); put(s, a, 1)
+        new = score()
+        if new <= cur:
+            cur = new
+            where[r] = b
+            if s is not None:
+                where[s] = a
+        else:
+            put(r, b, -1); put(r, a, 1)
+            if s is not None:
+                put(s, a, -1); put(s, b, 1)
+    return where
+
+
+def order(em, rs):
+    """Order of one wavefront's reactions: next the one sharing most species with the last few."""
+    used = {r: set(np.flatnonzero((em.nu_f[r] > 0) | (em.rev[r] & (em.nu_r[r] > 0))).tolist()) for r in rs}
+    left, out, recent = sorted(rs), [], []
+    while left:
+        near = set().union(*recent[-SEGMENT:]) if recent else set()
+        r = max(left, key=lambda r: (len(used[r] & near), -r))
+        left.remove(r)
+        out.append(r)
+        recent.append(used[r])
+    return out
+
+
+def plan(t, info, waves=WAVES):
+    """Everything the kernel text is written from: per wavefront the ordered reactions, its sums
+    (species), and the rounds in which sums go through LDS rows (slot of every (wave, species))."""
+    em = E._RateEmitter(t, info)
+    N = em.N
+    where = assign(em, waves)
+    rs = [order(em, [r for r in range(em.R) if where[r] == w]) for w in range(waves)]
+    sums = [sorted({int(k) for r in rs[w] for k in np.flatnonzero(em.net[r])}) for w in range(waves)]
+    react = sorted({int(k) for r in range(em.R) for k in np.flatnonzero(em.nu_f[r])})
+    wrow = {k: i for i, k in enumerate(range(N))}
+    rrow = {k: N + i for i, k in enumerate(react)}
+    third = sorted({int(k) for r in range(em.R) if em.kind[r] not in (M.ELEMENTARY, M.PLOG)
+                    for k in ([int(j) for j in np.flatnonzero(em.t['eff'][r] != 1.0)] if em.has_eff[r]
+                              else [int(em.t['collider'][r])] if em.t['collider'][r] >= 0 else [])})
+    crow = {k: N + len(react) + i for i, k in enumerate(third)}
+    rows = max(N + len(react) + len(third), waves)
+    rounds, cur, free = [], {}, rows
+    for w in range(waves):
+        if len(sums[w]) > rows:
+            raise ValueError('more sums in a wavefront than LDS rows')
+        if len(sums[w]) > free:
+            rounds.append(cur)
+            cur, free = {}, rows
+        for k in sums[w]:
+            cur[(w, k)] = rows - free
+            free -= 1
+    rounds.append(cur)
+    return dict(em=em, rs=rs, sums=sums, wrow=wrow, rrow=rrow, crow=crow, rows=rows, rounds=rounds,
+                waves=waves, where=where)
+
+
+def lds_bytes(p):
+    return 8 * (ROW * (p['rows'] + p['waves'] + 1) + 2 * p['em'].N * 14)
+
+
+def pays(t, info):
+    """Whether a straight-line mechanism's reactions are split. A state's modelled load has to be
+    worth the barriers and the per-wavefront prologue: 9 species / 21 reactions (5,000 cycles)
+    run 1,048,576 states in 56 us with one wavefront per 64 states and 132 split; 31 / 203
+    (41,000) in 1,234 and 423. The line lies between, at 16,000. The rows have to fit the LDS."""
+    em = E._RateEmitter(t, info)
+    if sum(reaction_cost(em, r) for r in range(em.R)) < 16000:
+        return False
+    return lds_bytes(plan(t, info)) <= 160 * 1024
+
+
+def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
+    p = plan(t, info, waves)
+    em = p['em']
+    N = em.N
+    mixed = variant == 'mixed_valu'
+    em.arrh32 = mixed
+    name = f'kx_bk1_{variant}'
+    lit = E._literal
+    own = [[k for k in range(N) if k % waves == v] for v in range(waves)]
+    per = max(len(o) for o in own)
+    S = E._Src()
+    # NASA-7: [piece: 0 = T > T_mid, 1 = T <= T_mid][species][14]: Gibbs in 0..6, enthalpy in 8..13
+    PT = np.zeros((2, N, 14))
+    for k in range(N):
+        PT[0, k, :7], PT[0, k, 8:14] = t['g_hi'][k], t['h_hi'][k]
+        PT[1, k, :7], PT[1, k, 8:14] = t['g_lo'][k], t['h_lo'][k]
+    tab = lambda nm, a: S(f'__device__ const double {name}_{nm}[{len(a)}] __attribute__((aligned(16))) = {{' +
+                          ', '.join(lit(v) for v in a) + '};', 0)
+    tab('poly', PT.reshape(-1))
+    tab('rcpW', list(t['rcpW']) + [0.0] * (waves * per - N))
+    tab('tmid', t['T_mid'])
+    plog = None
+    if np.any(em.kind == M.PLOG):
+        d = RL.bk1_data(t)
+        for nm, ct in (('plo', 'int'), ('plP', 'double'), ('pllnP', 'double'), ('plrcp', 'double'),
+                       ('plko', 'int'), ('plnk', 'int'), ('plk', 'double')):
+            S(RL._table(f'{name}_{nm}', d[nm], ct), 0)
+        for line in RL.plog_helpers(name):
+            S(line, 0)
+        plog = lambda r: f'{name}_plog({r}, P, lnP, log2T, rcpT)'
+    S(f'extern "C" __device__ const int {name}_lanes_per_state = {waves};', 0)
+    S(f'extern "C" __global__ void __launch_bounds__({64 * waves}) '
+      f'__attribute__((amdgpu_waves_per_eu({occupancy}, {occupancy})))', 0)
+    S(f'{name}(const int n_states, const long long offsetT, const long long offset,', 0)
+    S('            const double pressure_R, const double pressure_,', 0)
+    S('            const double* __restrict__ state, double* __restrict__ rates, const double Tref)', 0)
+    S('{', 0)
+    S(f'__shared__ __attribute__((aligned(16))) double poly_s[{PT.size}];')
+    S(f'__shared__ double rows[{p["rows"]} * {ROW}];        // w, rg, third-body C; then the wavefronts\' sums')
+    S(f'__shared__ double part[{waves + 1} * {ROW}];')
+    S(f'for (int i = threadIdx.x; i < {PT.size // 2}; i += {64 * waves})')
+    S(f'  ((double2*)poly_s)[i] = ((const double2*){name}_poly)[i];')
+    S('const int lane = threadIdx.x & 63;')
+    S('const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // part of the reactions')
+    S(f'const long long first = (long long)blockIdx.x * {ROW};')
+    S('const long long at = first + lane;')
+    S('const bool live = at < n_states;')
+    S('const long long id = live ? at : first;          // lanes past the end redo the first state, store nothing')
+    S('const double T = Tref * state[id];')
+    S('const double* const Y = state + id + offsetT;')
+    S(f'double c[{per}];')
+    S('double sum = 0.0;')
+    S('#pragma unroll')
+    S(f'for (int i = 0; i < {per}; ++i) {{')
+    S(f'  c[i] = Y[min(v + {waves} * i, {N - 1}) * offset];             // every load in flight before the first use')
+    S('}')
+    S('#pragma unroll')
+    S(f'for (int i = 0; i < {per}; ++i) {{')
+    S(f'  c[i] = fmax(0.0, c[i]) * {name}_rcpW[v + {waves} * i];          // 0 past the last species')
+    S('  sum += c[i];')
+    S('}')
+    S(f'part[v * {ROW} + lane] = sum;')
+    S(f'if (v == {waves - 1}) part[{waves} * {ROW} + lane] = log(T);   // once per state')
+    S('const double rcpT = 1.0 / T;')
+    S('const double T2 = T * T, T3 = T * T * T, T4 = T * T * T * T;')
+    S('const double rcpT2 = rcpT * rcpT;')
+    S('__syncthreads();')
+    S('double rcpMbar = 0.0;')
+    S('#pragma unroll')
+    S(f'for (int i = 0; i < {waves}; ++i) rcpMbar += part[i * {ROW} + lane];')
+    S(f'const double lnT = part[{waves} * {ROW} + lane];')
+    S('const double omlnT = 1.0 - lnT;')
+    S('const double log2T = lnT * 1.4426950408889634;')
+    S('const float Tf = (float)T, rcpTf = (float)rcpT, log2Tf = (float)log2T;')
+    S('const double P = pressure_, lnP = log(P);   // PLOG reactions (uniform per launch)')
+    S('(void)P; (void)lnP; (void)log2T; (void)rcpT2; (void)Tf; (void)rcpTf; (void)log2Tf;')
+    S('const double rho = pressure_R * rcpT / rcpMbar;')
+    S('const double Cm = rho * rcpMbar;')
+    S(f'const double C0 = {lit(float(t["one_atm_R"]))} * rcpT;')
+    S(f'const double rcpC0 = {lit(float(t["R_one_atm"]))} * T;')
+    S('// ---- species: w_k = C_k exp(g_k), rg_k = exp(-g_k), third-body concentrations')
+    rr = [p['rrow'].get(k, -1) for k in range(N)]
+    cr = [p['crow'].get(k, -1) for k in range(N)]
+    S(f'const double* const piece = poly_s;')
+    for i in range(per):
+        S('{')
+        S(f'  const int k = v + {waves} * {i};')
+        ks = [k for k in range(N) if k // waves == i]
+        if len(ks) < waves:
+            S(f'  if (k < {N}) {{')
+        else:
+            S('  {')
+        S(f'  const double ck = c[{i}] * rho;')
+        S(f'  const double* a = piece + 14 * k + (T > {name}_tmid[k] ? 0 : {14 * N});')
+        S('  const double gk = a[0] * omlnT + a[1] * T + a[2] * T2 + a[3] * T3 + a[4] * T4 + a[5] * rcpT - a[6];')
+        S('  const double ek = kx_exp(gk);')
+        S(f'  rows[k * {ROW} + lane] = ck * ek;')
+        # rg and third-body rows: uniform selects over the wavefront's species of this round
+        def pick(rowmap, val):
+            have = [k for k in ks if rowmap[k] >= 0]
+            if not have:
+                return
+            expr = '-1'
+            for k in have:
+                expr = f'v == {k % waves} ? {rowmap[k]} : ({expr})'
+            S(f'  {{ const int row = {expr}; if (row >= 0) rows[row * {ROW} + lane] = {val}; }}')
+        pick(rr, 'kx_rcp(ek)')
+        pick(cr, 'ck')
+        S('  }')
+        S('}')
+    S('__syncthreads();')
+    S('// ---- reactions of each wavefront')
+    mx = max(len(s) for s in p['sums'])
+    S(f'double wd[{mx}];')
+    S('#pragma unroll')
+    S(f'for (int i = 0; i < {mx}; ++i) wd[i] = 0.0;')
+    S('int o = lane;                                     // made opaque between segments')
+    sets, sidx = em.efficiency_sets()
+    for w in range(waves):
+        S(f'{"if" if w == 0 else "else if"} (v == {w}) {{' if w < waves - 1 else 'else {')
+        slot = {k: i for i, k in enumerate(p['sums'][w])}
+        have_third, pins = set(), []
+        for n, r in enumerate(p['rs'][w]):
+            if n % SEGMENT == 0:
+                # the segment's sums are needed as values here: the compiler otherwise defers
+                # them to the end of the wavefront's program, all values read from LDS alive
+                S(f'asm volatile("" : "+v"(o){"".join(f", {q}" for q in pins)});')
+                S('__builtin_amdgcn_sched_barrier(0);')
+                pins = []
+            # third body of this reaction, once per wavefront
+            need = None
+            if em.kind[r] not in (M.ELEMENTARY, M.PLOG):
+                need = em._third_w(r, sidx)
+            if need and need != 'Cm' and need not in have_third:
+                have_third.add(need)
+                if need.startswith('eff'):
+                    terms = ['Cm']
+                    for k, e in enumerate(sets[int(need[3:])]):
+                        if e != 1.0:
+                            terms.append(f'+ {lit(e - 1.0)} * rows[{p["crow"][k] * ROW} + o]')
+                    S(f'const double {need} = ' + ' '.join(terms) + ';')
+                else:
+                    S(f'const double {need} = rows[{p["crow"][int(need[1:])] * ROW} + o];')
+            ks = sorted({int(k) for k in np.flatnonzero((em.nu_f[r] > 0) | (em.rev[r] & (em.nu_r[r] > 0)))})
+            S(f'double q{r};')
+            S('{')
+            for k in ks:
+                S(f'const double W{k} = rows[{p["wrow"][k] * ROW} + o];')
+            for k in np.flatnonzero(em.nu_f[r]):
+                S(f'const double rg{k} = rows[{p["rrow"][int(k)] * ROW} + o];')
+            T_ = E._Src()
+            em.emit_reaction_p(T_, r, sidx, wvar='W', declare=False, plog=plog)
+            for line in T_.lines:
+                S.lines.append('  ' + line)
+            S('}')
+            for k in np.flatnonzero(em.net[r]):
+                nu = int(em.net[r, k])
+                term = f'q{r}' if abs(nu) == 1 else f'{lit(abs(nu))} * q{r}'
+                i = slot[int(k)]
+                if f'"+v"(wd[{i}])' not in pins:
+                    pins.append(f'"+v"(wd[{i}])')
+                S(f'wd[{i}] {"+=" if nu > 0 else "-="} {term};')
+        S('__builtin_amdgcn_sched_barrier(0);')
+        S('}')
+    S('// ---- the wavefronts\' sums meet in LDS, added by the species\' owners in wavefront order')
+    S(f'double acc[{per}];')
+    S('#pragma unroll')
+    S(f'for (int i = 0; i < {per}; ++i) acc[i] = 0.0;')
+    for rnd in p['rounds']:
+        S('__syncthreads();')
+        for w in sorted({w for w, _ in rnd}):
+            S(f'if (v == {w}) {{')
+            for i, k in enumerate(p['sums'][w]):
+                S(f'  rows[{rnd[(w, k)] * ROW} + lane] = wd[{i}];')
+            S('}')
+        S('__syncthreads();')
+        for v in range(waves):
+            S(f'{"if" if v == 0 else "else if"} (v == {v}) {{')
+            for i, k in enumerate(own[v]):
+                for w in range(waves):
+                    if (w, k) in rnd:
+                        S(f'  acc[{i}] += rows[{rnd[(w, k)] * ROW} + lane];')
+            S('}')
+    S('// ---- mass production rates and heat release rate')
+    S('double sh = 0.0;')
+    W = t['W']
+    for v in range(waves):
+        S(f'{"if" if v == 0 else "else if"} (v == {v}) {{')
+        S('  if (live) {')
+        for i, k in enumerate(own[v]):
+            val = f'{lit(W[k])} * acc[{i}]' if k in em.active else '0.0'
+            S(f'    rates[id + offsetT + {k} * offset] = {val};')
+        S('  }')
+        for i, k in enumerate(own[v]):
+            if k in em.active:
+                S(f'  {{ const double* a = piece + {14 * k + 8} + (T > {lit(float(t["T_mid"][k]))} ? 0 : {14 * N});')
+                S(f'    sh += acc[{i}] * (a[0] + a[1] * T + a[2] * T2 + a[3] * T3 + a[4] * T4 + a[5] * rcpT); }}')
+        S('}')
+    S(f'part[v * {ROW} + lane] = sh;')
+    S('__syncthreads();')
+    S('if (v == 0 && live) {')
+    S('  double sum_h = 0.0;')
+    S('  #pragma unroll')
+    S(f'  for (int i = 0; i < {waves}; ++i) sum_h += part[i * {ROW} + lane];')
+    S(f'  rates[id] = {lit(-float(t["R"]))} * T * sum_h;')
+    S('}')
+    S('}', 0)
+    return S.text()

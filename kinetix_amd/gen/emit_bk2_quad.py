@@ -200,7 +200,7 @@ def emit(t, info, waves=WAVES, staged=False, mfma=True):
         args = f'rows + {rows}, rows, nullptr'
     forms = [('kx_bk2_fp64', False), ('kx_bk2_fp64_mfma', False), ('kx_bk2_fp64_pstate', True)]
     for name, ps in forms if mfma else forms[::2]:
-        S(f'extern "C" __device__ const int {name}_states_per_wave = 16;', 0)
+        S(f'extern "C" __device__ const int {name}_states_per_group = 16;', 0)
         S(f'extern "C" __global__ void __launch_bounds__({64 * waves})', 0)
         S(f'{name}(const int n_states, const long long offsetT, const long long offset,', 0)
         S('            ' + ('const double* __restrict__ p_state,' if ps else 'const double pressure,'), 0)
@@ -223,7 +223,7 @@ def emit(t, info, waves=WAVES, staged=False, mfma=True):
         return S.text()
     S('// the surrogate\'s plain pass over a device queue of state ids (kxquad::queued)', 0)
     S(f'extern "C" __device__ const int kx_bk2q_lanes = {LPS};', 0)
-    S('extern "C" __device__ const int kx_bk2_fp64_queue_states_per_wave = 16;', 0)
+    S('extern "C" __device__ const int kx_bk2_fp64_queue_states_per_group = 16;', 0)
     S(f'extern "C" __global__ void __launch_bounds__({64 * waves})', 0)
     S('kx_bk2_fp64_queue(const int n_audit,', 0)
     S('            const int* __restrict__ queue, int* __restrict__ counters,', 0)

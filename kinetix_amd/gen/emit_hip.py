@@ -16,11 +16,12 @@ Design (MI355X-first, not a translation of the reference's rolled C):
   * the mechanism is straight-line code: every table index is a compile-time constant, so
     per-state arrays (concentrations, Gibbs exponentials, wdot) live in registers, not in
     scratch, and no rate constant / q_r array is ever materialised;
-  * BK1 (w-form) is emitted in a register-liveness order (liveness.py): each species' Gibbs
-    term and w = C exp(g) are computed at its first use, its omega-dot is stored after its
-    last reaction, and the reactions are ordered to keep the live set small;
-  * k = A * exp(beta lnT - Ta/T) (A kept exact instead of exp(ln A + ...));
-  * Troe's 10^x is exp10(x).
+  * BK1 multiplies k_f = A T^beta exp(-Ta/T) (A exact; no exponential for A T^n) by the reactants'
+    exp(-g) instead of adding the Gibbs terms to one exponent (exps: 503 -> 380 for GRI-3.0),
+    with the range-free exp2 / exp / log2 of csrc/kx_exp.h: 22,100 -> 12,800 VALU instructions
+    per wavefront, 4,194,304 GRI states 4.2 -> 3.1 ms. Small mechanisms run it in a
+    register-liveness order (liveness.py), larger ones split over the wavefronts of a workgroup
+    (emit_bk1_split.py).
 """
 from __future__ import annotations
 
@@ -485,44 +486,118 @@ class _RateEmitter:
                 S(f'  F *= Pr1 * {lit(d)} * pow(T, {lit(e)}) * pow({lit(a)} * exp({lit(-b)} * rcpT)'
                   f' + exp({lit(-rc)} * T), 1.0 / (1.0 + logPr * logPr));')
         elif kind in (M.LINDEMANN, M.TROE, M.SRI):
-            ratio = math.log2(t['A0'][r] / t['A'][r])
-            db = float(t['beta0'][r]) - float(t['beta'][r])
-            dT = float(t['Ta0'][r]) - float(t['Ta'][r])
-            # clamped below FLT_MAX: Pr / (1 + Pr) must stay finite (-> 1) in FP32; the FP32
-            # exponent is capped at 100 so exp2f stays finite (no 0 * inf at M = 0)
-            if getattr(self, 'arrh32', False):
-                S(f'  const float Pr = fminf((float){self._third_w(r, sidx)} * '
-                  f'__builtin_amdgcn_exp2f(fminf({self._log2_rate32(2.0 ** ratio, db, dT)}, 100.0f)), 1e30f);')
-            else:
-                S(f'  const float Pr = (float)fmin({self._third_w(r, sidx)} * '
-                  f'{pow2}({self._log2_rate(2.0 ** ratio, db, dT)}), 1e30);')
-            S('  const float Pr1 = Pr * __builtin_amdgcn_rcpf(1.0f + Pr);')
-            if kind == M.LINDEMANN:
-                S('  F *= (double)Pr1;')
-            elif kind == M.TROE:
-                A_, rT3, rT1, T2 = t['troe'][r]
-                L2E = 1.4426950408889634
-                term3 = (f' + __builtin_amdgcn_exp2f({float(-T2 * L2E)!r}f * rcpTf)' if T2 >= 0 else '')
-                S(f'  const float logFc = {0.30102999566398120!r}f * __builtin_amdgcn_logf('
-                  f'{float(1.0 - A_)!r}f * __builtin_amdgcn_exp2f({float(-rT3 * L2E)!r}f * Tf) + '
-                  f'{float(A_)!r}f * __builtin_amdgcn_exp2f({float(-rT1 * L2E)!r}f * Tf){term3});')
-                S(f'  const float logPr = {0.30102999566398120!r}f * __builtin_amdgcn_logf(Pr + 1e-37f);')
-                S('  const float tc = -0.4f - 0.67f * logFc + logPr;')
-                S('  const float tf = tc * __builtin_amdgcn_rcpf(0.75f - 1.27f * logFc - 0.14f * tc + 1e-37f);')
-                S(f'  const float Fc = __builtin_amdgcn_exp2f({3.3219280948873622!r}f * logFc * '
-                  f'__builtin_amdgcn_rcpf(1.0f + tf * tf));')
-                S('  F *= (double)(Pr1 * Fc);')
-            else:
-                a, b, rc, d, e = t['sri'][r]
-                S(f'  const float logPr = {0.30102999566398120!r}f * __builtin_amdgcn_logf(Pr + 1e-37f);')
-                S(f'  const float Fs = {float(d)!r}f * powf(Tf, {float(e)!r}f) * powf({float(a)!r}f * '
-                  f'expf({float(-b)!r}f * rcpTf) + expf({float(-rc)!r}f * Tf), '
-                  f'__builtin_amdgcn_rcpf(1.0f + logPr * logPr));')
-                S('  F *= (double)(Pr1 * Fs);')
+            self.emit_falloff32(S, r, sidx, math.log2(t['A0'][r] / t['A'][r]),
+                                float(t['beta0'][r]) - float(t['beta'][r]),
+                                float(t['Ta0'][r]) - float(t['Ta'][r]), pow2)
         fwd = _prod('w', self.nu_f[r]) or '1.0'
         if self.rev[r]:
             dnu = int(self.net[r].sum())
             rev = _prod('w', self.nu_r[r]) or '1.0'
+            c0 = '*'.join(['C0' if dnu < 0 else 'rcpC0'] * abs(dnu))
+            rev_term = f'({c0}) * {rev}' if c0 else rev
+            S(f'  q{r} = F * ({fwd} - {rev_term});')
+        else:
+            S(f'  q{r} = F * ({fwd});')
+        S('}')
+
+    def emit_falloff32(self, S, r, sidx, ratio, db, dT, pow2='kx_exp2'):
+        """FP32 Lindemann/Troe/SRI factor on F (mixed variants)."""
+        t, kind = self.t, self.kind[r]
+        # clamped below FLT_MAX: Pr / (1 + Pr) must stay finite (-> 1) in FP32; the FP32
+        # exponent is capped at 100 so exp2f stays finite (no 0 * inf at M = 0)
+        if getattr(self, 'arrh32', False):
+            S(f'  const float Pr = fminf((float){self._third_w(r, sidx)} * '
+              f'__builtin_amdgcn_exp2f(fminf({self._log2_rate32(2.0 ** ratio, db, dT)}, 100.0f)), 1e30f);')
+        else:
+            S(f'  const float Pr = (float)fmin({self._third_w(r, sidx)} * '
+              f'{pow2}({self._log2_rate(2.0 ** ratio, db, dT)}), 1e30);')
+        S('  const float Pr1 = Pr * __builtin_amdgcn_rcpf(1.0f + Pr);')
+        if kind == M.LINDEMANN:
+            S('  F *= (double)Pr1;')
+        elif kind == M.TROE:
+            A_, rT3, rT1, T2 = t['troe'][r]
+            L2E = 1.4426950408889634
+            term3 = (f' + __builtin_amdgcn_exp2f({float(-T2 * L2E)!r}f * rcpTf)' if T2 >= 0 else '')
+            S(f'  const float logFc = {0.30102999566398120!r}f * __builtin_amdgcn_logf('
+              f'{float(1.0 - A_)!r}f * __builtin_amdgcn_exp2f({float(-rT3 * L2E)!r}f * Tf) + '
+              f'{float(A_)!r}f * __builtin_amdgcn_exp2f({float(-rT1 * L2E)!r}f * Tf){term3});')
+            S(f'  const float logPr = {0.30102999566398120!r}f * __builtin_amdgcn_logf(Pr + 1e-37f);')
+            S('  const float tc = -0.4f - 0.67f * logFc + logPr;')
+            S('  const float tf = tc * __builtin_amdgcn_rcpf(0.75f - 1.27f * logFc - 0.14f * tc + 1e-37f);')
+            S(f'  const float Fc = __builtin_amdgcn_exp2f({3.3219280948873622!r}f * logFc * '
+              f'__builtin_amdgcn_rcpf(1.0f + tf * tf));')
+            S('  F *= (double)(Pr1 * Fc);')
+        else:
+            a, b, rc, d, e = t['sri'][r]
+            S(f'  const float logPr = {0.30102999566398120!r}f * __builtin_amdgcn_logf(Pr + 1e-37f);')
+            S(f'  const float Fs = {float(d)!r}f * powf(Tf, {float(e)!r}f) * powf({float(a)!r}f * '
+              f'expf({float(-b)!r}f * rcpTf) + expf({float(-rc)!r}f * Tf), '
+              f'__builtin_amdgcn_rcpf(1.0f + logPr * logPr));')
+            S('  F *= (double)(Pr1 * Fs);')
+
+    # ---- product form: q_r = [k_f prod_reactants rg] (prod_r w - C0^-dnu prod_p w) with w = C e,
+    # rg = 1 / e, e = exp(g): the w-form with the factor exp(-sum g) as a product
+    def rate_const_p(self, r):
+        """(FP64 expression of k_f / k_inf) for emit_reaction_p: no exponential for A T^n of
+        small integer n, else A times one exp2 (FP32 exponent in the mixed variant)."""
+        t = self.t
+        A, beta, Ta = float(t['A'][r]), float(t['beta'][r]), float(t['Ta'][r])
+        if self.arrh_key(beta, Ta) is None:
+            return self.arrh_expr(A, beta, Ta, None)
+        if getattr(self, 'arrh32', False):
+            return f'kx_exp2_f32({self._log2_rate32(A, beta, Ta)})'
+        return f'{lit(A)} * kx_exp2({self._log2_rate(1.0, beta, Ta)})'
+
+    def emit_reaction_p(self, S, r, sidx, wvar='w', declare=True, plog=None):
+        """Emit `double q<r>` (declare=False: assign it) in the product form. FP64 variant: everything in FP64, log2 Pr from
+        the exponent of k_0 / k_inf and one log2 of the third body (never a log of an exp);
+        mixed: FP32 exponents and falloff as in the w-form."""
+        t = self.t
+        kind = self.kind[r]
+        mixed = getattr(self, 'arrh32', False)
+        rg = ''.join(f' * rg{k}' * int(self.nu_f[r, k]) for k in range(self.N) if self.nu_f[r, k])
+        if declare:
+            S(f'double q{r};')
+        S(f'{{ // {r + 1}: {self.equations[r] if self.equations else ""}')
+        if kind == M.PLOG:
+            # log2 k_f interpolated linearly in ln P (see emit_reaction_w): plog names the
+            # helper over the loop-form tables (uniform loads and branches)
+            S(f'  double F = kx_exp2({plog(r) if plog else self._plog_log2k(r)}){rg};')
+        else:
+            S(f'  double F = {self.rate_const_p(r)}{rg};')
+        if kind == M.THREE_BODY:
+            S(f'  F *= {self._third_w(r, sidx)};')
+        elif kind in (M.LINDEMANN, M.TROE, M.SRI):
+            ratio = math.log2(t['A0'][r] / t['A'][r])
+            db = float(t['beta0'][r]) - float(t['beta'][r])
+            dT = float(t['Ta0'][r]) - float(t['Ta'][r])
+            if mixed:
+                self.emit_falloff32(S, r, sidx, ratio, db, dT)
+            else:
+                third = self._third_w(r, sidx)
+                S(f'  const double y0 = {self._log2_rate(2.0 ** ratio, db, dT)};')
+                S(f'  const double Pr = {third} * kx_exp2(y0);')
+                S('  F *= Pr * kx_rcp(1.0 + Pr);')
+                if kind != M.LINDEMANN:
+                    # log10 Pr, floored at -300 as log10(Pr + 1e-300)
+                    S(f'  const double lP = {lit(math.log10(2.0))} * fmax(y0 + kx_log2(fmax({third}, 1e-300)), -997.0);')
+                if kind == M.TROE:
+                    A_, rT3, rT1, T2 = t['troe'][r]
+                    L2E = 1.4426950408889634
+                    term3 = f' + kx_exp2({lit(-T2 * L2E)} * rcpT)' if T2 >= 0 else ''
+                    S(f'  const double l2F = kx_log2({lit(1.0 - A_)} * kx_exp2({lit(-rT3 * L2E)} * T) + '
+                      f'{lit(A_)} * kx_exp2({lit(-rT1 * L2E)} * T){term3});')
+                    S(f'  const double lF = {lit(math.log10(2.0))} * l2F;')
+                    S('  const double tc = -0.4 - 0.67 * lF + lP, td = 0.75 - 1.27 * lF - 0.14 * tc;')
+                    S('  F *= kx_exp2(l2F * (td * td) * kx_rcp(td * td + tc * tc));   // l2F / (1 + (tc / td)^2)')
+                elif kind == M.SRI:
+                    a, b, rc, d, e = t['sri'][r]
+                    S(f'  F *= {lit(d)} * pow(T, {lit(e)}) * pow({lit(a)} * exp({lit(-b)} * rcpT)'
+                      f' + exp({lit(-rc)} * T), 1.0 / (1.0 + lP * lP));')
+        fwd = _prod(wvar, self.nu_f[r]) or '1.0'
+        if self.rev[r]:
+            dnu = int(self.net[r].sum())
+            rev = _prod(wvar, self.nu_r[r]) or '1.0'
             c0 = '*'.join(['C0' if dnu < 0 else 'rcpC0'] * abs(dnu))
             rev_term = f'({c0}) * {rev}' if c0 else rev
             S(f'  q{r} = F * ({fwd} - {rev_term});')
@@ -678,17 +753,13 @@ def _emit_bk1_fp64(t, info, sched_window=1, wform=False, variant='fp64', arrh32=
 
 
 def _emit_bk1_live(t, info, variant='fp64', arrh32=False, order=None, waves=0):
-    """w-form BK1 (FP64 or mixed_valu) in a register-liveness order: reactions follow
-    liveness.order_reactions; g_k and w_k are computed at the species' first use; wd_k
-    starts at its first net coefficient and is stored (with its enthalpy term added to the
-    heat release sum) after its last one. The NASA-7 coefficients of both pieces sit in an
-    LDS table read at a per-lane offset (T > T_mid selects the piece without a branch).
-    waves > 0 asks the compiler for that many waves per SIMD (register budget 512/waves):
-    the mixed kernel runs 8 % faster at 2 (some VGPRs go to scratch, latency hides behind
-    the second wave); the FP64 kernel, with more live FP64 state, is faster at 1. Tried for
-    the mixed kernel's 128 spilled VGPRs, not kept: reading Y_k again at each species' first
-    use (through an opaque pointer) instead of keeping its concentration live, and scheduling
-    barriers every 1-16 reactions -- 126-166 spilled VGPRs in every combination."""
+    """Product-form BK1 (FP64 or mixed_valu), one wavefront per 64 states, in a register-liveness
+    order, for mechanisms too small to split (emit_bk1_split.pays): reactions follow
+    liveness.order_reactions; g_k, w_k and rg_k are computed at the species' first use; wd_k
+    starts at its first net coefficient and is stored (with its enthalpy term added to the heat
+    release sum) after its last one. The NASA-7 coefficients of both pieces sit in an LDS table
+    read at a per-lane offset (T > T_mid selects the piece without a branch). waves > 0 asks the
+    compiler for that many waves per SIMD (register budget 512/waves)."""
     from . import liveness
     N = int(t['n_species'])
     em = _RateEmitter(t, info)
@@ -709,13 +780,6 @@ def _emit_bk1_live(t, info, variant='fp64', arrh32=False, order=None, waves=0):
     S = _Src()
     S(f'__device__ const double {kname}_poly[{PT.size}] = {{' +
       ', '.join(_literal(v) for v in PT.reshape(-1)) + '};', 0)
-    if mixed:
-        S('__device__ __forceinline__ double kx_pow2v(double y)', 0)
-        S('{', 0)
-        S('const double n = __builtin_rint(y);')
-        S('const float m = __builtin_amdgcn_exp2f((float)(y - n));')
-        S('return __builtin_ldexp((double)m, (int)n);')
-        S('}', 0)
     attr = f' __attribute__((amdgpu_waves_per_eu({waves}, {waves})))' if waves else ''
     S(f'extern "C" __global__ void __launch_bounds__({BLOCK}){attr}', 0)
     S(f'{kname}(const int n_states, const long long offsetT, const long long offset,', 0)
@@ -772,9 +836,11 @@ def _emit_bk1_live(t, info, variant='fp64', arrh32=False, order=None, waves=0):
             P, o = f'P{_tag(tmid[k])}', 16 * k
             S(f'const double g{k} = {P}[{o}] * omlnT + {P}[{o + 1}] * T + {P}[{o + 2}] * T2 + '
               f'{P}[{o + 3}] * T3 + {P}[{o + 4}] * T4 + {P}[{o + 5}] * rcpT - {P}[{o + 6}];')
-            S(f'const double gl{k} = g{k} * {lit(L2E)};')
-            S(f'const double w{k} = c{k} * exp(g{k});')
-        em.emit_reaction_w(S, r, sidx, pow2='kx_pow2v' if mixed else 'exp2', fp64_falloff=not mixed)
+            S(f'const double e{k} = kx_exp(g{k});')
+            S(f'const double w{k} = c{k} * e{k};')
+            if G[:, k].any():
+                S(f'const double rg{k} = kx_rcp(e{k});')
+        em.emit_reaction_p(S, r, sidx)
         for k in np.flatnonzero(D[r]):
             k = int(k)
             nu = int(em.net[r, k])
@@ -1061,7 +1127,8 @@ HEADER = '''// GENERATED by kinetix_amd.gen.emit_hip for mechanism "{name}" -- d
 // {n_species} species ({n_active} active), {n_reactions} reactions. Target: gfx950 (CDNA4).
 #include <hip/hip_runtime.h>
 #include <math.h>
-#include "kx_rcp.h"      // kx_rcp: Newton-refined FP64 reciprocal (kinetix_amd/csrc)
+#include "kx_rcp.h"      // kx_rcp: refined FP64 reciprocal (kinetix_amd/csrc)
+#include "kx_exp.h"      // kx_exp2, kx_exp, kx_log2
 '''
 
 
@@ -1118,8 +1185,11 @@ def generate(tables, info, opts=None):
                     parts.append(BT.emit(tables, info, ps) if tile else emit_rolled.emit_bk2(tables, info, ps))
         parts.append(_with_pool('kx_thermo_fp64_k', _emit_thermo_fp64, tables, info))
         return '\n\n'.join(parts) + '\n'
-    order = None
-    if o['bk1_live']:
+    from . import emit_bk1_split as SP
+    order, split = None, o['bk1_live'] and SP.pays(tables, info)
+    if split:
+        parts.append(SP.emit(tables, info, 'fp64'))
+    elif o['bk1_live']:
         from . import liveness
         order = liveness.order_reactions(tables)
         parts.append(_with_pool('kx_bk1_fp64_k', _emit_bk1_live, tables, info, 'fp64', False, order,
@@ -1150,7 +1220,9 @@ def generate(tables, info, opts=None):
     from . import emit_mixed
     parts.append(_with_pool('kx_bk1_mixed_k', emit_mixed.emit, tables, info, o['mixed'],
                             lds=o['mixed_lds_pool']))
-    if o['bk1_live']:
+    if split:
+        parts.append(SP.emit(tables, info, 'mixed_valu'))
+    elif o['bk1_live']:
         parts.append(_with_pool('kx_bk1_mixed_valu_k', _emit_bk1_live, tables, info, 'mixed_valu',
                                 o['mixed_arrh32'], order, o['mixed_waves'], lds=o['lds_pool']))
     else:

@@ -2,23 +2,24 @@
 // 9 species (8 active), 21 reactions. Target: gfx950 (CDNA4).
 #include <hip/hip_runtime.h>
 #include <math.h>
-#include "kx_rcp.h"      // kx_rcp: Newton-refined FP64 reciprocal (kinetix_amd/csrc)
+#include "kx_rcp.h"      // kx_rcp: refined FP64 reciprocal (kinetix_amd/csrc)
+#include "kx_exp.h"      // kx_exp2, kx_exp, kx_log2
 
 
-__device__ double kx_bk1_fp64_k[76] = {1.4426950408889634, 496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, 1.5, 11.0, -0.21999999999999997, 10.0, 1000.0, 12186.596374704217, 8.205736608095969e-05, 45.37946752547428, -1.4, -75779.07893121493, 7.754887502163468, 1.51, -2490.1536763179456, -4.299027692777283, 2.67, -4566.491727125329, 1.570462931026041, 2.02, -9728.297161125503, 22.168520327912255, 35.14528036742985, 12.589885179290201, 31.723952184259364, -0.406, -12050.746610262851, 20.492283523798655, 0.6, 8.75352839227408, -2.32, -381.0007723999002, 0.19999999999999996, -9.999999999999999e+29, 0.8, -9.999999999999999e-31, 24.95393638235263, 3.255500733148386, -2882.189532064794, 0.015999, 23.984679905783736, -597.4916838512155, 25.522529810666775, -5771.63898738416, 0.002016, 24.522529810666775, 26.07704223964188, -214.16773600985246, 0.001008, 29.11147765933911, -6938.308654393763, 19.931568569324174, 24.78456615693749, 360.8181857521921, 0.018015, 48.06819724919299, -35159.80832188866, -11.26155130938291, 2127.1575135893813, 0.017006999999999998, 16.98815209769054, 1182.859295867297, 28.645814086990296, -8698.840043627297, 0.031998, 0.033006, 0.034013999999999996, -8.31446261815324};
+__device__ double kx_bk1_fp64_k[77] = {1.4426950408889634, 496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, 1.5, 11.0, -0.21999999999999997, 10.0, 1000.0, 12186.596374704217, 8.205736608095969e-05, 45770000000000.0, -1.4, -75779.07893121493, 216.0, 1.51, -2490.1536763179456, 0.0508, 2.67, -4566.491727125329, 2.9699999999999998, 2.02, -9728.297161125503, 4714000.0, 38000000000.0, 6165.0, 3547000000.0, -0.406, -12050.746610262851, 1475000.0, 0.6, 8.75352839227408, -2.32, -381.0007723999002, 0.3010299956639812, 0.19999999999999996, -1.4426950408889633e+30, 0.8, -1.4426950408889633e-30, 32500000.0, 9.549999999999999, -2882.189532064794, 0.015999, 16600000.0, -597.4916838512155, 48200000.0, -5771.63898738416, 0.002016, 24100000.0, 70790000.0, -214.16773600985246, 0.001008, 580000000.0, -6938.308654393763, 1000000.0, 28900000.0, 360.8181857521921, 0.018015, 295100000000000.0, -35159.80832188866, -11.26155130938291, 2127.1575135893813, 0.017006999999999998, 130000.0, 1182.859295867297, 420000000.0, -8698.840043627297, 0.031998, 0.033006, 0.034013999999999996, -8.31446261815324};
 __device__ const double kx_bk1_fp64_poly[288] = {2.99142337, -0.0003500322055, 9.389714483333335e-09, 7.692981816666665e-13, -7.913758949999998e-17, -835.033997, -1.35511017, 0.0, 2.99142337, 0.0003500322055, -1.8779428966666666e-08, -2.307894545e-12, 3.16550358e-16, -835.033997, 0.0, 0.0, 3.69757819, -0.0003067598445, 2.0980699833333335e-08, -1.479401233333333e-12, 5.682176549999999e-17, -1233.93018, 3.18916559, 0.0, 3.69757819, 0.0003067598445, -4.1961399666666664e-08, 4.4382037e-12, -2.27287062e-16, -1233.93018, 0.0, 0.0, 2.67214561, -0.001528146445, 1.4550433516666668e-07, -1.0008303249999999e-11, 3.195808934999999e-16, -29899.209, 6.86281681, 0.0, 2.67214561, 0.001528146445, -2.910086703333333e-07, 3.002490975e-11, -1.278323574e-15, -29899.209, 0.0, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, -0.460117638, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, 0.0, 0.0, 2.54205966, 1.377530955e-05, 5.171338916666667e-10, -3.7925561833333325e-13, 2.1840257499999995e-17, 29230.8027, 4.92030811, 0.0, 2.54205966, -1.377530955e-05, -1.0342677833333334e-09, 1.137766855e-12, -8.736102999999999e-17, 29230.8027, 0.0, 0.0, 2.86472886, -0.00052825224, 4.3180459666666676e-08, -2.5434889499999995e-12, 6.659793799999999e-17, 3683.62875, 5.70164073, 0.0, 2.86472886, 0.00052825224, -8.636091933333334e-08, 7.63046685e-12, -2.66391752e-16, 3683.62875, 0.0, 0.0, 4.0172109, -0.001119910065, 1.0560969166666667e-07, -9.520530833333331e-12, 5.395426749999999e-16, 111.856713, 3.78510215, 0.0, 4.0172109, 0.001119910065, -2.1121938333333332e-07, 2.85615925e-11, -2.1581707e-15, 111.856713, 0.0, 0.0, 4.57316685, -0.002168068195, 2.4578147e-07, -1.9574196416666664e-11, 7.158267799999999e-16, -18006.9609, 0.501136959, 0.0, 4.57316685, 0.002168068195, -4.9156294e-07, 5.872258925e-11, -2.86330712e-15, -18006.9609, 0.0, 0.0, 2.92664, -0.0007439885, 9.474601666666666e-08, -8.414199999999998e-12, 3.376675499999999e-16, -922.7977, 5.980528, 0.0, 2.92664, 0.0007439885, -1.8949203333333333e-07, 2.52426e-11, -1.3506701999999999e-15, -922.7977, 0.0, 0.0, 3.29812431, -0.000412472087, 1.3571692150000003e-07, 7.896195274999998e-12, -2.0674361199999996e-14, -1012.52087, -3.29409409, 0.0, 3.29812431, 0.000412472087, -2.71433843e-07, -2.3688585825e-11, 8.26974448e-14, -1012.52087, 0.0, 0.0, 3.2129364, -0.000563743175, 9.593584116666667e-08, -1.0948976916666665e-10, 4.3842769599999987e-14, -1005.24902, 6.03473759, 0.0, 3.2129364, 0.000563743175, -1.9187168233333332e-07, 3.284693075e-10, -1.753710784e-13, -1005.24902, 0.0, 0.0, 3.38684249, -0.00173749123, 1.0591160550000003e-06, -5.807151058333331e-10, 1.2532942349999995e-13, -30208.1133, 2.59023285, 0.0, 3.38684249, 0.00173749123, -2.11823211e-06, 1.7421453175e-09, -5.01317694e-13, -30208.1133, 0.0, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, -0.460117608, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, 0.0, 0.0, 2.94642878, 0.000819083245, -4.035052833333334e-07, 1.335702658333333e-10, -1.9453481799999996e-14, 29147.6445, 2.96399498, 0.0, 2.94642878, -0.000819083245, 8.070105666666667e-07, -4.007107975e-10, 7.78139272e-14, 29147.6445, 0.0, 0.0, 4.12530561, 0.001612724695, -1.087941151666667e-06, 4.832113691666665e-10, -1.0311868949999997e-13, 3346.30913, -0.69043296, 0.0, 4.12530561, -0.001612724695, 2.1758823033333334e-06, -1.4496341075e-09, 4.1247475799999997e-13, 3346.30913, 0.0, 0.0, 4.30179801, 0.002374560255, -3.5263815166666667e-06, 2.0230324499999997e-09, -4.64612562e-13, 294.80804, 3.71666245, 0.0, 4.30179801, -0.002374560255, 7.0527630333333326e-06, -6.06909735e-09, 1.8584502480000002e-12, 294.80804, 0.0, 0.0, 3.38875365, -0.003284612905, 2.475020966666667e-08, 3.8548379333333327e-10, -1.2357573749999998e-13, -17663.1465, 6.7853632, 0.0, 3.38875365, 0.003284612905, -4.950041933333333e-08, -1.15645138e-09, 4.9430295e-13, -17663.1465, 0.0, 0.0, 3.298677, -0.00070412, 6.60537e-07, -4.7012625e-10, 1.2224275e-13, -1020.9, 3.950372, 0.0, 3.298677, 0.00070412, -1.3210739999999999e-06, 1.41037875e-09, -4.889710000000001e-13, -1020.9, 0.0, 0.0};
 extern "C" __global__ void __launch_bounds__(256)
 kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
             const double pressure_R, const double pressure_,
             const double* __restrict__ state, double* __restrict__ rates, const double Tref)
 {
-  __shared__ double kx_bk1_fp64_k_s[76];
-  for (int b_ = threadIdx.x; b_ < 76; b_ += 4096) {
+  __shared__ double kx_bk1_fp64_k_s[77];
+  for (int b_ = threadIdx.x; b_ < 77; b_ += 4096) {
     double t_[16];
     #pragma unroll
-    for (int r_ = 0; r_ < 16; ++r_) t_[r_] = kx_bk1_fp64_k[min(b_ + r_ * 256, 75)];
+    for (int r_ = 0; r_ < 16; ++r_) t_[r_] = kx_bk1_fp64_k[min(b_ + r_ * 256, 76)];
     #pragma unroll
-    for (int r_ = 0; r_ < 16; ++r_) if (b_ + r_ * 256 < 76) kx_bk1_fp64_k_s[b_ + r_ * 256] = t_[r_];
+    for (int r_ = 0; r_ < 16; ++r_) if (b_ + r_ * 256 < 77) kx_bk1_fp64_k_s[b_ + r_ * 256] = t_[r_];
   }
   __syncthreads();
   __shared__ double poly_s[288];
@@ -77,28 +78,32 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   const double rcpC0 = kx_bk1_fp64_k_s[16] * T;
   double sum_h = 0.0;
   const double g0 = P1000000[0] * omlnT + P1000000[1] * T + P1000000[2] * T2 + P1000000[3] * T3 + P1000000[4] * T4 + P1000000[5] * rcpT - P1000000[6];
-  const double gl0 = g0 * kx_bk1_fp64_k_s[0];
-  const double w0 = c0 * exp(g0);
+  const double e0 = kx_exp(g0);
+  const double w0 = c0 * e0;
+  const double rg0 = kx_rcp(e0);
   const double g3 = P1000000[48] * omlnT + P1000000[49] * T + P1000000[50] * T2 + P1000000[51] * T3 + P1000000[52] * T4 + P1000000[53] * rcpT - P1000000[54];
-  const double gl3 = g3 * kx_bk1_fp64_k_s[0];
-  const double w3 = c3 * exp(g3);
+  const double e3 = kx_exp(g3);
+  const double w3 = c3 * e3;
+  const double rg3 = kx_rcp(e3);
   double q4;
   { // 5: H2 + M <=> H + H + M
-    double F = exp2(kx_bk1_fp64_k_s[17] + kx_bk1_fp64_k_s[18] * log2T + kx_bk1_fp64_k_s[19] * rcpT - gl0);
+    double F = kx_bk1_fp64_k_s[17] * kx_exp2(kx_bk1_fp64_k_s[18] * log2T + kx_bk1_fp64_k_s[19] * rcpT) * rg0;
     F *= eff0;
     q4 = F * (w0 - (rcpC0) * w3*w3);
   }
   double wd0 = -q4;
   double wd3 = 2.0 * q4;
   const double g2 = P1000000[32] * omlnT + P1000000[33] * T + P1000000[34] * T2 + P1000000[35] * T3 + P1000000[36] * T4 + P1000000[37] * rcpT - P1000000[38];
-  const double gl2 = g2 * kx_bk1_fp64_k_s[0];
-  const double w2 = c2 * exp(g2);
+  const double e2 = kx_exp(g2);
+  const double w2 = c2 * e2;
+  const double rg2 = kx_rcp(e2);
   const double g5 = P1000000[80] * omlnT + P1000000[81] * T + P1000000[82] * T2 + P1000000[83] * T3 + P1000000[84] * T4 + P1000000[85] * rcpT - P1000000[86];
-  const double gl5 = g5 * kx_bk1_fp64_k_s[0];
-  const double w5 = c5 * exp(g5);
+  const double e5 = kx_exp(g5);
+  const double w5 = c5 * e5;
+  const double rg5 = kx_rcp(e5);
   double q2;
   { // 3: H2 + OH <=> H2O + H
-    double F = exp2(kx_bk1_fp64_k_s[20] + kx_bk1_fp64_k_s[21] * log2T + kx_bk1_fp64_k_s[22] * rcpT - gl0 - gl5);
+    double F = kx_bk1_fp64_k_s[20] * kx_exp2(kx_bk1_fp64_k_s[21] * log2T + kx_bk1_fp64_k_s[22] * rcpT) * rg0 * rg5;
     q2 = F * (w0*w5 - w2*w3);
   }
   wd0 += -q2;
@@ -106,11 +111,12 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd3 += q2;
   double wd5 = -q2;
   const double g4 = P1000000[64] * omlnT + P1000000[65] * T + P1000000[66] * T2 + P1000000[67] * T3 + P1000000[68] * T4 + P1000000[69] * rcpT - P1000000[70];
-  const double gl4 = g4 * kx_bk1_fp64_k_s[0];
-  const double w4 = c4 * exp(g4);
+  const double e4 = kx_exp(g4);
+  const double w4 = c4 * e4;
+  const double rg4 = kx_rcp(e4);
   double q1;
   { // 2: O + H2 <=> H + OH
-    double F = exp2(kx_bk1_fp64_k_s[23] + kx_bk1_fp64_k_s[24] * log2T + kx_bk1_fp64_k_s[25] * rcpT - gl0 - gl4);
+    double F = kx_bk1_fp64_k_s[23] * kx_exp2(kx_bk1_fp64_k_s[24] * log2T + kx_bk1_fp64_k_s[25] * rcpT) * rg0 * rg4;
     q1 = F * (w0*w4 - w3*w5);
   }
   wd0 += -q1;
@@ -119,7 +125,7 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd5 += q1;
   double q3;
   { // 4: O + H2O <=> OH + OH
-    double F = exp2(kx_bk1_fp64_k_s[26] + kx_bk1_fp64_k_s[27] * log2T + kx_bk1_fp64_k_s[28] * rcpT - gl2 - gl4);
+    double F = kx_bk1_fp64_k_s[26] * kx_exp2(kx_bk1_fp64_k_s[27] * log2T + kx_bk1_fp64_k_s[28] * rcpT) * rg2 * rg4;
     q3 = F * (w2*w4 - w5*w5);
   }
   wd2 += -q3;
@@ -127,7 +133,7 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd5 += 2.0 * q3;
   double q6;
   { // 7: O + H + M <=> OH + M
-    double F = exp2(kx_bk1_fp64_k_s[29] + -1.0 * log2T - gl3 - gl4);
+    double F = kx_bk1_fp64_k_s[29] * rcpT * rg3 * rg4;
     F *= eff0;
     q6 = F * (w3*w4 - (C0) * w5);
   }
@@ -136,7 +142,7 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd5 += q6;
   double q7;
   { // 8: H + OH + M <=> H2O + M
-    double F = exp2(kx_bk1_fp64_k_s[30] + -2.0 * log2T - gl3 - gl5);
+    double F = kx_bk1_fp64_k_s[30] * rcpT2 * rg3 * rg5;
     F *= eff0;
     q7 = F * (w3*w5 - (C0) * w2);
   }
@@ -144,11 +150,12 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd3 += -q7;
   wd5 += -q7;
   const double g1 = P1000000[16] * omlnT + P1000000[17] * T + P1000000[18] * T2 + P1000000[19] * T3 + P1000000[20] * T4 + P1000000[21] * rcpT - P1000000[22];
-  const double gl1 = g1 * kx_bk1_fp64_k_s[0];
-  const double w1 = c1 * exp(g1);
+  const double e1 = kx_exp(g1);
+  const double w1 = c1 * e1;
+  const double rg1 = kx_rcp(e1);
   double q5;
   { // 6: O + O + M <=> O2 + M
-    double F = exp2(kx_bk1_fp64_k_s[31] + -0.5 * log2T - gl4 - gl4);
+    double F = kx_bk1_fp64_k_s[31] * kx_exp2(-0.5 * log2T) * rg4 * rg4;
     F *= eff0;
     q5 = F * (w4*w4 - (C0) * w1);
   }
@@ -156,7 +163,7 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd4 += -2.0 * q5;
   double q0;
   { // 1: H + O2 <=> O + OH
-    double F = exp2(kx_bk1_fp64_k_s[32] + kx_bk1_fp64_k_s[33] * log2T + kx_bk1_fp64_k_s[34] * rcpT - gl1 - gl3);
+    double F = kx_bk1_fp64_k_s[32] * kx_exp2(kx_bk1_fp64_k_s[33] * log2T + kx_bk1_fp64_k_s[34] * rcpT) * rg1 * rg3;
     q0 = F * (w1*w3 - w4*w5);
   }
   wd1 += -q0;
@@ -164,18 +171,20 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd4 += q0;
   wd5 += q0;
   const double g6 = P1000000[96] * omlnT + P1000000[97] * T + P1000000[98] * T2 + P1000000[99] * T3 + P1000000[100] * T4 + P1000000[101] * rcpT - P1000000[102];
-  const double gl6 = g6 * kx_bk1_fp64_k_s[0];
-  const double w6 = c6 * exp(g6);
+  const double e6 = kx_exp(g6);
+  const double w6 = c6 * e6;
+  const double rg6 = kx_rcp(e6);
   double q8;
   { // 9: H + O2 (+M) <=> HO2 (+M)
-    double F = exp2(kx_bk1_fp64_k_s[35] + kx_bk1_fp64_k_s[36] * log2T - gl1 - gl3);
-    const double Pr = eff1 * exp2(kx_bk1_fp64_k_s[37] + kx_bk1_fp64_k_s[38] * log2T + kx_bk1_fp64_k_s[39] * rcpT);
-    const double Pr1 = Pr / (1.0 + Pr);
-    const double logFc = log10(kx_bk1_fp64_k_s[40] * exp(kx_bk1_fp64_k_s[41] * T) + kx_bk1_fp64_k_s[42] * exp(kx_bk1_fp64_k_s[43] * T));
-    const double logPr = log10(Pr + 1e-300);
-    const double tc = -0.4 - 0.67 * logFc + logPr;
-    const double tf = tc / (0.75 - 1.27 * logFc - 0.14 * tc + 1e-300);
-    F *= Pr1 * exp10(logFc / (1.0 + tf * tf));
+    double F = kx_bk1_fp64_k_s[35] * kx_exp2(kx_bk1_fp64_k_s[36] * log2T) * rg1 * rg3;
+    const double y0 = kx_bk1_fp64_k_s[37] + kx_bk1_fp64_k_s[38] * log2T + kx_bk1_fp64_k_s[39] * rcpT;
+    const double Pr = eff1 * kx_exp2(y0);
+    F *= Pr * kx_rcp(1.0 + Pr);
+    const double lP = kx_bk1_fp64_k_s[40] * fmax(y0 + kx_log2(fmax(eff1, 1e-300)), -997.0);
+    const double l2F = kx_log2(kx_bk1_fp64_k_s[41] * kx_exp2(kx_bk1_fp64_k_s[42] * T) + kx_bk1_fp64_k_s[43] * kx_exp2(kx_bk1_fp64_k_s[44] * T));
+    const double lF = kx_bk1_fp64_k_s[40] * l2F;
+    const double tc = -0.4 - 0.67 * lF + lP, td = 0.75 - 1.27 * lF - 0.14 * tc;
+    F *= kx_exp2(l2F * (td * td) * kx_rcp(td * td + tc * tc));   // l2F / (1 + (tc / td)^2)
     q8 = F * (w1*w3 - (C0) * w6);
   }
   wd1 += -q8;
@@ -183,7 +192,7 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   double wd6 = q8;
   double q11;
   { // 12: HO2 + O <=> O2 + OH
-    double F = exp2(kx_bk1_fp64_k_s[44] - gl4 - gl6);
+    double F = kx_bk1_fp64_k_s[45] * rg4 * rg6;
     q11 = F * (w4*w6 - w1*w5);
   }
   wd1 += q11;
@@ -191,22 +200,23 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd5 += q11;
   wd6 += -q11;
   const double g7 = P1000000[112] * omlnT + P1000000[113] * T + P1000000[114] * T2 + P1000000[115] * T3 + P1000000[116] * T4 + P1000000[117] * rcpT - P1000000[118];
-  const double gl7 = g7 * kx_bk1_fp64_k_s[0];
-  const double w7 = c7 * exp(g7);
+  const double e7 = kx_exp(g7);
+  const double w7 = c7 * e7;
+  const double rg7 = kx_rcp(e7);
   double q18;
   { // 19: H2O2 + O <=> OH + HO2
-    double F = exp2(kx_bk1_fp64_k_s[45] + 2.0 * log2T + kx_bk1_fp64_k_s[46] * rcpT - gl4 - gl7);
+    double F = kx_bk1_fp64_k_s[46] * kx_exp2(2.0 * log2T + kx_bk1_fp64_k_s[47] * rcpT) * rg4 * rg7;
     q18 = F * (w4*w7 - w5*w6);
   }
   wd4 += -q18;
-  rates[id + offsetT + 4 * offset] = kx_bk1_fp64_k_s[47] * wd4;
+  rates[id + offsetT + 4 * offset] = kx_bk1_fp64_k_s[48] * wd4;
   sum_h += wd4 * (P1000000[72] + P1000000[73] * T + P1000000[74] * T2 + P1000000[75] * T3 + P1000000[76] * T4 + P1000000[77] * rcpT);
   wd5 += q18;
   wd6 += q18;
   double wd7 = -q18;
   double q9;
   { // 10: HO2 + H <=> H2 + O2
-    double F = exp2(kx_bk1_fp64_k_s[48] + kx_bk1_fp64_k_s[49] * rcpT - gl3 - gl6);
+    double F = kx_bk1_fp64_k_s[49] * kx_exp2(kx_bk1_fp64_k_s[50] * rcpT) * rg3 * rg6;
     q9 = F * (w3*w6 - w0*w1);
   }
   wd0 += q9;
@@ -215,18 +225,18 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd6 += -q9;
   double q17;
   { // 18: H2O2 + H <=> HO2 + H2
-    double F = exp2(kx_bk1_fp64_k_s[50] + kx_bk1_fp64_k_s[51] * rcpT - gl3 - gl7);
+    double F = kx_bk1_fp64_k_s[51] * kx_exp2(kx_bk1_fp64_k_s[52] * rcpT) * rg3 * rg7;
     q17 = F * (w3*w7 - w0*w6);
   }
   wd0 += q17;
-  rates[id + offsetT + 0 * offset] = kx_bk1_fp64_k_s[52] * wd0;
+  rates[id + offsetT + 0 * offset] = kx_bk1_fp64_k_s[53] * wd0;
   sum_h += wd0 * (P1000000[8] + P1000000[9] * T + P1000000[10] * T2 + P1000000[11] * T3 + P1000000[12] * T4 + P1000000[13] * rcpT);
   wd3 += -q17;
   wd6 += q17;
   wd7 += -q17;
   double q16;
   { // 17: H2O2 + H <=> H2O + OH
-    double F = exp2(kx_bk1_fp64_k_s[53] + kx_bk1_fp64_k_s[46] * rcpT - gl3 - gl7);
+    double F = kx_bk1_fp64_k_s[54] * kx_exp2(kx_bk1_fp64_k_s[47] * rcpT) * rg3 * rg7;
     q16 = F * (w3*w7 - w2*w5);
   }
   wd2 += q16;
@@ -235,17 +245,17 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd7 += -q16;
   double q10;
   { // 11: HO2 + H <=> OH + OH
-    double F = exp2(kx_bk1_fp64_k_s[54] + kx_bk1_fp64_k_s[55] * rcpT - gl3 - gl6);
+    double F = kx_bk1_fp64_k_s[55] * kx_exp2(kx_bk1_fp64_k_s[56] * rcpT) * rg3 * rg6;
     q10 = F * (w3*w6 - w5*w5);
   }
   wd3 += -q10;
-  rates[id + offsetT + 3 * offset] = kx_bk1_fp64_k_s[56] * wd3;
+  rates[id + offsetT + 3 * offset] = kx_bk1_fp64_k_s[57] * wd3;
   sum_h += wd3 * (P1000000[56] + P1000000[57] * T + P1000000[58] * T2 + P1000000[59] * T3 + P1000000[60] * T4 + P1000000[61] * rcpT);
   wd5 += 2.0 * q10;
   wd6 += -q10;
   double q20;
   { // 21: H2O2 + OH <=> HO2 + H2O
-    double F = exp2(kx_bk1_fp64_k_s[57] + kx_bk1_fp64_k_s[58] * rcpT - gl5 - gl7);
+    double F = kx_bk1_fp64_k_s[58] * kx_exp2(kx_bk1_fp64_k_s[59] * rcpT) * rg5 * rg7;
     q20 = F * (w5*w7 - w2*w6);
   }
   wd2 += q20;
@@ -254,7 +264,7 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd7 += -q20;
   double q19;
   { // 20: H2O2 + OH <=> HO2 + H2O
-    double F = exp2(kx_bk1_fp64_k_s[59] - gl5 - gl7);
+    double F = kx_bk1_fp64_k_s[60] * rg5 * rg7;
     q19 = F * (w5*w7 - w2*w6);
   }
   wd2 += q19;
@@ -263,34 +273,35 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd7 += -q19;
   double q12;
   { // 13: HO2 + OH <=> H2O + O2
-    double F = exp2(kx_bk1_fp64_k_s[60] + kx_bk1_fp64_k_s[61] * rcpT - gl5 - gl6);
+    double F = kx_bk1_fp64_k_s[61] * kx_exp2(kx_bk1_fp64_k_s[62] * rcpT) * rg5 * rg6;
     q12 = F * (w5*w6 - w1*w2);
   }
   wd1 += q12;
   wd2 += q12;
-  rates[id + offsetT + 2 * offset] = kx_bk1_fp64_k_s[62] * wd2;
+  rates[id + offsetT + 2 * offset] = kx_bk1_fp64_k_s[63] * wd2;
   sum_h += wd2 * (P1000000[40] + P1000000[41] * T + P1000000[42] * T2 + P1000000[43] * T3 + P1000000[44] * T4 + P1000000[45] * rcpT);
   wd5 += -q12;
   wd6 += -q12;
   double q15;
   { // 16: H2O2 (+M) <=> OH + OH (+M)
-    double F = exp2(kx_bk1_fp64_k_s[63] + kx_bk1_fp64_k_s[64] * rcpT - gl7);
-    const double Pr = eff0 * exp2(kx_bk1_fp64_k_s[65] + kx_bk1_fp64_k_s[66] * rcpT);
-    const double Pr1 = Pr / (1.0 + Pr);
-    const double logFc = log10(0.5 * exp(kx_bk1_fp64_k_s[41] * T) + 0.5 * exp(kx_bk1_fp64_k_s[43] * T));
-    const double logPr = log10(Pr + 1e-300);
-    const double tc = -0.4 - 0.67 * logFc + logPr;
-    const double tf = tc / (0.75 - 1.27 * logFc - 0.14 * tc + 1e-300);
-    F *= Pr1 * exp10(logFc / (1.0 + tf * tf));
+    double F = kx_bk1_fp64_k_s[64] * kx_exp2(kx_bk1_fp64_k_s[65] * rcpT) * rg7;
+    const double y0 = kx_bk1_fp64_k_s[66] + kx_bk1_fp64_k_s[67] * rcpT;
+    const double Pr = eff0 * kx_exp2(y0);
+    F *= Pr * kx_rcp(1.0 + Pr);
+    const double lP = kx_bk1_fp64_k_s[40] * fmax(y0 + kx_log2(fmax(eff0, 1e-300)), -997.0);
+    const double l2F = kx_log2(0.5 * kx_exp2(kx_bk1_fp64_k_s[42] * T) + 0.5 * kx_exp2(kx_bk1_fp64_k_s[44] * T));
+    const double lF = kx_bk1_fp64_k_s[40] * l2F;
+    const double tc = -0.4 - 0.67 * lF + lP, td = 0.75 - 1.27 * lF - 0.14 * tc;
+    F *= kx_exp2(l2F * (td * td) * kx_rcp(td * td + tc * tc));   // l2F / (1 + (tc / td)^2)
     q15 = F * (w7 - (rcpC0) * w5*w5);
   }
   wd5 += 2.0 * q15;
-  rates[id + offsetT + 5 * offset] = kx_bk1_fp64_k_s[67] * wd5;
+  rates[id + offsetT + 5 * offset] = kx_bk1_fp64_k_s[68] * wd5;
   sum_h += wd5 * (P1000000[88] + P1000000[89] * T + P1000000[90] * T2 + P1000000[91] * T3 + P1000000[92] * T4 + P1000000[93] * rcpT);
   wd7 += -q15;
   double q14;
   { // 15: HO2 + HO2 <=> H2O2 + O2
-    double F = exp2(kx_bk1_fp64_k_s[68] + kx_bk1_fp64_k_s[69] * rcpT - gl6 - gl6);
+    double F = kx_bk1_fp64_k_s[69] * kx_exp2(kx_bk1_fp64_k_s[70] * rcpT) * rg6 * rg6;
     q14 = F * (w6*w6 - w1*w7);
   }
   wd1 += q14;
@@ -298,20 +309,20 @@ kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,
   wd7 += q14;
   double q13;
   { // 14: HO2 + HO2 <=> H2O2 + O2
-    double F = exp2(kx_bk1_fp64_k_s[70] + kx_bk1_fp64_k_s[71] * rcpT - gl6 - gl6);
+    double F = kx_bk1_fp64_k_s[71] * kx_exp2(kx_bk1_fp64_k_s[72] * rcpT) * rg6 * rg6;
     q13 = F * (w6*w6 - w1*w7);
   }
   wd1 += q13;
-  rates[id + offsetT + 1 * offset] = kx_bk1_fp64_k_s[72] * wd1;
+  rates[id + offsetT + 1 * offset] = kx_bk1_fp64_k_s[73] * wd1;
   sum_h += wd1 * (P1000000[24] + P1000000[25] * T + P1000000[26] * T2 + P1000000[27] * T3 + P1000000[28] * T4 + P1000000[29] * rcpT);
   wd6 += -2.0 * q13;
-  rates[id + offsetT + 6 * offset] = kx_bk1_fp64_k_s[73] * wd6;
+  rates[id + offsetT + 6 * offset] = kx_bk1_fp64_k_s[74] * wd6;
   sum_h += wd6 * (P1000000[104] + P1000000[105] * T + P1000000[106] * T2 + P1000000[107] * T3 + P1000000[108] * T4 + P1000000[109] * rcpT);
   wd7 += q13;
-  rates[id + offsetT + 7 * offset] = kx_bk1_fp64_k_s[74] * wd7;
+  rates[id + offsetT + 7 * offset] = kx_bk1_fp64_k_s[75] * wd7;
   sum_h += wd7 * (P1000000[120] + P1000000[121] * T + P1000000[122] * T2 + P1000000[123] * T3 + P1000000[124] * T4 + P1000000[125] * rcpT);
   rates[id + offsetT + 8 * offset] = 0.0;
-  rates[id] = kx_bk1_fp64_k_s[75] * T * sum_h;
+  rates[id] = kx_bk1_fp64_k_s[76] * T * sum_h;
 }
 
 __device__ double kx_bk2_fp64_k[413] = {496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, -0.008078545001735974, 0.004640788076965983, -0.0008759648030331312, 7.705769878407621e-05, -2.4732690890948386e-06, -0.009701327965813461, 0.004014325009517167, -0.00046791121609389516, 1.9380878155402322e-05, 9.240931195427016e-08, 0.004416853642772773, -0.003177573597181277, 0.0008133762876392088, -8.454229462698178e-05, 3.1913602502646043e-06, -0.02494681207473229, 0.013946115930444028, -0.0026011928734167586, 0.00022520946625312265, -7.131543528603997e-06, -0.01978919058591089, 0.009984564215123963, -0.0017087964642905347, 0.00013470040249623274, -3.857904702508071e-06, 0.031782681005851694, -0.021944709939377426, 0.005452754910092157, -0.0005578687529719978, 2.081257384420758e-05, -0.009169918908787118, 0.005424364464357365, -0.0010322095278337612, 9.207446814291079e-05, -2.9857817128234677e-06, -0.004562289268899475, 0.002451084127422514, -0.0004462621814763049, 3.755034814762184e-05, -1.157471595806185e-06, -0.0005572856088248942, -0.0005667709603605706, 0.0003231082930933187, -4.3068136081084276e-05, 1.8913297388140362e-06, -0.02669027788754572, 0.013931611307090428, -0.0024745908346480517, 0.00020278396526946714, -6.0779893075179144e-06, -0.009139457743520542, 0.005406345497771159, -0.0010287806747187474, 9.176860986668201e-05, -2.9758633710047717e-06, -0.00447124565900482, 0.002402171063395955, -0.00043735671372372337, 3.6801005208845666e-05, -1.134373456642212e-06, -0.0005484689037145654, -0.0005578041893842721, 0.00031799646085891946, -4.2386763640324535e-05, 1.861407386056745e-06, -0.026643356521131357, 0.013907119608599413, -0.002470240517141307, 0.00020242747213886954, -6.067304234706083e-06, -0.00610805793895662, 0.003368407717981707, -0.0006236209254916101, 5.35018330210794e-05, -1.6801339433900964e-06, -0.008071230238450928, 0.004636586049716245, -0.000875171655852957, 7.698792646406944e-05, -2.471029653901744e-06, -0.003103321303261743, 0.001620714531033315, -0.0002880080052608885, 2.361277988302796e-05, -7.081063564031256e-07, 0.0021021151307411773, -0.0018281498403758074, 0.0005252030760262369, -5.765803219995976e-05, 2.261877759925591e-06, -0.01977995988629229, 0.009979906899153058, -0.0017079993934378086, 0.00013463757127695383, -3.856105176642129e-06, -0.00453900788868428, 0.0024385762354091935, -0.0004439849037963053, 3.7358728572273574e-05, -1.1515650136680093e-06, -0.0044474877159452345, 0.0023894071385980073, -0.00043503282085484055, 3.6605463238430545e-05, -1.128345968543702e-06, -0.008064342962574994, 0.004632629596200829, -0.0008744248615664428, 7.69222317592718e-05, -2.4689210951839414e-06, -0.003080603052233275, 0.0016088498879742715, -0.00028589960670274603, 2.343991958002464e-05, -7.029225754199007e-07, 0.002091088185931271, -0.0018185600195835118, 0.0005224480483656208, -5.735557876659116e-05, 2.250012757457966e-06, -0.01977127235377411, 0.009975523636185077, -0.0017072492250684143, 0.00013457843727046, -3.8544115413058705e-06, -0.004516996851676411, 0.002426750833673122, -0.00044183188525341653, 3.717756467530665e-05, -1.1459807228342708e-06, -0.004425021460770202, 0.002377337171479474, -0.0004328352749623568, 3.6420552625893784e-05, -1.1226461869886008e-06, -0.003056268300680219, 0.0015961410249217102, -0.0002836411865881341, 2.325475952865116e-05, -6.973699462936345e-07, -0.007323280548518961, 0.004247486239705284, -0.0008033594542404216, 7.096837773058077e-05, -2.2842690699268453e-06, -0.0030300534762926507, 0.0015963119456045255, -0.00028558271238279467, 2.3589003022771934e-05, -7.128139183221726e-07, 0.0032788592659172256, -0.00250547772369024, 0.0006678164162055433, -7.083587044777799e-05, 2.7134922012112525e-06, -0.01855279389830936, 0.0094550381895321, -0.0016339242326464177, 0.0001301601496250026, -3.7729752245399467e-06, -0.004334076415420444, 0.0023487751084627826, -0.00043025471405932087, 3.645330576694408e-05, -1.1313281839182982e-06, -0.0042515394211224454, 0.0023040456622892163, -0.00042206105813855777, 3.57590987428835e-05, -1.1097834719835844e-06, -0.003008377376100812, 0.0015848924053416147, -0.00028353973870733935, 2.342025432013938e-05, -7.0771465983169e-07, -0.002987842465005617, 0.0015740740735393358, -0.000281604322168895, 2.326038978842067e-05, -7.028838637541137e-07, 0.12027235504272604, 0.002016, 0.031998, 0.018015, 0.001008, 0.015999, 0.017006999999999998, 0.033006, 0.034013999999999996, 0.028014, -0.00032862351581483524, 0.0004740294432841943, -8.852339013585402e-05, 8.188000383370648e-06, -2.7751168466432606e-07, -0.006186428071776672, 0.0036188245122608246, -0.0006861983404511037, 5.916012709636698e-05, -1.9049771784408624e-06, 0.009686042407342398, -0.005171565609328, 0.0010297953041896915, -8.310422563573157e-05, 2.354038528031193e-06, -0.005094323314826246, 0.002811619155977377, -0.0005132615516489704, 4.251063805997887e-05, -1.315280069428127e-06, -0.00493602340766566, 0.0030943263930736814, -0.0006001283031197708, 5.318270134909568e-05, -1.7573576309832766e-06, -0.005011998459919715, 0.003141954126978508, -0.0006093654512091636, 5.400128711751042e-05, -1.7844068013008786e-06, -0.006234584035867565, 0.0036469939149016244, -0.0006915397979542224, 5.9620637252299345e-05, -1.9198057695974414e-06, -0.006281649296902439, 0.003674525297847103, -0.0006967602747207073, 6.007071713564113e-05, -1.93429850225971e-06, -0.00523250345894259, 0.003124981120294317, -0.0005968857242896726, 5.1908396951434225e-05, -1.6850989393098777e-06, 0.5855901795610634, 1.1688313766866358, 0.5790424617421424, 1.0011435340788952, 0.45180100180492244, 0.3799178428257963, 0.577221031059996, 0.9688191706725953, 0.5781821492964924, 0.9853691816620461, 0.5858554726647912, 1.17846335668192, 0.5861055914396313, 1.187866567986582, 0.5843626518920434, 1.1282454750636195, 0.2933835155678699, 0.14698656195273008, 0.4606439199892965, 0.39901865594136454, 0.24856753896630487, 0.1047198079220346, 0.45637761328314064, 0.38967321277930606, 0.5019271716268474, 0.5058342382850256, 0.5037745309672377, 0.5115286060914264, 0.4914866877666277, 0.4754171363284603, 0.3349071947099823, 0.19370397937838635, 0.5317867168954801, 0.6139169540608385, 0.2852810237328657, 0.13874886868757655, 0.49242068280067725, 0.47802535093447335, 0.49636276512795546, 0.4892688386299563, 0.5332593579911572, 0.6204090762707718, 0.5346635287638544, 0.6267385674946784, 0.5251863130881791, 0.5864737980346304, 0.537284965911771, 0.6389431042462725, 0.5900108360947904, 1.4004756540493521, 0.5865652330854575, 1.2060345555502854, 0.5901484899998148, 1.4117064242065558, 0.590278131912589, 1.422675943648791, 0.5893719327304141, 1.3532190343594586, 0.34390743782108935, 0.20489954354482498, 0.5072495179928722, 0.5225249110995452, 0.5386611186975299, 0.6455659904716762, 0.5399719543367936, 0.6520222570130803, 0.5310996819942161, 0.6109372600719221, 0.339258223198384, 0.19906554041450197, 0.5345004970202478, 0.6259964840511291, 0.5035595467215294, 0.5108606747104101, 0.28919053164284375, 0.14268958497128517, 0.49613799703295625, 0.48861722252465745, 0.5359262141538373, 0.632552092068409, 0.5281016203495429, 0.5982798184109316, 0.29124930606045696, 0.1447902464661838, 0.4980502831747219, 0.4942033398320063, 0.4583516807884874, 0.3939663882750188, 0.24670514653555417, 0.1031323986394481, 0.4494595518956552, 0.3750296462434639, 0.45406048073935207, 0.38470019701269975, 0.5018695242857543, 0.5056581684076131, 0.4894442530766966, 0.46978461587258163, 0.4561153626350659, 0.3891068173524205, 0.24491049741137022, 0.10161506669396154, 0.44717754391695114, 0.3703298924648816, 0.4981092665821893, 0.49437718261166247, 0.48744356316319537, 0.4643588147494246, 0.3026643726685863, 0.15676176803269137, 0.5080994053292183, 0.5252736485479127, 0.47030347200416284, 0.4211559788726505, 0.256691094546128, 0.11179751589804368, 0.4616953174228584, 0.4013607489460244, 0.46615532203069365, 0.4114753219535881, 0.509926610569937, 0.5312661177096261, 0.5116759275851055, 0.5371129596441585, -0.8503729092966488, 0.5051399280760361, -0.1104804550441928, 0.010639067121890734, -0.0003779077750558578, 0.08382372697003578, -0.05012782216213958, 0.011207048058734315, -0.001096674893926796, 4.018025027370487e-05, -0.4078841481366471, 0.2538669087825695, -0.05881256015913525, 0.006000160600397597, -0.0002255201175463123, -0.1916147865778396, 0.09553835562718409, -0.01652347249331514, 0.0012966391376799933, -3.7215514533395276e-05, 0.026829834800389706, -0.015740865784532876, 0.003721730592628103, -0.0003812998919268347, 1.469997421486766e-05, -0.2450231089634615, 0.15010008535956404, -0.03385280923529587, 0.0033641154802256526, -0.00012339729420903357, -0.018484431132663775, 0.01137376106367077, -0.0026436277213459916, 0.0002847169953556508, -1.0883625749554333e-05, -0.0743153856031247, 0.04626701894459687, -0.010888331203035992, 0.0011573863619973013, -4.533051653340974e-05, 0.00261278335752093, 0.0015933299717707057, -0.0009842997034338733, 0.00016507388594153203, -8.29740664451892e-06};
@@ -1738,26 +1749,20 @@ kx_bk1_mixed(const int n_states, const long long offsetT, const long long offset
   rates[id] = kx_bk1_mixed_k[229] * T * sum_h;
 }
 
-__device__ double kx_bk1_mixed_valu_k[26] = {1.4426950408889634, 496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, 1.5, 11.0, -0.21999999999999997, 10.0, 1000.0, 12186.596374704217, 8.205736608095969e-05, 0.015999, 0.002016, 0.001008, 0.018015, 0.017006999999999998, 0.031998, 0.033006, 0.034013999999999996, -8.31446261815324};
+__device__ double kx_bk1_mixed_valu_k[30] = {1.4426950408889634, 496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, 1.5, 11.0, -0.21999999999999997, 10.0, 1000.0, 12186.596374704217, 8.205736608095969e-05, 4714000.0, 38000000000.0, 32500000.0, 0.015999, 0.002016, 0.001008, 1000000.0, 0.018015, 0.017006999999999998, 0.031998, 0.033006, 0.034013999999999996, -8.31446261815324};
 __device__ const double kx_bk1_mixed_valu_poly[288] = {2.99142337, -0.0003500322055, 9.389714483333335e-09, 7.692981816666665e-13, -7.913758949999998e-17, -835.033997, -1.35511017, 0.0, 2.99142337, 0.0003500322055, -1.8779428966666666e-08, -2.307894545e-12, 3.16550358e-16, -835.033997, 0.0, 0.0, 3.69757819, -0.0003067598445, 2.0980699833333335e-08, -1.479401233333333e-12, 5.682176549999999e-17, -1233.93018, 3.18916559, 0.0, 3.69757819, 0.0003067598445, -4.1961399666666664e-08, 4.4382037e-12, -2.27287062e-16, -1233.93018, 0.0, 0.0, 2.67214561, -0.001528146445, 1.4550433516666668e-07, -1.0008303249999999e-11, 3.195808934999999e-16, -29899.209, 6.86281681, 0.0, 2.67214561, 0.001528146445, -2.910086703333333e-07, 3.002490975e-11, -1.278323574e-15, -29899.209, 0.0, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, -0.460117638, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, 0.0, 0.0, 2.54205966, 1.377530955e-05, 5.171338916666667e-10, -3.7925561833333325e-13, 2.1840257499999995e-17, 29230.8027, 4.92030811, 0.0, 2.54205966, -1.377530955e-05, -1.0342677833333334e-09, 1.137766855e-12, -8.736102999999999e-17, 29230.8027, 0.0, 0.0, 2.86472886, -0.00052825224, 4.3180459666666676e-08, -2.5434889499999995e-12, 6.659793799999999e-17, 3683.62875, 5.70164073, 0.0, 2.86472886, 0.00052825224, -8.636091933333334e-08, 7.63046685e-12, -2.66391752e-16, 3683.62875, 0.0, 0.0, 4.0172109, -0.001119910065, 1.0560969166666667e-07, -9.520530833333331e-12, 5.395426749999999e-16, 111.856713, 3.78510215, 0.0, 4.0172109, 0.001119910065, -2.1121938333333332e-07, 2.85615925e-11, -2.1581707e-15, 111.856713, 0.0, 0.0, 4.57316685, -0.002168068195, 2.4578147e-07, -1.9574196416666664e-11, 7.158267799999999e-16, -18006.9609, 0.501136959, 0.0, 4.57316685, 0.002168068195, -4.9156294e-07, 5.872258925e-11, -2.86330712e-15, -18006.9609, 0.0, 0.0, 2.92664, -0.0007439885, 9.474601666666666e-08, -8.414199999999998e-12, 3.376675499999999e-16, -922.7977, 5.980528, 0.0, 2.92664, 0.0007439885, -1.8949203333333333e-07, 2.52426e-11, -1.3506701999999999e-15, -922.7977, 0.0, 0.0, 3.29812431, -0.000412472087, 1.3571692150000003e-07, 7.896195274999998e-12, -2.0674361199999996e-14, -1012.52087, -3.29409409, 0.0, 3.29812431, 0.000412472087, -2.71433843e-07, -2.3688585825e-11, 8.26974448e-14, -1012.52087, 0.0, 0.0, 3.2129364, -0.000563743175, 9.593584116666667e-08, -1.0948976916666665e-10, 4.3842769599999987e-14, -1005.24902, 6.03473759, 0.0, 3.2129364, 0.000563743175, -1.9187168233333332e-07, 3.284693075e-10, -1.753710784e-13, -1005.24902, 0.0, 0.0, 3.38684249, -0.00173749123, 1.0591160550000003e-06, -5.807151058333331e-10, 1.2532942349999995e-13, -30208.1133, 2.59023285, 0.0, 3.38684249, 0.00173749123, -2.11823211e-06, 1.7421453175e-09, -5.01317694e-13, -30208.1133, 0.0, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, -0.460117608, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, 0.0, 0.0, 2.94642878, 0.000819083245, -4.035052833333334e-07, 1.335702658333333e-10, -1.9453481799999996e-14, 29147.6445, 2.96399498, 0.0, 2.94642878, -0.000819083245, 8.070105666666667e-07, -4.007107975e-10, 7.78139272e-14, 29147.6445, 0.0, 0.0, 4.12530561, 0.001612724695, -1.087941151666667e-06, 4.832113691666665e-10, -1.0311868949999997e-13, 3346.30913, -0.69043296, 0.0, 4.12530561, -0.001612724695, 2.1758823033333334e-06, -1.4496341075e-09, 4.1247475799999997e-13, 3346.30913, 0.0, 0.0, 4.30179801, 0.002374560255, -3.5263815166666667e-06, 2.0230324499999997e-09, -4.64612562e-13, 294.80804, 3.71666245, 0.0, 4.30179801, -0.002374560255, 7.0527630333333326e-06, -6.06909735e-09, 1.8584502480000002e-12, 294.80804, 0.0, 0.0, 3.38875365, -0.003284612905, 2.475020966666667e-08, 3.8548379333333327e-10, -1.2357573749999998e-13, -17663.1465, 6.7853632, 0.0, 3.38875365, 0.003284612905, -4.950041933333333e-08, -1.15645138e-09, 4.9430295e-13, -17663.1465, 0.0, 0.0, 3.298677, -0.00070412, 6.60537e-07, -4.7012625e-10, 1.2224275e-13, -1020.9, 3.950372, 0.0, 3.298677, 0.00070412, -1.3210739999999999e-06, 1.41037875e-09, -4.889710000000001e-13, -1020.9, 0.0, 0.0};
-__device__ __forceinline__ double kx_pow2v(double y)
-{
-  const double n = __builtin_rint(y);
-  const float m = __builtin_amdgcn_exp2f((float)(y - n));
-  return __builtin_ldexp((double)m, (int)n);
-}
 extern "C" __global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(2, 2)))
 kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long offset,
             const double pressure_R, const double pressure_,
             const double* __restrict__ state, double* __restrict__ rates, const double Tref)
 {
-  __shared__ double kx_bk1_mixed_valu_k_s[26];
-  for (int b_ = threadIdx.x; b_ < 26; b_ += 4096) {
+  __shared__ double kx_bk1_mixed_valu_k_s[30];
+  for (int b_ = threadIdx.x; b_ < 30; b_ += 4096) {
     double t_[16];
     #pragma unroll
-    for (int r_ = 0; r_ < 16; ++r_) t_[r_] = kx_bk1_mixed_valu_k[min(b_ + r_ * 256, 25)];
+    for (int r_ = 0; r_ < 16; ++r_) t_[r_] = kx_bk1_mixed_valu_k[min(b_ + r_ * 256, 29)];
     #pragma unroll
-    for (int r_ = 0; r_ < 16; ++r_) if (b_ + r_ * 256 < 26) kx_bk1_mixed_valu_k_s[b_ + r_ * 256] = t_[r_];
+    for (int r_ = 0; r_ < 16; ++r_) if (b_ + r_ * 256 < 30) kx_bk1_mixed_valu_k_s[b_ + r_ * 256] = t_[r_];
   }
   __syncthreads();
   __shared__ double poly_s[288];
@@ -1816,30 +1821,32 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   const double rcpC0 = kx_bk1_mixed_valu_k_s[16] * T;
   double sum_h = 0.0;
   const double g0 = P1000000[0] * omlnT + P1000000[1] * T + P1000000[2] * T2 + P1000000[3] * T3 + P1000000[4] * T4 + P1000000[5] * rcpT - P1000000[6];
-  const double gl0 = g0 * kx_bk1_mixed_valu_k_s[0];
-  const double w0 = c0 * exp(g0);
+  const double e0 = kx_exp(g0);
+  const double w0 = c0 * e0;
+  const double rg0 = kx_rcp(e0);
   const double g3 = P1000000[48] * omlnT + P1000000[49] * T + P1000000[50] * T2 + P1000000[51] * T3 + P1000000[52] * T4 + P1000000[53] * rcpT - P1000000[54];
-  const double gl3 = g3 * kx_bk1_mixed_valu_k_s[0];
-  const double w3 = c3 * exp(g3);
+  const double e3 = kx_exp(g3);
+  const double w3 = c3 * e3;
+  const double rg3 = kx_rcp(e3);
   double q4;
   { // 5: H2 + M <=> H + H + M
-    const float ya = 45.37946752547428f + -1.4f * log2Tf + -75779.07893121493f * rcpTf;
-    double F = kx_pow2v((double)ya - gl0);
+    double F = kx_exp2_f32(45.37946752547428f + -1.4f * log2Tf + -75779.07893121493f * rcpTf) * rg0;
     F *= eff0;
     q4 = F * (w0 - (rcpC0) * w3*w3);
   }
   double wd0 = -q4;
   double wd3 = 2.0 * q4;
   const double g2 = P1000000[32] * omlnT + P1000000[33] * T + P1000000[34] * T2 + P1000000[35] * T3 + P1000000[36] * T4 + P1000000[37] * rcpT - P1000000[38];
-  const double gl2 = g2 * kx_bk1_mixed_valu_k_s[0];
-  const double w2 = c2 * exp(g2);
+  const double e2 = kx_exp(g2);
+  const double w2 = c2 * e2;
+  const double rg2 = kx_rcp(e2);
   const double g5 = P1000000[80] * omlnT + P1000000[81] * T + P1000000[82] * T2 + P1000000[83] * T3 + P1000000[84] * T4 + P1000000[85] * rcpT - P1000000[86];
-  const double gl5 = g5 * kx_bk1_mixed_valu_k_s[0];
-  const double w5 = c5 * exp(g5);
+  const double e5 = kx_exp(g5);
+  const double w5 = c5 * e5;
+  const double rg5 = kx_rcp(e5);
   double q2;
   { // 3: H2 + OH <=> H2O + H
-    const float ya = 7.754887502163468f + 1.51f * log2Tf + -2490.1536763179456f * rcpTf;
-    double F = kx_pow2v((double)ya - gl0 - gl5);
+    double F = kx_exp2_f32(7.754887502163468f + 1.51f * log2Tf + -2490.1536763179456f * rcpTf) * rg0 * rg5;
     q2 = F * (w0*w5 - w2*w3);
   }
   wd0 += -q2;
@@ -1847,12 +1854,12 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd3 += q2;
   double wd5 = -q2;
   const double g4 = P1000000[64] * omlnT + P1000000[65] * T + P1000000[66] * T2 + P1000000[67] * T3 + P1000000[68] * T4 + P1000000[69] * rcpT - P1000000[70];
-  const double gl4 = g4 * kx_bk1_mixed_valu_k_s[0];
-  const double w4 = c4 * exp(g4);
+  const double e4 = kx_exp(g4);
+  const double w4 = c4 * e4;
+  const double rg4 = kx_rcp(e4);
   double q1;
   { // 2: O + H2 <=> H + OH
-    const float ya = -4.299027692777283f + 2.67f * log2Tf + -4566.491727125329f * rcpTf;
-    double F = kx_pow2v((double)ya - gl0 - gl4);
+    double F = kx_exp2_f32(-4.299027692777283f + 2.67f * log2Tf + -4566.491727125329f * rcpTf) * rg0 * rg4;
     q1 = F * (w0*w4 - w3*w5);
   }
   wd0 += -q1;
@@ -1861,8 +1868,7 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd5 += q1;
   double q3;
   { // 4: O + H2O <=> OH + OH
-    const float ya = 1.570462931026041f + 2.02f * log2Tf + -9728.297161125503f * rcpTf;
-    double F = kx_pow2v((double)ya - gl2 - gl4);
+    double F = kx_exp2_f32(1.570462931026041f + 2.02f * log2Tf + -9728.297161125503f * rcpTf) * rg2 * rg4;
     q3 = F * (w2*w4 - w5*w5);
   }
   wd2 += -q3;
@@ -1870,8 +1876,7 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd5 += 2.0 * q3;
   double q6;
   { // 7: O + H + M <=> OH + M
-    const float ya = 22.168520327912255f + -1.0f * log2Tf;
-    double F = kx_pow2v((double)ya - gl3 - gl4);
+    double F = kx_bk1_mixed_valu_k_s[17] * rcpT * rg3 * rg4;
     F *= eff0;
     q6 = F * (w3*w4 - (C0) * w5);
   }
@@ -1880,8 +1885,7 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd5 += q6;
   double q7;
   { // 8: H + OH + M <=> H2O + M
-    const float ya = 35.14528036742985f + -2.0f * log2Tf;
-    double F = kx_pow2v((double)ya - gl3 - gl5);
+    double F = kx_bk1_mixed_valu_k_s[18] * rcpT2 * rg3 * rg5;
     F *= eff0;
     q7 = F * (w3*w5 - (C0) * w2);
   }
@@ -1889,12 +1893,12 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd3 += -q7;
   wd5 += -q7;
   const double g1 = P1000000[16] * omlnT + P1000000[17] * T + P1000000[18] * T2 + P1000000[19] * T3 + P1000000[20] * T4 + P1000000[21] * rcpT - P1000000[22];
-  const double gl1 = g1 * kx_bk1_mixed_valu_k_s[0];
-  const double w1 = c1 * exp(g1);
+  const double e1 = kx_exp(g1);
+  const double w1 = c1 * e1;
+  const double rg1 = kx_rcp(e1);
   double q5;
   { // 6: O + O + M <=> O2 + M
-    const float ya = 12.589885179290201f + -0.5f * log2Tf;
-    double F = kx_pow2v((double)ya - gl4 - gl4);
+    double F = kx_exp2_f32(12.589885179290201f + -0.5f * log2Tf) * rg4 * rg4;
     F *= eff0;
     q5 = F * (w4*w4 - (C0) * w1);
   }
@@ -1902,8 +1906,7 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd4 += -2.0 * q5;
   double q0;
   { // 1: H + O2 <=> O + OH
-    const float ya = 31.723952184259364f + -0.406f * log2Tf + -12050.746610262851f * rcpTf;
-    double F = kx_pow2v((double)ya - gl1 - gl3);
+    double F = kx_exp2_f32(31.723952184259364f + -0.406f * log2Tf + -12050.746610262851f * rcpTf) * rg1 * rg3;
     q0 = F * (w1*w3 - w4*w5);
   }
   wd1 += -q0;
@@ -1911,12 +1914,12 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd4 += q0;
   wd5 += q0;
   const double g6 = P1000000[96] * omlnT + P1000000[97] * T + P1000000[98] * T2 + P1000000[99] * T3 + P1000000[100] * T4 + P1000000[101] * rcpT - P1000000[102];
-  const double gl6 = g6 * kx_bk1_mixed_valu_k_s[0];
-  const double w6 = c6 * exp(g6);
+  const double e6 = kx_exp(g6);
+  const double w6 = c6 * e6;
+  const double rg6 = kx_rcp(e6);
   double q8;
   { // 9: H + O2 (+M) <=> HO2 (+M)
-    const float ya = 20.492283523798655f + 0.6f * log2Tf;
-    double F = kx_pow2v((double)ya - gl1 - gl3);
+    double F = kx_exp2_f32(20.492283523798655f + 0.6f * log2Tf) * rg1 * rg3;
     const float Pr = fminf((float)eff1 * __builtin_amdgcn_exp2f(fminf(8.75352839227408f + -2.32f * log2Tf + -381.0007723999002f * rcpTf, 100.0f)), 1e30f);
     const float Pr1 = Pr * __builtin_amdgcn_rcpf(1.0f + Pr);
     const float logFc = 0.3010299956639812f * __builtin_amdgcn_logf(0.19999999999999996f * __builtin_amdgcn_exp2f(-1.4426950408889633e+30f * Tf) + 0.8f * __builtin_amdgcn_exp2f(-1.4426950408889633e-30f * Tf));
@@ -1932,8 +1935,7 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   double wd6 = q8;
   double q11;
   { // 12: HO2 + O <=> O2 + OH
-    const float ya = 24.95393638235263f;
-    double F = kx_pow2v((double)ya - gl4 - gl6);
+    double F = kx_bk1_mixed_valu_k_s[19] * rg4 * rg6;
     q11 = F * (w4*w6 - w1*w5);
   }
   wd1 += q11;
@@ -1941,24 +1943,23 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd5 += q11;
   wd6 += -q11;
   const double g7 = P1000000[112] * omlnT + P1000000[113] * T + P1000000[114] * T2 + P1000000[115] * T3 + P1000000[116] * T4 + P1000000[117] * rcpT - P1000000[118];
-  const double gl7 = g7 * kx_bk1_mixed_valu_k_s[0];
-  const double w7 = c7 * exp(g7);
+  const double e7 = kx_exp(g7);
+  const double w7 = c7 * e7;
+  const double rg7 = kx_rcp(e7);
   double q18;
   { // 19: H2O2 + O <=> OH + HO2
-    const float ya = 3.255500733148386f + 2.0f * log2Tf + -2882.189532064794f * rcpTf;
-    double F = kx_pow2v((double)ya - gl4 - gl7);
+    double F = kx_exp2_f32(3.255500733148386f + 2.0f * log2Tf + -2882.189532064794f * rcpTf) * rg4 * rg7;
     q18 = F * (w4*w7 - w5*w6);
   }
   wd4 += -q18;
-  rates[id + offsetT + 4 * offset] = kx_bk1_mixed_valu_k_s[17] * wd4;
+  rates[id + offsetT + 4 * offset] = kx_bk1_mixed_valu_k_s[20] * wd4;
   sum_h += wd4 * (P1000000[72] + P1000000[73] * T + P1000000[74] * T2 + P1000000[75] * T3 + P1000000[76] * T4 + P1000000[77] * rcpT);
   wd5 += q18;
   wd6 += q18;
   double wd7 = -q18;
   double q9;
   { // 10: HO2 + H <=> H2 + O2
-    const float ya = 23.984679905783736f + -597.4916838512155f * rcpTf;
-    double F = kx_pow2v((double)ya - gl3 - gl6);
+    double F = kx_exp2_f32(23.984679905783736f + -597.4916838512155f * rcpTf) * rg3 * rg6;
     q9 = F * (w3*w6 - w0*w1);
   }
   wd0 += q9;
@@ -1967,20 +1968,18 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd6 += -q9;
   double q17;
   { // 18: H2O2 + H <=> HO2 + H2
-    const float ya = 25.522529810666775f + -5771.63898738416f * rcpTf;
-    double F = kx_pow2v((double)ya - gl3 - gl7);
+    double F = kx_exp2_f32(25.522529810666775f + -5771.63898738416f * rcpTf) * rg3 * rg7;
     q17 = F * (w3*w7 - w0*w6);
   }
   wd0 += q17;
-  rates[id + offsetT + 0 * offset] = kx_bk1_mixed_valu_k_s[18] * wd0;
+  rates[id + offsetT + 0 * offset] = kx_bk1_mixed_valu_k_s[21] * wd0;
   sum_h += wd0 * (P1000000[8] + P1000000[9] * T + P1000000[10] * T2 + P1000000[11] * T3 + P1000000[12] * T4 + P1000000[13] * rcpT);
   wd3 += -q17;
   wd6 += q17;
   wd7 += -q17;
   double q16;
   { // 17: H2O2 + H <=> H2O + OH
-    const float ya = 24.522529810666775f + -2882.189532064794f * rcpTf;
-    double F = kx_pow2v((double)ya - gl3 - gl7);
+    double F = kx_exp2_f32(24.522529810666775f + -2882.189532064794f * rcpTf) * rg3 * rg7;
     q16 = F * (w3*w7 - w2*w5);
   }
   wd2 += q16;
@@ -1989,19 +1988,17 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd7 += -q16;
   double q10;
   { // 11: HO2 + H <=> OH + OH
-    const float ya = 26.07704223964188f + -214.16773600985246f * rcpTf;
-    double F = kx_pow2v((double)ya - gl3 - gl6);
+    double F = kx_exp2_f32(26.07704223964188f + -214.16773600985246f * rcpTf) * rg3 * rg6;
     q10 = F * (w3*w6 - w5*w5);
   }
   wd3 += -q10;
-  rates[id + offsetT + 3 * offset] = kx_bk1_mixed_valu_k_s[19] * wd3;
+  rates[id + offsetT + 3 * offset] = kx_bk1_mixed_valu_k_s[22] * wd3;
   sum_h += wd3 * (P1000000[56] + P1000000[57] * T + P1000000[58] * T2 + P1000000[59] * T3 + P1000000[60] * T4 + P1000000[61] * rcpT);
   wd5 += 2.0 * q10;
   wd6 += -q10;
   double q20;
   { // 21: H2O2 + OH <=> HO2 + H2O
-    const float ya = 29.11147765933911f + -6938.308654393763f * rcpTf;
-    double F = kx_pow2v((double)ya - gl5 - gl7);
+    double F = kx_exp2_f32(29.11147765933911f + -6938.308654393763f * rcpTf) * rg5 * rg7;
     q20 = F * (w5*w7 - w2*w6);
   }
   wd2 += q20;
@@ -2010,8 +2007,7 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd7 += -q20;
   double q19;
   { // 20: H2O2 + OH <=> HO2 + H2O
-    const float ya = 19.931568569324174f;
-    double F = kx_pow2v((double)ya - gl5 - gl7);
+    double F = kx_bk1_mixed_valu_k_s[23] * rg5 * rg7;
     q19 = F * (w5*w7 - w2*w6);
   }
   wd2 += q19;
@@ -2020,20 +2016,18 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd7 += -q19;
   double q12;
   { // 13: HO2 + OH <=> H2O + O2
-    const float ya = 24.78456615693749f + 360.8181857521921f * rcpTf;
-    double F = kx_pow2v((double)ya - gl5 - gl6);
+    double F = kx_exp2_f32(24.78456615693749f + 360.8181857521921f * rcpTf) * rg5 * rg6;
     q12 = F * (w5*w6 - w1*w2);
   }
   wd1 += q12;
   wd2 += q12;
-  rates[id + offsetT + 2 * offset] = kx_bk1_mixed_valu_k_s[20] * wd2;
+  rates[id + offsetT + 2 * offset] = kx_bk1_mixed_valu_k_s[24] * wd2;
   sum_h += wd2 * (P1000000[40] + P1000000[41] * T + P1000000[42] * T2 + P1000000[43] * T3 + P1000000[44] * T4 + P1000000[45] * rcpT);
   wd5 += -q12;
   wd6 += -q12;
   double q15;
   { // 16: H2O2 (+M) <=> OH + OH (+M)
-    const float ya = 48.06819724919299f + -35159.80832188866f * rcpTf;
-    double F = kx_pow2v((double)ya - gl7);
+    double F = kx_exp2_f32(48.06819724919299f + -35159.80832188866f * rcpTf) * rg7;
     const float Pr = fminf((float)eff0 * __builtin_amdgcn_exp2f(fminf(-11.26155130938291f + 2127.1575135893813f * rcpTf, 100.0f)), 1e30f);
     const float Pr1 = Pr * __builtin_amdgcn_rcpf(1.0f + Pr);
     const float logFc = 0.3010299956639812f * __builtin_amdgcn_logf(0.5f * __builtin_amdgcn_exp2f(-1.4426950408889633e+30f * Tf) + 0.5f * __builtin_amdgcn_exp2f(-1.4426950408889633e-30f * Tf));
@@ -2045,13 +2039,12 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
     q15 = F * (w7 - (rcpC0) * w5*w5);
   }
   wd5 += 2.0 * q15;
-  rates[id + offsetT + 5 * offset] = kx_bk1_mixed_valu_k_s[21] * wd5;
+  rates[id + offsetT + 5 * offset] = kx_bk1_mixed_valu_k_s[25] * wd5;
   sum_h += wd5 * (P1000000[88] + P1000000[89] * T + P1000000[90] * T2 + P1000000[91] * T3 + P1000000[92] * T4 + P1000000[93] * rcpT);
   wd7 += -q15;
   double q14;
   { // 15: HO2 + HO2 <=> H2O2 + O2
-    const float ya = 16.98815209769054f + 1182.859295867297f * rcpTf;
-    double F = kx_pow2v((double)ya - gl6 - gl6);
+    double F = kx_exp2_f32(16.98815209769054f + 1182.859295867297f * rcpTf) * rg6 * rg6;
     q14 = F * (w6*w6 - w1*w7);
   }
   wd1 += q14;
@@ -2059,21 +2052,20 @@ kx_bk1_mixed_valu(const int n_states, const long long offsetT, const long long o
   wd7 += q14;
   double q13;
   { // 14: HO2 + HO2 <=> H2O2 + O2
-    const float ya = 28.645814086990296f + -8698.840043627297f * rcpTf;
-    double F = kx_pow2v((double)ya - gl6 - gl6);
+    double F = kx_exp2_f32(28.645814086990296f + -8698.840043627297f * rcpTf) * rg6 * rg6;
     q13 = F * (w6*w6 - w1*w7);
   }
   wd1 += q13;
-  rates[id + offsetT + 1 * offset] = kx_bk1_mixed_valu_k_s[22] * wd1;
+  rates[id + offsetT + 1 * offset] = kx_bk1_mixed_valu_k_s[26] * wd1;
   sum_h += wd1 * (P1000000[24] + P1000000[25] * T + P1000000[26] * T2 + P1000000[27] * T3 + P1000000[28] * T4 + P1000000[29] * rcpT);
   wd6 += -2.0 * q13;
-  rates[id + offsetT + 6 * offset] = kx_bk1_mixed_valu_k_s[23] * wd6;
+  rates[id + offsetT + 6 * offset] = kx_bk1_mixed_valu_k_s[27] * wd6;
   sum_h += wd6 * (P1000000[104] + P1000000[105] * T + P1000000[106] * T2 + P1000000[107] * T3 + P1000000[108] * T4 + P1000000[109] * rcpT);
   wd7 += q13;
-  rates[id + offsetT + 7 * offset] = kx_bk1_mixed_valu_k_s[24] * wd7;
+  rates[id + offsetT + 7 * offset] = kx_bk1_mixed_valu_k_s[28] * wd7;
   sum_h += wd7 * (P1000000[120] + P1000000[121] * T + P1000000[122] * T2 + P1000000[123] * T3 + P1000000[124] * T4 + P1000000[125] * rcpT);
   rates[id + offsetT + 8 * offset] = 0.0;
-  rates[id] = kx_bk1_mixed_valu_k_s[25] * T * sum_h;
+  rates[id] = kx_bk1_mixed_valu_k_s[29] * T * sum_h;
 }
 
 __device__ double kx_sur_k[10] = {496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, 0.12027235504272604};

@@ -1,0 +1,122 @@
+"""Production rates split over wavefronts (kinetix_amd/gen/emit_bk1_split.py) and the range-free
+exponentials they use (kinetix_amd/csrc/kx_exp.h)."""
+import os
+import re
+from decimal import Decimal, getcontext
+
+import numpy as np
+import pytest
+
+from kinetix_amd import states
+from kinetix_amd.gen import emit_bk1_split as SP
+from kinetix_amd.gen import tables
+from oracle import pyoracle as po
+
+ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
+P_ATM = 101325.0
+
+
+def load(mech):
+    return tables.load(os.path.join(ROOT, 'kinetix_amd', 'mechs', mech))
+
+
+@pytest.mark.parametrize('mech', ['gri30', 'NH3Konnov_edit', 'chempolimi_edit', 'synth40cov'])
+def test_plan_covers_every_reaction_and_sum(mech):
+    """Every reaction in one wavefront, every (wavefront, species) sum in one LDS slot of one
+    round, slots inside the rows and never shared within a round, and the sums of all
+    wavefronts added up give nu^T q."""
+    info, t = load(mech)
+    assert SP.pays(t, info)
+    p = SP.plan(t, info)
+    em = p['em']
+    assert sorted(r for rs in p['rs'] for r in rs) == list(range(em.R))
+    seen = {}
+    for rnd in p['rounds']:
+        assert len(set(rnd.values())) == len(rnd) and max(rnd.values()) < p['rows']
+        for key in rnd:
+            assert key not in seen
+            seen[key] = True
+    assert set(seen) == {(w, k) for w in range(p['waves']) for k in p['sums'][w]}
+    assert sorted([*p['wrow'].values(), *p['rrow'].values(), *p['crow'].values()]) == \
+        list(range(em.N + len(p['rrow']) + len(p['crow'])))
+    q = np.random.default_rng(1).normal(size=em.R)
+    wd = np.zeros(em.N)
+    for w, rs in enumerate(p['rs']):
+        part = {k: sum(em.net[r, k] * q[r] for r in rs) for k in p['sums'][w]}
+        for k, v in part.items():
+            wd[k] += v
+    np.testing.assert_allclose(wd, em.net.T @ q, rtol=1e-12, atol=1e-12)
+    assert not SP.pays(*reversed(load('LiDryer')))
+
+
+def _poly(body):
+    """Coefficients of a Horner chain, lowest first, from the C source."""
+    c = re.findall(r'(?:double p =|fma\(p, \w,) ([-0-9.e]+)\)?;', body)
+    return [Decimal(v) for v in reversed(c)]
+
+
+def test_exponential_polynomials():
+    """The polynomials of kx_exp.h against exp2, exp and log2 in 50 digits: relative error below
+    2.1e-17 (a fifth of FP64 rounding) over the reduced ranges, and ln 2's two parts exact."""
+    getcontext().prec = 50
+    src = open(os.path.join(ROOT, 'kinetix_amd', 'csrc', 'kx_exp.h')).read()
+    body = {n: src.split(f'double {n}(double')[1].split('\n}\n')[0] for n in ('kx_exp2', 'kx_exp', 'kx_log2')}
+    ln2 = Decimal(2).ln()
+    ev = lambda p, x: sum((c * x ** k for k, c in enumerate(p) if k), p[0])
+    grid = [Decimal(i) / 200 for i in range(-100, 101) if i]
+    p = [Decimal(float(c)) for c in _poly(body['kx_exp2'])]
+    assert len(p) == 12
+    assert max(abs(ev(p, x) / (x * ln2).exp() - 1) for x in grid) < Decimal('2.1e-17')
+    p = [Decimal(float(c)) for c in _poly(body['kx_exp'])]
+    assert len(p) == 12
+    assert max(abs(ev(p, x * ln2) / (x * ln2).exp() - 1) for x in grid) < Decimal('2.1e-17')
+    hi, lo = Decimal(0.6931471228599548), Decimal(5.7699990475432854e-08)
+    assert '0.6931471228599548' in body['kx_exp'] and '5.7699990475432854e-08' in body['kx_exp']
+    assert abs(hi + lo - ln2) <= Decimal(2) ** -78            # half a unit in the last place of lo
+    assert int(np.frexp(0.6931471228599548)[0] * 2 ** 24) == np.frexp(0.6931471228599548)[0] * 2 ** 24
+    p = [Decimal(float(c)) for c in _poly(body['kx_log2'])]
+    assert len(p) == 8
+    for i in range(1, 100):
+        m = (Decimal('0.5').sqrt() * (100 - i) + Decimal(2).sqrt() * i) / 100
+        if m == 1:
+            continue
+        s = (m - 1) / (m + 1)
+        assert abs(s * ev(p, s * s) / (m.ln() / ln2) - 1) < Decimal('2.1e-17')
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize('mech,n,p_atm', [('gri30', 1, 1.0), ('gri30', 63, 1.0), ('gri30', 1000, 20.0),
+                                          ('NH3Konnov_edit', 65, 0.05), ('NH3Konnov_edit', 257, 3.0),
+                                          ('chempolimi_edit', 64, 2000.0), ('synth40cov', 129, 1.0),
+                                          ('LiDryer', 300, 5.0)])
+def test_split_rates_at_group_edges(mech, n, p_atm):
+    """FP64 and mixed rates at state counts around the 64-state groups on a strided view, cold
+    and hot (300-3000 K, both NASA-7 pieces), against the oracle; nothing outside the view."""
+    import torch
+    from kinetix_amd.api import Kinetix
+    info, t = load(mech)
+    N, lo = int(t['n_species']), 3
+    ld = n + 11
+    s, _ = states.sample_any(ld, info['species'], t['W'], T_range=(300.0, 3000.0), seed=41 + n)
+    kx = Kinetix(mech, device=0)
+    got = {}
+    try:
+        kx.build(P_ATM, 1.0, states.reference_mass_fractions(info['species'], t['W']))
+        ds = torch.from_numpy(s).cuda().reshape(-1)[lo:]
+        for mixed in (False, True):
+            r = torch.full((N + 1, ld), np.nan, dtype=torch.float64, device='cuda')
+            kx.productionRates(n, ld, ld, p_atm, ds, r.reshape(-1)[lo:], mixed=mixed)
+            torch.cuda.synchronize()
+            got[mixed] = r.cpu().numpy()
+    finally:
+        kx.close()
+    orc = po.Oracle(t)
+    sub = np.ascontiguousarray(s[:, lo:lo + n])
+    ref, scale = orc.production_rates(sub, p_atm * P_ATM, scale=True)
+    # mixed: FP32 exponents up to 300 at 300 K, 300 ln 2 / 2^23 = 2.5e-5, and FP32 falloff
+    for mixed, tol in ((False, 1e-12), (True, 4e-5)):
+        a = got[mixed]
+        assert np.all(np.isnan(a[:, :lo])) and np.all(np.isnan(a[:, lo + n:]))
+        # against the magnitude of the terms each rate is the sum of
+        err = np.abs(a[:, lo:lo + n] - ref) / np.maximum(np.maximum(np.abs(ref), scale), 1e-300)
+        assert np.nanmax(err) < tol, (mixed, float(np.nanmax(err)))
