@@ -1,10 +1,10 @@
 """Production rates (BK1) with the reactions split over the wavefronts of a workgroup: kx_bk1_fp64
-and kx_bk1_mixed_valu for straight-line mechanisms (benchmark/okl/productionRates.okl:10-62,
+and kx_bk1_mixed_valu as straight-line code (benchmark/okl/productionRates.okl:10-62,
 kinetix/core/reaction_rates.py:616-1333).
 
-One lane still works on one state, but a workgroup's WAVES wavefronts share the same 64 states:
+One lane still works on one state, but a workgroup's 8 or 12 wavefronts share the same 64 states:
 
-  species    wavefront v takes the species k = v, v + WAVES, ...: Y, the Gibbs term g_k from the
+  species    wavefront v takes the species k = v, v + waves, ...: Y, the Gibbs term g_k from the
              LDS NASA-7 table, e = exp(g_k), and puts w_k = C_k e and rg_k = 1 / e into LDS rows of 64
              states (512 B: every access is conflict-free);
   reactions  each wavefront runs its own part of the reactions as straight-line code (product
@@ -27,11 +27,23 @@ wavefronts of 256 registers: 625 / 478 us, 15.4 us; 16: 949 / 774; two groups of
 workgroup in step: 715 / 566; a loop over groups instead of one per workgroup: 826 / 618 (the
 compiler hoists the constants and spills).
 
+Large mechanisms (shape) have one workgroup per CU; where the rows fill the LDS (plan's tight),
+partial sums share them, the NASA-7 table stays in global memory and a third body's C_k is w_k
+rg_k. Before, a loop over reaction descriptors with a state's species shared by 32 lanes (LDS
+gathers and atomics, 160+ instructions a reaction; here 26 to 56, as constants are in the code and
+equal exponentials are shared): 129 species / 1,231 reactions, 100,003 states FP64 1,732 -> 244
+us, mixed 1,310 -> 211, 1,000 states 1,253 -> 30; 160 / 1,000, 524,288 states 5,340 -> 1,825,
+mixed 4,164 -> 1,469, 1,000 states 1,298 -> 50. Of a group's 133,000 cycles at 160 / 1,000,
+loading Y takes 13,000 (nothing beside it hides that), the species 20,000, the reactions
+74,000 (61,000 of FP64 issue), the sums 11,000 (40,000 while each round took all sums of two or
+three wavefronts: one reloaded its spilled sums while the others waited), the rest the end.
+
 The reactions are dealt to the wavefronts by modelled cost with as few (wavefront, species) sums
-as possible (assign), and the values read from LDS are cached for SEGMENT reactions at a time.
+as possible (assign), and the values read from LDS are cached for a segment of reactions.
 """
 from __future__ import annotations
 
+import math
 import random
 
 import numpy as np
@@ -43,6 +55,8 @@ from . import mechanism as M
 WAVES = 8                # wavefronts that share 64 states' reactions
 SEGMENT = 6              # reactions between points where values read from LDS are dropped
 ROW = 64                 # states per workgroup
+LDS_MAX = 160 * 1024
+MAX_SUMS = 100           # sums of a wavefront that stay in registers (two each, of 256)
 
 
 def reaction_cost(em, r):
@@ -61,7 +75,7 @@ def reaction_cost(em, r):
     return c
 
 
-def assign(em, waves=WAVES, iters=40000, seed=7):
+def assign(em, waves=WAVES, seed=7):
     """Wavefront of every reaction: greedy by cost, then a seeded local search over moves and
     swaps, minimising the largest load (in cycles) plus 12 cycles per (wavefront, species) sum
     and 40 per (wavefront, third-body set)."""
@@ -100,10 +114,14 @@ def assign(em, waves=WAVES, iters=40000, seed=7):
 
     def score():
         per = [load[w] + 12 * len(cnt[w]) + 40 * len(scnt[w]) for w in range(waves)]
-        return waves * max(per) + sum(12 * len(c) for c in cnt) * 3
+        over = sum(max(0, len(c) - MAX_SUMS) for c in cnt)
+        return waves * max(per) + sum(12 * len(c) for c in cnt) * 3 + 2000 * over
     rng = random.Random(seed)
     cur = score()
-    for _ in range(iters):
+    # with sums beyond MAX_SUMS the search starts as an annealing (the descent gets stuck there)
+    hot = 300.0 if max(len(c) for c in cnt) > MAX_SUMS else 0.0
+    iters = 500 * R if hot else max(40000, 120 * R)
+    for it in range(iters):
         r = rng.randrange(R)
         a = where[r]
         if rng.random() < 0.5:
@@ -119,7 +137,7 @@ def assign(em, waves=WAVES, iters=40000, seed=7):
         if s is not None:
             put(s, b, -1); put(s, a, 1)
         new = score()
-        if new <= cur:
+        if new <= cur or (hot and rng.random() < math.exp((cur - new) / (hot * (1.0 - it / iters)))):
             cur = new
             where[r] = b
             if s is not None:
@@ -153,46 +171,78 @@ def plan(t, info, waves=WAVES):
     rs = [order(em, [r for r in range(em.R) if where[r] == w]) for w in range(waves)]
     sums = [sorted({int(k) for r in rs[w] for k in np.flatnonzero(em.net[r])}) for w in range(waves)]
     react = sorted({int(k) for r in range(em.R) for k in np.flatnonzero(em.nu_f[r])})
-    wrow = {k: i for i, k in enumerate(range(N))}
-    rrow = {k: N + i for i, k in enumerate(react)}
     third = sorted({int(k) for r in range(em.R) if em.kind[r] not in (M.ELEMENTARY, M.PLOG)
                     for k in ([int(j) for j in np.flatnonzero(em.t['eff'][r] != 1.0)] if em.has_eff[r]
                               else [int(em.t['collider'][r])] if em.t['collider'][r] >= 0 else [])})
+    # tight: no room for everything; the NASA-7 table stays in global memory, the wavefronts'
+    # partial sums share the rows, and C_k of a species with an rg row is w_k rg_k
+    tight = lds_bytes(N, N + len(react) + len(third), waves, False) > LDS_MAX
+    if tight:
+        third = [k for k in third if k not in react]
+    wrow = {k: i for i, k in enumerate(range(N))}
+    rrow = {k: N + i for i, k in enumerate(react)}
     crow = {k: N + len(react) + i for i, k in enumerate(third)}
-    rows = max(N + len(react) + len(third), waves)
+    rows = max(N + len(react) + len(third), waves + 1)
+    if tight:
+        rows = max(rows, LDS_MAX // (8 * ROW))      # one workgroup per CU: fewer rounds for the sums
+    # a round takes all wavefronts' sums of some species: every wavefront writes in every round
     rounds, cur, free = [], {}, rows
-    for w in range(waves):
-        if len(sums[w]) > rows:
-            raise ValueError('more sums in a wavefront than LDS rows')
-        if len(sums[w]) > free:
+    for k in range(N):
+        ws = [w for w in range(waves) if k in sums[w]]
+        if len(ws) > free:
             rounds.append(cur)
             cur, free = {}, rows
-        for k in sums[w]:
+        for w in ws:
             cur[(w, k)] = rows - free
             free -= 1
     rounds.append(cur)
     return dict(em=em, rs=rs, sums=sums, wrow=wrow, rrow=rrow, crow=crow, rows=rows, rounds=rounds,
-                waves=waves, where=where)
+                waves=waves, where=where, tight=tight)
 
 
-def lds_bytes(p):
-    return 8 * (ROW * (p['rows'] + p['waves'] + 1) + 2 * p['em'].N * 14)
+def lds_bytes(N, rows, waves, tight):
+    return 8 * ROW * rows if tight else 8 * (ROW * (rows + waves + 1) + 2 * N * 14)
+
+
+def shape(t, info):
+    """(plan, wavefronts per SIMD, reactions per segment) of a mechanism, or None when it does
+    not fit.
+
+    Two workgroups of 8 per CU at 128 registers where the LDS holds two and a wavefront's sums
+    stay in registers (53 species / 325 reactions: 617 us for 1,048,576 states; one workgroup
+    per CU of 4 wavefronts with all registers 625). Larger mechanisms have one workgroup per CU:
+    12 wavefronts of 168 registers up to 52 sums (129 / 1,231, 100,003 states: 251 us; 8 of 256
+    registers 262, 16 of 128, which spill, 305), else 8 of 256 up to 112 sums, with values from LDS
+    kept for three reactions at a time instead of six (160 / 1,000, 524,288 states, 108 sums:
+    2,205 us against 2,258 with four; 12 wavefronts would have 99 sums for 168 registers)."""
+    fits = lambda p: lds_bytes(p['em'].N, p['rows'], p['waves'], p['tight']) <= LDS_MAX
+    most = lambda p: max(len(s) for s in p['sums'])
+    p8 = plan(t, info)
+    if not fits(p8):
+        return None
+    if lds_bytes(p8['em'].N, p8['rows'], WAVES, p8['tight']) <= LDS_MAX // 2 and most(p8) <= 36:
+        return p8, 4, SEGMENT
+    p12 = plan(t, info, 12)
+    if fits(p12) and most(p12) <= 52:
+        return p12, 3, SEGMENT
+    return (p8, 2, SEGMENT if most(p8) <= 80 else 3) if most(p8) <= 112 else None
 
 
 def pays(t, info):
-    """Whether a straight-line mechanism's reactions are split. A state's modelled load has to be
-    worth the barriers and the per-wavefront prologue: 9 species / 21 reactions (5,000 cycles)
-    run 1,048,576 states in 56 us with one wavefront per 64 states and 132 split; 31 / 203
-    (41,000) in 1,234 and 423. The line lies between, at 16,000. The rows have to fit the LDS."""
+    """The shape if a mechanism's reactions are split, else None. A state's modelled load has to be worth the
+    barriers and the per-wavefront prologue: 9 species / 21 reactions (5,000 cycles) run
+    1,048,576 states in 56 us with one wavefront per 64 states and 132 split; 31 / 203
+    (41,000) in 1,234 and 423. The line lies between, at 16,000."""
     em = E._RateEmitter(t, info)
     if sum(reaction_cost(em, r) for r in range(em.R)) < 16000:
-        return False
-    return lds_bytes(plan(t, info)) <= 160 * 1024
+        return None
+    return shape(t, info)
 
 
-def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
-    p = plan(t, info, waves)
-    em = p['em']
+def emit(t, info, variant='fp64', shaped=None):
+    p, occupancy, segment = shaped or shape(t, info)
+    waves = p['waves']
+    em = E._RateEmitter(t, info)
     N = em.N
     mixed = variant == 'mixed_valu'
     em.arrh32 = mixed
@@ -227,11 +277,17 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
     S('            const double pressure_R, const double pressure_,', 0)
     S('            const double* __restrict__ state, double* __restrict__ rates, const double Tref)', 0)
     S('{', 0)
-    S(f'__shared__ __attribute__((aligned(16))) double poly_s[{PT.size}];')
+    staged, tight = not p['tight'], p['tight']
+    if staged:
+        S(f'__shared__ __attribute__((aligned(16))) double poly_s[{PT.size}];')
     S(f'__shared__ double rows[{p["rows"]} * {ROW}];        // w, rg, third-body C; then the wavefronts\' sums')
-    S(f'__shared__ double part[{waves + 1} * {ROW}];')
-    S(f'for (int i = threadIdx.x; i < {PT.size // 2}; i += {64 * waves})')
-    S(f'  ((double2*)poly_s)[i] = ((const double2*){name}_poly)[i];')
+    if tight:
+        S('double* const part = rows;               // before w is written and after the sums are read')
+    else:
+        S(f'__shared__ double part[{waves + 1} * {ROW}];')
+    if staged:
+        S(f'for (int i = threadIdx.x; i < {PT.size // 2}; i += {64 * waves})')
+        S(f'  ((double2*)poly_s)[i] = ((const double2*){name}_poly)[i];')
     S('const int lane = threadIdx.x & 63;')
     S('const int v = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);      // part of the reactions')
     S(f'const long long first = (long long)blockIdx.x * {ROW};')
@@ -261,6 +317,8 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
     S('#pragma unroll')
     S(f'for (int i = 0; i < {waves}; ++i) rcpMbar += part[i * {ROW} + lane];')
     S(f'const double lnT = part[{waves} * {ROW} + lane];')
+    if tight:
+        S('__syncthreads();')
     S('const double omlnT = 1.0 - lnT;')
     S('const double log2T = lnT * 1.4426950408889634;')
     S('const float Tf = (float)T, rcpTf = (float)rcpT, log2Tf = (float)log2T;')
@@ -273,7 +331,7 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
     S('// ---- species: w_k = C_k exp(g_k), rg_k = exp(-g_k), third-body concentrations')
     rr = [p['rrow'].get(k, -1) for k in range(N)]
     cr = [p['crow'].get(k, -1) for k in range(N)]
-    S(f'const double* const piece = poly_s;')
+    S(f'const double* const piece = {"poly_s" if staged else name + "_poly"};')
     for i in range(per):
         S('{')
         S(f'  const int k = v + {waves} * {i};')
@@ -308,12 +366,14 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
     S(f'for (int i = 0; i < {mx}; ++i) wd[i] = 0.0;')
     S('int o = lane;                                     // made opaque between segments')
     sets, sidx = em.efficiency_sets()
+    at = lambda row: f'rows[{row * ROW} + o]'
+    conc = lambda k: at(p['crow'][k]) if k in p['crow'] else f'({at(p["wrow"][k])} * {at(p["rrow"][k])})'
     for w in range(waves):
         S(f'{"if" if w == 0 else "else if"} (v == {w}) {{' if w < waves - 1 else 'else {')
         slot = {k: i for i, k in enumerate(p['sums'][w])}
         have_third, pins = set(), []
         for n, r in enumerate(p['rs'][w]):
-            if n % SEGMENT == 0:
+            if n % segment == 0:
                 # the segment's sums are needed as values here: the compiler otherwise defers
                 # them to the end of the wavefront's program, all values read from LDS alive
                 S(f'asm volatile("" : "+v"(o){"".join(f", {q}" for q in pins)});')
@@ -329,10 +389,10 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
                     terms = ['Cm']
                     for k, e in enumerate(sets[int(need[3:])]):
                         if e != 1.0:
-                            terms.append(f'+ {lit(e - 1.0)} * rows[{p["crow"][k] * ROW} + o]')
+                            terms.append(f'+ {lit(e - 1.0)} * {conc(k)}')
                     S(f'const double {need} = ' + ' '.join(terms) + ';')
                 else:
-                    S(f'const double {need} = rows[{p["crow"][int(need[1:])] * ROW} + o];')
+                    S(f'const double {need} = {conc(int(need[1:]))};')
             ks = sorted({int(k) for k in np.flatnonzero((em.nu_f[r] > 0) | (em.rev[r] & (em.nu_r[r] > 0)))})
             S(f'double q{r};')
             S('{')
@@ -363,7 +423,8 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
         for w in sorted({w for w, _ in rnd}):
             S(f'if (v == {w}) {{')
             for i, k in enumerate(p['sums'][w]):
-                S(f'  rows[{rnd[(w, k)] * ROW} + lane] = wd[{i}];')
+                if (w, k) in rnd:
+                    S(f'  rows[{rnd[(w, k)] * ROW} + lane] = wd[{i}];')
             S('}')
         S('__syncthreads();')
         for v in range(waves):
@@ -373,9 +434,24 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
                     if (w, k) in rnd:
                         S(f'  acc[{i}] += rows[{rnd[(w, k)] * ROW} + lane];')
             S('}')
-    S('// ---- mass production rates and heat release rate')
-    S('double sh = 0.0;')
+    S('// ---- heat release rate and mass production rates; the stores last, so that no table load waits')
+    S('// behind them; where registers are short powers of T again instead of held over the reactions')
+    S('double Te = T, sh = 0.0;')
+    if tight:
+        S('asm volatile("" : "+v"(Te));')
+    S('const double Te2 = Te * Te, Te3 = Te * Te * Te, Te4 = Te * Te * Te * Te;')
     W = t['W']
+    for v in range(waves):
+        S(f'{"if" if v == 0 else "else if"} (v == {v}) {{')
+        for i, k in enumerate(own[v]):
+            if k in em.active:
+                S(f'  {{ const double* a = piece + {14 * k + 8} + (T > {lit(float(t["T_mid"][k]))} ? 0 : {14 * N});')
+                S(f'    sh += acc[{i}] * (a[0] + a[1] * Te + a[2] * Te2 + a[3] * Te3 + a[4] * Te4 + a[5] * rcpT); }}')
+        S('}')
+    if tight:
+        S('__syncthreads();                       // the last round\'s rows read by all')
+    S(f'part[v * {ROW} + lane] = sh;')
+    S('__syncthreads();')
     for v in range(waves):
         S(f'{"if" if v == 0 else "else if"} (v == {v}) {{')
         S('  if (live) {')
@@ -383,13 +459,7 @@ def emit(t, info, variant='fp64', waves=WAVES, occupancy=4):
             val = f'{lit(W[k])} * acc[{i}]' if k in em.active else '0.0'
             S(f'    rates[id + offsetT + {k} * offset] = {val};')
         S('  }')
-        for i, k in enumerate(own[v]):
-            if k in em.active:
-                S(f'  {{ const double* a = piece + {14 * k + 8} + (T > {lit(float(t["T_mid"][k]))} ? 0 : {14 * N});')
-                S(f'    sh += acc[{i}] * (a[0] + a[1] * T + a[2] * T2 + a[3] * T3 + a[4] * T4 + a[5] * rcpT); }}')
         S('}')
-    S(f'part[v * {ROW} + lane] = sh;')
-    S('__syncthreads();')
     S('if (v == 0 && live) {')
     S('  double sum_h = 0.0;')
     S('  #pragma unroll')

@@ -1162,12 +1162,20 @@ def generate(tables, info, opts=None):
                            n_active=info['n_active_species'], n_reactions=info['n_reactions'])]
     from . import emit_rolled
     if o.get('rolled') or int(tables['n_species']) > emit_rolled.ROLL_N:
-        # large mechanism: loop forms (private per-lane species arrays, uniform table loads);
+        # large mechanism: no code that unrolls the pairs or keeps a state's species in registers,
         # no MFMA-accumulation variant and no surrogate (its width is fixed at 64)
-        # production rates: several lanes per state, species arrays in LDS (emit_coop)
+        # production rates: straight-line reactions split over a workgroup's wavefronts where the
+        # species' rows fit the LDS (129 species / 1,231 reactions, 100,003 states: 238 us against
+        # 1,732 in loop form; 160 / 1,000, 524,288 states: 1,825 against 5,340); beyond that, or
+        # asked for (rolled), several lanes per state over a reaction loop (emit_coop). Code and
+        # compile time grow with the reactions (1,231: 0.5 MB, 29 s; 1,000 with fewer shared terms:
+        # 0.8 MB, 54 s): past 2,000 the loop stays
+        from . import emit_bk1_split as SP
         from . import emit_coop
-        parts.append(emit_coop.emit_bk1(tables, info, 'fp64', o['coop_lps']))
-        parts.append(emit_coop.emit_bk1(tables, info, 'mixed_valu', o['coop_lps']))
+        split = None if o.get('rolled') or int(tables['n_reactions']) > 2000 else SP.pays(tables, info)
+        for variant in ('fp64', 'mixed_valu'):
+            parts.append(SP.emit(tables, info, variant, split) if split else
+                         emit_coop.emit_bk1(tables, info, variant, o['coop_lps']))
         if 'cond' in tables:
             # transport: four lanes per state with the pair rows streamed through LDS up to 160
             # species (160 species, 2,097,152 states: 12.1 ms against 36.7 in 64-state tiles);
@@ -1188,7 +1196,7 @@ def generate(tables, info, opts=None):
     from . import emit_bk1_split as SP
     order, split = None, o['bk1_live'] and SP.pays(tables, info)
     if split:
-        parts.append(SP.emit(tables, info, 'fp64'))
+        parts.append(SP.emit(tables, info, 'fp64', split))
     elif o['bk1_live']:
         from . import liveness
         order = liveness.order_reactions(tables)
@@ -1221,7 +1229,7 @@ def generate(tables, info, opts=None):
     parts.append(_with_pool('kx_bk1_mixed_k', emit_mixed.emit, tables, info, o['mixed'],
                             lds=o['mixed_lds_pool']))
     if split:
-        parts.append(SP.emit(tables, info, 'mixed_valu'))
+        parts.append(SP.emit(tables, info, 'mixed_valu', split))
     elif o['bk1_live']:
         parts.append(_with_pool('kx_bk1_mixed_valu_k', _emit_bk1_live, tables, info, 'mixed_valu',
                                 o['mixed_arrh32'], order, o['mixed_waves'], lds=o['lds_pool']))

@@ -49,6 +49,25 @@ def test_plan_covers_every_reaction_and_sum(mech):
     assert not SP.pays(*reversed(load('LiDryer')))
 
 
+@pytest.mark.parametrize('mech,waves,occupancy', [('gri30', 8, 4), ('EtOHKonnov', 12, 3), ('synth160', 8, 2)])
+def test_shapes(mech, waves, occupancy):
+    """The layout by size: rows within the LDS, a species' sums of all wavefronts in one round,
+    and every third body's concentration from its own row or from w and rg rows."""
+    info, t = load(mech)
+    p, occ, segment = SP.pays(t, info)
+    em = p['em']
+    assert (p['waves'], occ) == (waves, occupancy) and segment in (3, SP.SEGMENT)
+    assert p['tight'] == (occupancy < 4)
+    assert SP.lds_bytes(em.N, p['rows'], waves, p['tight']) <= SP.LDS_MAX // (2 if occupancy == 4 else 1)
+    for k in range(em.N):
+        assert len({i for i, rnd in enumerate(p['rounds']) for w, j in rnd if j == k}) <= 1
+    for r in range(em.R):
+        if em.kind[r] not in (SP.M.ELEMENTARY, SP.M.PLOG):
+            third = np.flatnonzero(em.t['eff'][r] != 1.0) if em.has_eff[r] else \
+                [k for k in (int(em.t['collider'][r]),) if k >= 0]
+            assert all(k in p['crow'] or k in p['rrow'] for k in third)
+
+
 def _poly(body):
     """Coefficients of a Horner chain, lowest first, from the C source."""
     c = re.findall(r'(?:double p =|fma\(p, \w,) ([-0-9.e]+)\)?;', body)
@@ -88,7 +107,8 @@ def test_exponential_polynomials():
 @pytest.mark.parametrize('mech,n,p_atm', [('gri30', 1, 1.0), ('gri30', 63, 1.0), ('gri30', 1000, 20.0),
                                           ('NH3Konnov_edit', 65, 0.05), ('NH3Konnov_edit', 257, 3.0),
                                           ('chempolimi_edit', 64, 2000.0), ('synth40cov', 129, 1.0),
-                                          ('LiDryer', 300, 5.0)])
+                                          ('LiDryer', 300, 5.0), ('EtOHKonnov', 1, 1.0),
+                                          ('EtOHKonnov', 129, 20.0), ('synth160', 191, 0.3)])
 def test_split_rates_at_group_edges(mech, n, p_atm):
     """FP64 and mixed rates at state counts around the 64-state groups on a strided view, cold
     and hot (300-3000 K, both NASA-7 pieces), against the oracle; nothing outside the view."""
