@@ -21,7 +21,7 @@ under 128 registers, and four waves per SIMD hide each other's latencies; a smal
 falls with the length of one wavefront's program.
 
 Measured (before: one wavefront per 64 states, product form): GRI-3.0, 1,048,576 states FP64 762
--> 617 us, mixed 517 -> 440, 1,000 states FP64 41 -> 13.0 us; NH3Konnov_edit 2,510 -> 518 and
+-> 610 us, mixed 517 -> 425, 1,000 states FP64 41 -> 13.0 us; NH3Konnov_edit 2,510 -> 518 and
 2,236 -> 378 us. Bound: FP64 issue and its power (75 % of the issue slots at 2.06 GHz). 4
 wavefronts of 256 registers: 625 / 478 us, 15.4 us; 16: 949 / 774; two groups of 64 states per
 workgroup in step: 715 / 566; a loop over groups instead of one per workgroup: 826 / 618 (the
@@ -55,6 +55,7 @@ from . import mechanism as M
 WAVES = 8                # wavefronts that share 64 states' reactions
 SEGMENT = 6              # reactions between points where values read from LDS are dropped
 ROW = 64                 # states per workgroup
+HOT_ROWS = 2             # rows a wavefront keeps in registers
 LDS_MAX = 160 * 1024
 MAX_SUMS = 100           # sums of a wavefront that stay in registers (two each, of 256)
 
@@ -149,17 +150,54 @@ def assign(em, waves=WAVES, seed=7):
     return where
 
 
-def order(em, rs):
-    """Order of one wavefront's reactions: next the one sharing most species with the last few."""
+def rows_of(em, r):
+    """The LDS rows a reaction reads: w of its reactants and (reversible) products, rg of its
+    reactants."""
+    ks = np.flatnonzero((em.nu_f[r] > 0) | (em.rev[r] & (em.nu_r[r] > 0)))
+    return {('w', int(k)) for k in ks} | {('rg', int(k)) for k in np.flatnonzero(em.nu_f[r])}
+
+
+def order(em, rs, segment=SEGMENT, hot_rows=HOT_ROWS, seed=7):
+    """Order of one wavefront's reactions and its hot rows, the rows that most segments read,
+    which stay in registers: greedy (next the reaction sharing most species with the last few),
+    then a seeded search over swaps between segments for the fewest rows read. hot_rows None:
+    greedy only (registers are short: 160 species 1,835 us, with the search 1,893, as the longer
+    reuse spills more sums). 53 species: 975 rows read per group greedy, 859 searched, 779 with two
+    hot; 4,194,304 states mixed, which is near the LDS rate, 1,754 us -> 1,711 -> 1,690, FP64 2,454 ->
+    2,399 -> 2,393 (four hot, which spill, 1,801 and 2,415; segments of 8 or 10 no faster)."""
     used = {r: set(np.flatnonzero((em.nu_f[r] > 0) | (em.rev[r] & (em.nu_r[r] > 0))).tolist()) for r in rs}
     left, out, recent = sorted(rs), [], []
     while left:
-        near = set().union(*recent[-SEGMENT:]) if recent else set()
+        near = set().union(*recent[-segment:]) if recent else set()
         r = max(left, key=lambda r: (len(used[r] & near), -r))
         left.remove(r)
         out.append(r)
         recent.append(used[r])
-    return out
+    if hot_rows is None:
+        return out, frozenset()
+    rows = {r: rows_of(em, r) for r in rs}
+    segs = [out[i:i + segment] for i in range(0, len(out), segment)]
+    read = lambda s, hot: len(set().union(*[rows[r] for r in s]) - hot)
+
+    def search(hot, iters=6000):
+        rng = random.Random(seed)
+        c = [read(s, hot) for s in segs]
+        for _ in range(iters if len(segs) > 1 else 0):
+            a, b = rng.sample(range(len(segs)), 2)
+            i, j = rng.randrange(len(segs[a])), rng.randrange(len(segs[b]))
+            A, B = list(segs[a]), list(segs[b])
+            A[i], B[j] = B[j], A[i]
+            ca, cb = read(A, hot), read(B, hot)
+            if ca + cb <= c[a] + c[b]:
+                segs[a], segs[b], c[a], c[b] = A, B, ca, cb
+    search(frozenset())
+    n = {}
+    for s in segs:
+        for x in set().union(*[rows[r] for r in s]):
+            n[x] = n.get(x, 0) + 1
+    hot = frozenset(sorted(n, key=lambda x: (-n[x], x))[:hot_rows])
+    search(hot)
+    return [r for s in segs for r in s], hot
 
 
 def plan(t, info, waves=WAVES):
@@ -168,8 +206,8 @@ def plan(t, info, waves=WAVES):
     em = E._RateEmitter(t, info)
     N = em.N
     where = assign(em, waves)
-    rs = [order(em, [r for r in range(em.R) if where[r] == w]) for w in range(waves)]
-    sums = [sorted({int(k) for r in rs[w] for k in np.flatnonzero(em.net[r])}) for w in range(waves)]
+    parts = [[r for r in range(em.R) if where[r] == w] for w in range(waves)]
+    sums = [sorted({int(k) for r in parts[w] for k in np.flatnonzero(em.net[r])}) for w in range(waves)]
     react = sorted({int(k) for r in range(em.R) for k in np.flatnonzero(em.nu_f[r])})
     third = sorted({int(k) for r in range(em.R) if em.kind[r] not in (M.ELEMENTARY, M.PLOG)
                     for k in ([int(j) for j in np.flatnonzero(em.t['eff'][r] != 1.0)] if em.has_eff[r]
@@ -196,7 +234,7 @@ def plan(t, info, waves=WAVES):
             cur[(w, k)] = rows - free
             free -= 1
     rounds.append(cur)
-    return dict(em=em, rs=rs, sums=sums, wrow=wrow, rrow=rrow, crow=crow, rows=rows, rounds=rounds,
+    return dict(em=em, rs=parts, sums=sums, wrow=wrow, rrow=rrow, crow=crow, rows=rows, rounds=rounds,
                 waves=waves, where=where, tight=tight)
 
 
@@ -241,8 +279,10 @@ def pays(t, info):
 
 def emit(t, info, variant='fp64', shaped=None):
     p, occupancy, segment = shaped or shape(t, info)
+    hot_rows = HOT_ROWS if segment == SEGMENT else None
     waves = p['waves']
     em = E._RateEmitter(t, info)
+    runs = [order(em, rs, segment, hot_rows) for rs in p['rs']]
     N = em.N
     mixed = variant == 'mixed_valu'
     em.arrh32 = mixed
@@ -261,6 +301,8 @@ def emit(t, info, variant='fp64', shaped=None):
     tab('poly', PT.reshape(-1))
     tab('rcpW', list(t['rcpW']) + [0.0] * (waves * per - N))
     tab('tmid', t['T_mid'])
+    S(RL._table(f'{name}_rrow', [p['rrow'].get(k, -1) for k in range(N)], 'int'), 0)
+    S(RL._table(f'{name}_crow', [p['crow'].get(k, -1) for k in range(N)], 'int'), 0)
     plog = None
     if np.any(em.kind == M.PLOG):
         d = RL.bk1_data(t)
@@ -282,7 +324,7 @@ def emit(t, info, variant='fp64', shaped=None):
         S(f'__shared__ __attribute__((aligned(16))) double poly_s[{PT.size}];')
     S(f'__shared__ double rows[{p["rows"]} * {ROW}];        // w, rg, third-body C; then the wavefronts\' sums')
     if tight:
-        S('double* const part = rows;               // before w is written and after the sums are read')
+        S(f'double* const part = rows + {N * ROW};   // before rg is written and after the sums are read')
     else:
         S(f'__shared__ double part[{waves + 1} * {ROW}];')
     if staged:
@@ -306,6 +348,7 @@ def emit(t, info, variant='fp64', shaped=None):
     S(f'for (int i = 0; i < {per}; ++i) {{')
     S(f'  c[i] = fmax(0.0, c[i]) * {name}_rcpW[v + {waves} * i];          // 0 past the last species')
     S('  sum += c[i];')
+    S(f'  if (v + {waves} * i < {N}) rows[(v + {waves} * i) * {ROW} + lane] = c[i];   // for the loop over species')
     S('}')
     S(f'part[v * {ROW} + lane] = sum;')
     S(f'if (v == {waves - 1}) part[{waves} * {ROW} + lane] = log(T);   // once per state')
@@ -329,35 +372,22 @@ def emit(t, info, variant='fp64', shaped=None):
     S(f'const double C0 = {lit(float(t["one_atm_R"]))} * rcpT;')
     S(f'const double rcpC0 = {lit(float(t["R_one_atm"]))} * T;')
     S('// ---- species: w_k = C_k exp(g_k), rg_k = exp(-g_k), third-body concentrations')
-    rr = [p['rrow'].get(k, -1) for k in range(N)]
-    cr = [p['crow'].get(k, -1) for k in range(N)]
+    S('// (a loop: the exponential\'s constants stay in registers; unrolled they were moved there for')
+    S('// each species, a third of the phase\'s vector instructions)')
     S(f'const double* const piece = {"poly_s" if staged else name + "_poly"};')
-    for i in range(per):
-        S('{')
-        S(f'  const int k = v + {waves} * {i};')
-        ks = [k for k in range(N) if k // waves == i]
-        if len(ks) < waves:
-            S(f'  if (k < {N}) {{')
-        else:
-            S('  {')
-        S(f'  const double ck = c[{i}] * rho;')
-        S(f'  const double* a = piece + 14 * k + (T > {name}_tmid[k] ? 0 : {14 * N});')
-        S('  const double gk = a[0] * omlnT + a[1] * T + a[2] * T2 + a[3] * T3 + a[4] * T4 + a[5] * rcpT - a[6];')
-        S('  const double ek = kx_exp(gk);')
-        S(f'  rows[k * {ROW} + lane] = ck * ek;')
-        # rg and third-body rows: uniform selects over the wavefront's species of this round
-        def pick(rowmap, val):
-            have = [k for k in ks if rowmap[k] >= 0]
-            if not have:
-                return
-            expr = '-1'
-            for k in have:
-                expr = f'v == {k % waves} ? {rowmap[k]} : ({expr})'
-            S(f'  {{ const int row = {expr}; if (row >= 0) rows[row * {ROW} + lane] = {val}; }}')
-        pick(rr, 'kx_rcp(ek)')
-        pick(cr, 'ck')
-        S('  }')
-        S('}')
+    S('#pragma unroll 1')
+    S(f'for (int k = v; k < {N}; k += {waves}) {{')
+    S(f'  const int rr = {name}_rrow[k], cr = {name}_crow[k];')
+    S(f'  const double ck = rows[k * {ROW} + lane] * rho;')
+    S(f'  const double* a = piece + 14 * k + (T > {name}_tmid[k] ? 0 : {14 * N});')
+    S('  const double gk = a[0] * omlnT + a[1] * T + a[2] * T2 + a[3] * T3 + a[4] * T4 + a[5] * rcpT - a[6];')
+    S('  const double ek = kx_exp(gk);')
+    S(f'  rows[k * {ROW} + lane] = ck * ek;')
+    S(f'  if (rr >= 0) rows[rr * {ROW} + lane] = kx_rcp(ek);')
+    if p['crow']:
+        S(f'  if (cr >= 0) rows[cr * {ROW} + lane] = ck;')
+    S('  (void)cr;')
+    S('}')
     S('__syncthreads();')
     S('// ---- reactions of each wavefront')
     mx = max(len(s) for s in p['sums'])
@@ -372,7 +402,11 @@ def emit(t, info, variant='fp64', shaped=None):
         S(f'{"if" if w == 0 else "else if"} (v == {w}) {{' if w < waves - 1 else 'else {')
         slot = {k: i for i, k in enumerate(p['sums'][w])}
         have_third, pins = set(), []
-        for n, r in enumerate(p['rs'][w]):
+        run, hot = runs[w]
+        for x, k in sorted(hot):
+            S(f'const double hot_{x}{k} = {at(p["wrow" if x == "w" else "rrow"][k])};')
+        row = lambda x, k: f'hot_{x}{k}' if (x, k) in hot else at(p['wrow' if x == 'w' else 'rrow'][k])
+        for n, r in enumerate(run):
             if n % segment == 0:
                 # the segment's sums are needed as values here: the compiler otherwise defers
                 # them to the end of the wavefront's program, all values read from LDS alive
@@ -397,9 +431,9 @@ def emit(t, info, variant='fp64', shaped=None):
             S(f'double q{r};')
             S('{')
             for k in ks:
-                S(f'const double W{k} = rows[{p["wrow"][k] * ROW} + o];')
+                S(f'const double W{k} = {row("w", k)};')
             for k in np.flatnonzero(em.nu_f[r]):
-                S(f'const double rg{k} = rows[{p["rrow"][int(k)] * ROW} + o];')
+                S(f'const double rg{k} = {row("rg", int(k))};')
             T_ = E._Src()
             em.emit_reaction_p(T_, r, sidx, wvar='W', declare=False, plog=plog)
             for line in T_.lines:

@@ -68,6 +68,26 @@ def test_shapes(mech, waves, occupancy):
             assert all(k in p['crow'] or k in p['rrow'] for k in third)
 
 
+@pytest.mark.parametrize('mech', ['gri30', 'NH3Konnov_edit', 'EtOHKonnov'])
+def test_order_reads_fewer_rows(mech):
+    """A wavefront's searched order keeps its reactions, is the same each time, and reads no more
+    LDS rows (distinct rows of every segment, hot rows once) than the greedy order."""
+    info, t = load(mech)
+    p, _, segment = SP.pays(t, info)
+    em = p['em']
+
+    def reads(o, hot):
+        rows = [set().union(*[SP.rows_of(em, r) for r in o[i:i + segment]]) for i in range(0, len(o), segment)]
+        return len(hot) + sum(len(x - hot) for x in rows)
+    for rs in p['rs']:
+        plain, none = SP.order(em, rs, segment, None)
+        o, hot = SP.order(em, rs, segment)
+        assert sorted(plain) == sorted(o) == sorted(rs) and not none
+        assert len(hot) <= SP.HOT_ROWS and hot <= set().union(*[SP.rows_of(em, r) for r in rs])
+        assert (o, hot) == SP.order(em, rs, segment)
+        assert reads(o, hot) <= reads(plain, none)
+
+
 def _poly(body):
     """Coefficients of a Horner chain, lowest first, from the C source."""
     c = re.findall(r'(?:double p =|fma\(p, \w,) ([-0-9.e]+)\)?;', body)
