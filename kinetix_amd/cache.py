@@ -54,8 +54,8 @@ def generator_digest():
     """SHA-256 over the generator's sources (the code that decides what is generated and how
     it compiles): any change to them invalidates every cache entry."""
     files = sorted(glob.glob(os.path.join(PKG, 'gen', '*.py')))
-    files += [os.path.join(PKG, 'build.py'), os.path.join(PKG, 'csrc', 'kx_mlp_wave.h'),
-              os.path.join(PKG, 'csrc', 'kx_rcp.h')]
+    files += [os.path.join(PKG, 'build.py')]
+    files += [os.path.join(PKG, 'csrc', f) for f in ('kx_mlp_wave.h', 'kx_rcp.h', 'kx_exp.h', 'kx_bk2_quad.h')]
     h = hashlib.sha256()
     for f in files:
         h.update(os.path.basename(f).encode() + b'\0')
