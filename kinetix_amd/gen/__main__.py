@@ -22,7 +22,7 @@ def main(argv=None):
     ap.add_argument('--no-transport', action='store_true', help='skip transport fits/kernels')
     ap.add_argument('--tables-only', action='store_true', help='write tables, no kernels')
     ap.add_argument('--rolled', action='store_true',
-                    help='loop forms of the FP64/mixed kernels (default above 96 species)')
+                    help='loop forms of the FP64/mixed kernels (default where no other form fits)')
     ap.add_argument('--bk2-loop', action='store_true',
                     help='with the loop forms: transport one state per lane instead of state tiles')
     args = ap.parse_args(argv)

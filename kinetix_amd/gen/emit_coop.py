@@ -1,4 +1,6 @@
-"""Cooperative (several lanes per state) production-rate kernels for large mechanisms.
+"""Cooperative (several lanes per state) production-rate kernels in loop form: mechanisms whose
+reactions are not split as straight-line code (emit_bk1_split: rows beyond the LDS or more than
+2,000 reactions), and those asked for with --rolled.
 
 The one-state-per-lane loop forms (emit_rolled) keep each state's species arrays -- w, the
 Gibbs terms, omega-dot: ~4 KB at 160 species -- in per-lane scratch. With 64 lanes and many

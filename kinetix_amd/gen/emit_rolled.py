@@ -25,7 +25,7 @@ import numpy as np
 from . import emit_hip as E
 from . import mechanism as M
 
-ROLL_N = 96          # mechanisms with more species than this get the loop forms
+ROLL_N = 96          # mechanisms with more species than this: no unrolled pairs (emit_hip.generate)
 BK2_BLOCK = 8        # j-species held in registers by the blocked BK2 pair loops (8: 2 waves/SIMD)
 BK2_KUNROLL = 2      # k-loop unroll (overlaps the next pair coefficients' loads)
 
