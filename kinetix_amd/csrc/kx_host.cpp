@@ -151,6 +151,17 @@ int launch(Mech* m, const char* name, long long n_lanes, void* stream, void** ar
   return KX_OK;
 }
 
+// States that one launch of a kernel takes: HIP refuses a grid of 2^32 threads or more, which a
+// kernel with several lanes per state reaches below INT_MAX states. Whole workgroups.
+long long states_per_launch(Mech* m, const char* name)
+{
+  auto b = m->block.find(name);
+  auto l = m->lanes.find(name);
+  if (b == m->block.end()) return 0x7fffffffLL;
+  const long long lanes = l == m->lanes.end() ? 1 : l->second;
+  return 0xffffffffLL / b->second * (b->second / lanes);
+}
+
 // An explicit grid of workgroups of the kernel's launch bound.
 int launch_grid(Mech* m, const char* name, long long grid, void* stream, void** args)
 {
@@ -369,7 +380,18 @@ static int production_rates_impl(const char* kernel, kx_mech_t h, int n, int off
   const double* s = d_state;
   double* r = d_rates;
   void* args[] = {&n, &oT, &o, &pressure_R, &pressure_, &s, &r, &Tref};
-  return launch(m, kernel, n, stream, args);
+  // more states than a launch takes (8 lanes per state: 536,870,848) go in pieces: a state's
+  // rows lie at fixed distances from its first value, so a piece is the same call further on
+  const long long most = states_per_launch(m, kernel);
+  long long left = n;
+  do {
+    n = (int)std::min(left, most);
+    rc = launch(m, kernel, n, stream, args);
+    s += n;
+    r += n;
+    left -= n;
+  } while (rc == KX_OK && left > 0);
+  return rc;
 }
 
 int kx_production_rates(kx_mech_t h, int n, int offsetT, int offset, double pressure,
