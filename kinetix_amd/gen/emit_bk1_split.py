@@ -222,7 +222,9 @@ def plan(t, info, waves=WAVES):
     crow = {k: N + len(react) + i for i, k in enumerate(third)}
     rows = max(N + len(react) + len(third), waves + 1)
     if tight:
-        rows = max(rows, LDS_MAX // (8 * ROW))      # one workgroup per CU: fewer rounds for the sums
+        # emit's `part` (waves + 1 rows) starts where the rg rows do; one workgroup per CU: all
+        # of the LDS, for fewer rounds of the sums
+        rows = max(rows, N + waves + 1, LDS_MAX // (8 * ROW))
     # a round takes all wavefronts' sums of some species: every wavefront writes in every round
     rounds, cur, free = [], {}, rows
     for k in range(N):

@@ -68,6 +68,31 @@ def test_shapes(mech, waves, occupancy):
             assert all(k in p['crow'] or k in p['rrow'] for k in third)
 
 
+def padded(t, N):
+    """A mechanism's tables with inert species appended up to N."""
+    n, R = int(t['n_species']), int(t['n_reactions'])
+    out = dict(t, n_species=N)
+    for k in ('nu_f', 'nu_r', 'eff'):
+        a = np.asarray(t[k]).reshape(R, n)
+        out[k] = np.concatenate([a, np.full((R, N - n), 1 if k == 'eff' else 0, a.dtype)], axis=1)
+    for k in ('W', 'rcpW', 'T_mid', 'g_lo', 'g_hi', 'h_lo', 'h_hi'):
+        a = np.asarray(t[k])
+        out[k] = np.concatenate([a, np.repeat(a[-1:], N - n, axis=0)])
+    return out
+
+
+@pytest.mark.parametrize('waves', [8, 12])
+@pytest.mark.parametrize('N', [290, 308, 315, 319])
+def test_tight_rows_hold_the_partial_sums(N, waves):
+    """Many species, few of them reactants: the tight layout's wavefront sums and ln T (waves + 1
+    rows from row N on) lie within the rows, or the plan does not fit the LDS."""
+    info, t = load('LiDryer')
+    p = SP.plan(padded(t, N), info, waves)
+    assert p['tight'] and p['rows'] >= N + waves + 1
+    if N + waves + 1 > SP.LDS_MAX // (8 * SP.ROW):
+        assert SP.lds_bytes(N, p['rows'], waves, True) > SP.LDS_MAX
+
+
 @pytest.mark.parametrize('mech', ['gri30', 'NH3Konnov_edit', 'EtOHKonnov'])
 def test_order_reads_fewer_rows(mech):
     """A wavefront's searched order keeps its reactions, is the same each time, and reads no more
