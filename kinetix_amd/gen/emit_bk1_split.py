@@ -307,7 +307,7 @@ def emit(t, info, variant='fp64', shaped=None):
     S(RL._table(f'{name}_crow', [p['crow'].get(k, -1) for k in range(N)], 'int'), 0)
     plog = None
     if np.any(em.kind == M.PLOG):
-        d = RL.bk1_data(t)
+        d = RL.plog_data(t)
         for nm, ct in (('plo', 'int'), ('plP', 'double'), ('pllnP', 'double'), ('plrcp', 'double'),
                        ('plko', 'int'), ('plnk', 'int'), ('plk', 'double')):
             S(RL._table(f'{name}_{nm}', d[nm], ct), 0)

@@ -239,12 +239,20 @@ def bk1_data(t):
         dbl[r] = row
     # FP32 copies of the Arrhenius and low-pressure exponent coefficients (mixed variant)
     flt = dbl[:, :6].astype(np.float32)
-    # PLOG points: per reaction a range of points (ascending P), per point a range of
-    # Arrhenius rates (log2 A, beta, Ta log2 e) summed at that pressure
+    return dict(plog_data(t), flt=flt,
+                fsp=f_sp, rsp=r_sp, nsp=n_sp, nnu=n_nu, meta=meta, dbl=dbl,
+                setoff=np.array(set_off), setsp=np.array(set_sp), sete=np.array(set_e),
+                nsets=len(sets), MX=MX, MS=MS)
+
+
+def plog_data(t):
+    """PLOG points: per reaction a range of points (ascending P), per point a range of Arrhenius
+    rates (log2 A, beta, Ta log2 e) summed at that pressure."""
+    L2E = 1.4426950408889634
     em = E._RateEmitter(t, None)
     plo, plP, pllnP, plrcp, plko, plnk, plk = [0], [], [], [], [], [], []
-    for r in range(R):
-        if kind[r] == M.PLOG:
+    for r in range(em.R):
+        if em.kind[r] == M.PLOG:
             pts = em.plog_points(r)
             for i, (P, rates) in enumerate(pts):
                 plP.append(P)
@@ -255,11 +263,8 @@ def bk1_data(t):
                 for A, b, Ta in rates:
                     plk += [math.log2(A), b, Ta * L2E]
         plo.append(len(plP))
-    return dict(flt=flt, plo=np.array(plo), plP=np.array(plP), pllnP=np.array(pllnP),
-                plrcp=np.array(plrcp), plko=np.array(plko), plnk=np.array(plnk), plk=np.array(plk),
-                fsp=f_sp, rsp=r_sp, nsp=n_sp, nnu=n_nu, meta=meta, dbl=dbl,
-                setoff=np.array(set_off), setsp=np.array(set_sp), sete=np.array(set_e),
-                nsets=len(sets), MX=MX, MS=MS)
+    return dict(plo=np.array(plo), plP=np.array(plP), pllnP=np.array(pllnP),
+                plrcp=np.array(plrcp), plko=np.array(plko), plnk=np.array(plnk), plk=np.array(plk))
 
 
 def _bk1_tables(t, pre):

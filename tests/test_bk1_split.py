@@ -93,6 +93,24 @@ def test_tight_rows_hold_the_partial_sums(N, waves):
         assert SP.lds_bytes(N, p['rows'], waves, True) > SP.LDS_MAX
 
 
+@pytest.mark.parametrize('reactants,products', [({0: 5}, {1: 3}), ({0: 1}, {k: 1 for k in range(1, 11)})])
+def test_global_reactions_beside_plog(reactants, products):
+    """A mechanism with PLOG reactions takes a reaction of more molecules or species than the loop
+    forms' descriptors hold (4 molecules a side, 8 species): straight-line code has no limit."""
+    info, t = load('NH3Konnov_edit')
+    assert np.any(t['kind'] == SP.M.PLOG)
+    t = {k: np.array(v) if isinstance(v, np.ndarray) else v for k, v in t.items()}
+    r = int(np.flatnonzero(t['kind'] == SP.M.ELEMENTARY)[5])
+    t['reversible'][r] = 0
+    for key, nu in (('nu_f', reactants), ('nu_r', products)):
+        t[key][r] = 0
+        for k, v in nu.items():
+            t[key][r, k] = v
+    src = SP.emit(t, info, 'fp64', SP.pays(t, info))
+    line = next(ln for ln in src.split(f'{{ // {r + 1}: ')[1].split('\n') if 'double F' in ln)
+    assert line.count('rg0') == reactants[0]
+
+
 @pytest.mark.parametrize('mech', ['gri30', 'NH3Konnov_edit', 'EtOHKonnov'])
 def test_order_reads_fewer_rows(mech):
     """A wavefront's searched order keeps its reactions, is the same each time, and reads no more
