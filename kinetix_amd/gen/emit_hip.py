@@ -542,6 +542,8 @@ class _RateEmitter:
         small integer n, else A times one exp2 (FP32 exponent in the mixed variant)."""
         t = self.t
         A, beta, Ta = float(t['A'][r]), float(t['beta'][r]), float(t['Ta'][r])
+        if A <= 0.0:
+            raise ValueError(f'reaction {r + 1}: rate coefficients with A <= 0')
         if self.arrh_key(beta, Ta) is None:
             return self.arrh_expr(A, beta, Ta, None)
         if getattr(self, 'arrh32', False):

@@ -111,6 +111,21 @@ def test_global_reactions_beside_plog(reactants, products):
     assert line.count('rg0') == reactants[0]
 
 
+@pytest.mark.parametrize('A', [0.0, -1e3])
+def test_rate_coefficients_without_a_logarithm_are_refused(A):
+    """A <= 0 is no Arrhenius coefficient, with or without an exponential beside it."""
+    info, t = load('gri30')
+    for beta, Ta in ((0.0, 0.0), (1.0, 0.0), (0.5, 100.0)):
+        c = dict(t, A=t['A'].copy(), beta=t['beta'].copy(), Ta=t['Ta'].copy())
+        r = int(np.flatnonzero(t['kind'] == SP.M.ELEMENTARY)[0])
+        c['A'][r], c['beta'][r], c['Ta'][r] = A, beta, Ta
+        for variant in ('fp64', 'mixed_valu'):
+            em = SP.E._RateEmitter(c, info)
+            em.arrh32 = variant == 'mixed_valu'
+            with pytest.raises(ValueError):
+                em.rate_const_p(r)
+
+
 @pytest.mark.parametrize('mech', ['gri30', 'NH3Konnov_edit', 'EtOHKonnov'])
 def test_order_reads_fewer_rows(mech):
     """A wavefront's searched order keeps its reactions, is the same each time, and reads no more
