@@ -1,6 +1,7 @@
 // FP64 exp2, exp and log2 for the production-rate kernels, without the library functions' range
 // handling (a third of their instructions): results beyond the double range come out of ldexp as
-// infinity or zero, a NaN stays NaN; infinite arguments are the caller's to avoid.
+// infinity or zero, a NaN stays NaN; infinite arguments, and of exp2 and exp those whose binary
+// exponent is no int (|x| above 2^31, 1.4e9), are the caller's to avoid.
 //
 // Method: reduction to |r| <= 1/2 (exp2) or |r| <= ln 2 / 2 (exp; ln 2 in two parts, the first of
 // 24 bits, so that n ln2_hi is exact), a degree-11 polynomial, and the power of two by ldexp. log2:

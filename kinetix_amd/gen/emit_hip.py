@@ -586,9 +586,12 @@ class _RateEmitter:
                 if kind == M.TROE:
                     A_, rT3, rT1, T2 = t['troe'][r]
                     L2E = 1.4426950408889634
-                    term3 = f' + kx_exp2({lit(-T2 * L2E)} * rcpT)' if T2 >= 0 else ''
-                    S(f'  const double l2F = kx_log2({lit(1.0 - A_)} * kx_exp2({lit(-rT3 * L2E)} * T) + '
-                      f'{lit(A_)} * kx_exp2({lit(-rT1 * L2E)} * T){term3});')
+                    # the parameters that switch a term off (T3 of 1e-30, T2 of 1e30) as a factor for
+                    # which kx_exp2's exponent is an int and 2^y still 0: between 1 and 20,000 K
+                    cT = lambda rT: lit(max(-1e5, min(1e5, -rT * L2E)))
+                    term3 = f' + kx_exp2({lit(max(-1e9, -T2 * L2E))} * rcpT)' if T2 >= 0 else ''
+                    S(f'  const double l2F = kx_log2({lit(1.0 - A_)} * kx_exp2({cT(rT3)} * T) + '
+                      f'{lit(A_)} * kx_exp2({cT(rT1)} * T){term3});')
                     S(f'  const double lF = {lit(math.log10(2.0))} * l2F;')
                     S('  const double tc = -0.4 - 0.67 * lF + lP, td = 0.75 - 1.27 * lF - 0.14 * tc;')
                     S('  F *= kx_exp2(l2F * (td * td) * kx_rcp(td * td + tc * tc));   // l2F / (1 + (tc / td)^2)')

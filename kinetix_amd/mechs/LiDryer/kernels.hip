@@ -6,7 +6,7 @@
 #include "kx_exp.h"      // kx_exp2, kx_exp, kx_log2
 
 
-__device__ double kx_bk1_fp64_k[77] = {1.4426950408889634, 496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, 1.5, 11.0, -0.21999999999999997, 10.0, 1000.0, 12186.596374704217, 8.205736608095969e-05, 45770000000000.0, -1.4, -75779.07893121493, 216.0, 1.51, -2490.1536763179456, 0.0508, 2.67, -4566.491727125329, 2.9699999999999998, 2.02, -9728.297161125503, 4714000.0, 38000000000.0, 6165.0, 3547000000.0, -0.406, -12050.746610262851, 1475000.0, 0.6, 8.75352839227408, -2.32, -381.0007723999002, 0.3010299956639812, 0.19999999999999996, -1.4426950408889633e+30, 0.8, -1.4426950408889633e-30, 32500000.0, 9.549999999999999, -2882.189532064794, 0.015999, 16600000.0, -597.4916838512155, 48200000.0, -5771.63898738416, 0.002016, 24100000.0, 70790000.0, -214.16773600985246, 0.001008, 580000000.0, -6938.308654393763, 1000000.0, 28900000.0, 360.8181857521921, 0.018015, 295100000000000.0, -35159.80832188866, -11.26155130938291, 2127.1575135893813, 0.017006999999999998, 130000.0, 1182.859295867297, 420000000.0, -8698.840043627297, 0.031998, 0.033006, 0.034013999999999996, -8.31446261815324};
+__device__ double kx_bk1_fp64_k[77] = {1.4426950408889634, 496.031746031746, 31.251953247077942, 55.50929780738274, 992.063492063492, 62.503906494155885, 58.79931792791204, 30.297521662727988, 29.39965896395602, 35.69643749553794, 1.5, 11.0, -0.21999999999999997, 10.0, 1000.0, 12186.596374704217, 8.205736608095969e-05, 45770000000000.0, -1.4, -75779.07893121493, 216.0, 1.51, -2490.1536763179456, 0.0508, 2.67, -4566.491727125329, 2.9699999999999998, 2.02, -9728.297161125503, 4714000.0, 38000000000.0, 6165.0, 3547000000.0, -0.406, -12050.746610262851, 1475000.0, 0.6, 8.75352839227408, -2.32, -381.0007723999002, 0.3010299956639812, 0.19999999999999996, -100000.0, 0.8, -1.4426950408889633e-30, 32500000.0, 9.549999999999999, -2882.189532064794, 0.015999, 16600000.0, -597.4916838512155, 48200000.0, -5771.63898738416, 0.002016, 24100000.0, 70790000.0, -214.16773600985246, 0.001008, 580000000.0, -6938.308654393763, 1000000.0, 28900000.0, 360.8181857521921, 0.018015, 295100000000000.0, -35159.80832188866, -11.26155130938291, 2127.1575135893813, 0.017006999999999998, 130000.0, 1182.859295867297, 420000000.0, -8698.840043627297, 0.031998, 0.033006, 0.034013999999999996, -8.31446261815324};
 __device__ const double kx_bk1_fp64_poly[288] = {2.99142337, -0.0003500322055, 9.389714483333335e-09, 7.692981816666665e-13, -7.913758949999998e-17, -835.033997, -1.35511017, 0.0, 2.99142337, 0.0003500322055, -1.8779428966666666e-08, -2.307894545e-12, 3.16550358e-16, -835.033997, 0.0, 0.0, 3.69757819, -0.0003067598445, 2.0980699833333335e-08, -1.479401233333333e-12, 5.682176549999999e-17, -1233.93018, 3.18916559, 0.0, 3.69757819, 0.0003067598445, -4.1961399666666664e-08, 4.4382037e-12, -2.27287062e-16, -1233.93018, 0.0, 0.0, 2.67214561, -0.001528146445, 1.4550433516666668e-07, -1.0008303249999999e-11, 3.195808934999999e-16, -29899.209, 6.86281681, 0.0, 2.67214561, 0.001528146445, -2.910086703333333e-07, 3.002490975e-11, -1.278323574e-15, -29899.209, 0.0, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, -0.460117638, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, 0.0, 0.0, 2.54205966, 1.377530955e-05, 5.171338916666667e-10, -3.7925561833333325e-13, 2.1840257499999995e-17, 29230.8027, 4.92030811, 0.0, 2.54205966, -1.377530955e-05, -1.0342677833333334e-09, 1.137766855e-12, -8.736102999999999e-17, 29230.8027, 0.0, 0.0, 2.86472886, -0.00052825224, 4.3180459666666676e-08, -2.5434889499999995e-12, 6.659793799999999e-17, 3683.62875, 5.70164073, 0.0, 2.86472886, 0.00052825224, -8.636091933333334e-08, 7.63046685e-12, -2.66391752e-16, 3683.62875, 0.0, 0.0, 4.0172109, -0.001119910065, 1.0560969166666667e-07, -9.520530833333331e-12, 5.395426749999999e-16, 111.856713, 3.78510215, 0.0, 4.0172109, 0.001119910065, -2.1121938333333332e-07, 2.85615925e-11, -2.1581707e-15, 111.856713, 0.0, 0.0, 4.57316685, -0.002168068195, 2.4578147e-07, -1.9574196416666664e-11, 7.158267799999999e-16, -18006.9609, 0.501136959, 0.0, 4.57316685, 0.002168068195, -4.9156294e-07, 5.872258925e-11, -2.86330712e-15, -18006.9609, 0.0, 0.0, 2.92664, -0.0007439885, 9.474601666666666e-08, -8.414199999999998e-12, 3.376675499999999e-16, -922.7977, 5.980528, 0.0, 2.92664, 0.0007439885, -1.8949203333333333e-07, 2.52426e-11, -1.3506701999999999e-15, -922.7977, 0.0, 0.0, 3.29812431, -0.000412472087, 1.3571692150000003e-07, 7.896195274999998e-12, -2.0674361199999996e-14, -1012.52087, -3.29409409, 0.0, 3.29812431, 0.000412472087, -2.71433843e-07, -2.3688585825e-11, 8.26974448e-14, -1012.52087, 0.0, 0.0, 3.2129364, -0.000563743175, 9.593584116666667e-08, -1.0948976916666665e-10, 4.3842769599999987e-14, -1005.24902, 6.03473759, 0.0, 3.2129364, 0.000563743175, -1.9187168233333332e-07, 3.284693075e-10, -1.753710784e-13, -1005.24902, 0.0, 0.0, 3.38684249, -0.00173749123, 1.0591160550000003e-06, -5.807151058333331e-10, 1.2532942349999995e-13, -30208.1133, 2.59023285, 0.0, 3.38684249, 0.00173749123, -2.11823211e-06, 1.7421453175e-09, -5.01317694e-13, -30208.1133, 0.0, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, -0.460117608, 0.0, 2.5, 0.0, 0.0, 0.0, 0.0, 25471.627, 0.0, 0.0, 2.94642878, 0.000819083245, -4.035052833333334e-07, 1.335702658333333e-10, -1.9453481799999996e-14, 29147.6445, 2.96399498, 0.0, 2.94642878, -0.000819083245, 8.070105666666667e-07, -4.007107975e-10, 7.78139272e-14, 29147.6445, 0.0, 0.0, 4.12530561, 0.001612724695, -1.087941151666667e-06, 4.832113691666665e-10, -1.0311868949999997e-13, 3346.30913, -0.69043296, 0.0, 4.12530561, -0.001612724695, 2.1758823033333334e-06, -1.4496341075e-09, 4.1247475799999997e-13, 3346.30913, 0.0, 0.0, 4.30179801, 0.002374560255, -3.5263815166666667e-06, 2.0230324499999997e-09, -4.64612562e-13, 294.80804, 3.71666245, 0.0, 4.30179801, -0.002374560255, 7.0527630333333326e-06, -6.06909735e-09, 1.8584502480000002e-12, 294.80804, 0.0, 0.0, 3.38875365, -0.003284612905, 2.475020966666667e-08, 3.8548379333333327e-10, -1.2357573749999998e-13, -17663.1465, 6.7853632, 0.0, 3.38875365, 0.003284612905, -4.950041933333333e-08, -1.15645138e-09, 4.9430295e-13, -17663.1465, 0.0, 0.0, 3.298677, -0.00070412, 6.60537e-07, -4.7012625e-10, 1.2224275e-13, -1020.9, 3.950372, 0.0, 3.298677, 0.00070412, -1.3210739999999999e-06, 1.41037875e-09, -4.889710000000001e-13, -1020.9, 0.0, 0.0};
 extern "C" __global__ void __launch_bounds__(256)
 kx_bk1_fp64(const int n_states, const long long offsetT, const long long offset,

@@ -126,6 +126,28 @@ def test_rate_coefficients_without_a_logarithm_are_refused(A):
                 em.rate_const_p(r)
 
 
+def test_troe_terms_switched_off_have_int_exponents():
+    """Parameters that switch a Troe term off (T3 = 1e-30, T2 = 1e30 in these mechanisms): the
+    exponents handed to kx_exp2, whose power of two is an int, stay in its range from 1 to
+    20,000 K and far below -1,075, where 2^y is 0."""
+    off = 0
+    for mech in ('LiDryer', 'NH3Konnov_edit', 'chempolimi_edit'):
+        info, t = load(mech)
+        em = SP.E._RateEmitter(t, info)
+        _, sidx = em.efficiency_sets()
+        for r in np.flatnonzero(t['kind'] == SP.M.TROE):
+            S = SP.E._Src()
+            em.emit_reaction_p(S, int(r), sidx)
+            line = next(ln for ln in S.lines if 'l2F = kx_log2' in ln)
+            for c, at in re.findall(r'kx_exp2\(([-0-9.e+]+) \* (T|rcpT)\)', line):
+                y = [float(c) * (T if at == 'T' else 1.0 / T) for T in (1.0, 300.0, 20000.0)]
+                assert max(abs(v) for v in y) < 2 ** 31
+                off += max(y) < -2000
+            rT3, rT1, T2 = t['troe'][r][1:]
+            assert len(re.findall('kx_exp2', line)) == (3 if T2 >= 0 else 2)
+    assert off >= 10
+
+
 @pytest.mark.parametrize('mech', ['gri30', 'NH3Konnov_edit', 'EtOHKonnov'])
 def test_order_reads_fewer_rows(mech):
     """A wavefront's searched order keeps its reactions, is the same each time, and reads no more
