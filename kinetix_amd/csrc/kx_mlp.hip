@@ -172,12 +172,22 @@ struct GradArgs {
   float* db;           // M
 };
 
+// x[0] + .. + x[K - 1], in pairs
+template <int K, class V>
+__device__ __forceinline__ V pairwise(const V* x)
+{
+  if constexpr (K == 1) return x[0];
+  else return pairwise<K / 2>(x) + pairwise<K - K / 2>(x + K / 2);
+}
+
 // A (16 RM) x 16 tile of dW per workgroup, the batch split over its WAVES wavefronts and summed in
 // wavefront order through LDS: deterministic, and no workspace beyond the caller's. The
 // operands are read in MFMA layout straight from memory (lane l: row l / 16 of four, RM
 // consecutive columns from RM (l % 16)), two batches of U steps of 4 rows in flight: the operands
 // come from other XCDs' L2s, ~2 us away (one batch of 8: 78 us for a hidden layer's launch at
-// batch 8,192, two of 16: 49). Tiles of column 0 add up db.
+// batch 8,192, two of 16: 49). Tiles of column 0 add up db: pairwise within a batch of loads and
+// over wavefronts and rows (at batch 8,192 within 4.2e-8 of the FP64 sums, as 256 strided sums and a
+// tree; one running sum per lane, added in wavefront order: 1.2e-7, and no faster).
 template <int RM, int WAVES>
 constexpr int grad_lds() { return WAVES * 64 * (4 * RM + RM); }
 
@@ -209,10 +219,9 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
 #pragma unroll
     for (int u = 0; u < U; ++u)
 #pragma unroll
-      for (int e = 0; e < RM; ++e) {
+      for (int e = 0; e < RM; ++e)
         acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(va[u][e], vb[u], acc[e], 0, 0, 0);
-        bs[e] += va[u][e];
-      }
+    bs += pairwise<U>(va);
   };
   if (U <= steps) load(va[0], vb[0], 0);
   for (; s + 2 * U <= steps; s += 2 * U) {
@@ -224,15 +233,18 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
     __builtin_amdgcn_sched_barrier(0);
   }
   if (s + U <= steps) { products(va[0], vb[0]); s += U; }
+  vec t0 = {}, t1 = {};                           // the rest of the rows: even and odd ones
   for (; s < steps; ++s) {
     const vec ta = *(const vec*)(a + (size_t)4 * s * g.M);
     const float tb = b[(size_t)4 * s * g.N];
 #pragma unroll
-    for (int e = 0; e < RM; ++e) {
+    for (int e = 0; e < RM; ++e)
       acc[e] = __builtin_amdgcn_mfma_f32_16x16x4f32(ta[e], tb, acc[e], 0, 0, 0);
-      bs[e] += ta[e];
-    }
+    const vec t = t0 + ta;
+    t0 = t1;
+    t1 = t;
   }
+  bs += t0 + t1;
   float* red = lds;                               // [wave][RM * 4][64]
   float* redb = lds + WAVES * 64 * 4 * RM;        // [wave][RM][64]
 #pragma unroll
@@ -250,10 +262,12 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
   }
   if (n0 == 0 && threadIdx.x < 16 * RM) {
     const int e = threadIdx.x >> 4, c = threadIdx.x & 15;
-    float v = 0.0f;
+    float v[4 * WAVES];
+#pragma unroll
     for (int k = 0; k < WAVES; ++k)
-      for (int r = 0; r < 4; ++r) v += redb[(k * RM + e) * 64 + 16 * r + c];
-    g.db[m0 + RM * c + e] = v;
+#pragma unroll
+      for (int r = 0; r < 4; ++r) v[4 * k + r] = redb[(k * RM + e) * 64 + 16 * r + c];
+    g.db[m0 + RM * c + e] = pairwise<4 * WAVES>(v);
   }
 }
 

@@ -75,6 +75,50 @@ def test_forward_and_gradients_vs_oracle(L, case):
     assert abs(float(part.sum()) / (B * 55) - loss) <= 1e-5 * loss
 
 
+def backward(L, p, X, T):
+    """(gradients, work) of one batch: work holds dZ of layer 1, then of layer 2, at the end."""
+    B, H = X.shape[0], hidden_width()
+    dp, dX, dT = t32(p), t32(X), t32(T)
+    acts = torch.full((6 * B * H + B * IN,), np.nan, dtype=torch.float32, device=dev)
+    grads = torch.full_like(dp, np.nan)
+    work = torch.full((2 * B * H,), np.nan, dtype=torch.float32, device=dev)
+    part = torch.full(((B * IN + 255) // 256,), np.nan, dtype=torch.float32, device=dev)
+    assert L.kx_mlp_forward(_p(dp), B, _p(dX), _p(acts), None) == 0
+    assert L.kx_mlp_backward(_p(dp), B, _p(dX), _p(acts), _p(dT), _p(grads), _p(work), _p(part), None) == 0
+    torch.cuda.synchronize()
+    return grads.cpu().numpy(), work.cpu().numpy().reshape(2, B, H)
+
+
+def inputs(B, seed):
+    rng = np.random.default_rng(seed)
+    X = rng.normal(size=(B, IN)).astype(np.float32)
+    X[:, 55:] = 0.0
+    return X, rng.normal(size=(B, IN)).astype(np.float32)
+
+
+@pytest.mark.parametrize('B', [64, 960, 8192, 8256])
+def test_bias_gradient_sums(L, case, B):
+    """The bias gradients of layers 1 (16 wavefronts) and 2 (8) are no further from the FP64 sums
+    of their dZ than FP32 sums in 256 strided parts and a tree (the columns' own rounding: 1.3
+    covers the spread of a norm over 3 x 256 columns)."""
+    p, _, _ = case
+    H = hidden_width()
+    db = (H * IN, H * IN + H + H * H)                       # offsets of b1, b2
+    e, ref = np.zeros(2), np.zeros(2)
+    for seed in (11, 12, 13):
+        g, dZ = backward(L, p, *inputs(B, seed))
+        for i, z in enumerate(dZ):
+            exact = z.astype(np.float64).sum(0)
+            parts = np.zeros((256, H), np.float32)
+            for r in range(0, B, 256):
+                parts[:min(256, B - r)] += z[r:r + 256]
+            while len(parts) > 1:
+                parts = parts[:len(parts) // 2] + parts[len(parts) // 2:]
+            e[i] += ((g[db[i]:db[i] + H] - exact) ** 2).sum()
+            ref[i] += ((parts[0] - exact) ** 2).sum()
+    assert np.all(np.sqrt(e / ref) < 1.3), np.sqrt(e / ref)
+
+
 def test_adam_vs_oracle(L, case):
     p, _, _ = case
     rng = np.random.default_rng(4)
