@@ -57,7 +57,8 @@ __device__ __forceinline__ uint16_t to_bf16(float f)
 // ---- training GEMMs on FP32 MFMA (v_mfma_f32_32x32x2_f32, 16x16x4): full FP32 products and sums
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4t __attribute__((ext_vector_type(4)));
-typedef float f32x2t __attribute__((ext_vector_type(2)));
+// in the caller's arrays, which are aligned as float
+typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));
 
 // What a GEMM tile does with its result c at (row, col):
 //   BIAS_GELU  Z = c + bias[col], H = gelu(Z)          (hidden layer forward)
@@ -99,13 +100,13 @@ __device__ __forceinline__ void gemm_tile(const GemmArgs& g, int tm, int tn, flo
 #pragma unroll
     for (int r = 0; r < LA; ++r) {
       const int e = threadIdx.x + r * TH;
-      ra[r] = *(const f32x4t*)(g.A + (size_t)(m0 + e / (kBK / 4)) * g.K + k0 + 4 * (e % (kBK / 4)));
+      ra[r] = *(const f32x4u*)(g.A + (size_t)(m0 + e / (kBK / 4)) * g.K + k0 + 4 * (e % (kBK / 4)));
     }
 #pragma unroll
     for (int r = 0; r < LB; ++r) {
       const int e = threadIdx.x + r * TH;
-      if (TB) rb[r] = *(const f32x4t*)(g.B + (size_t)(k0 + e / (NT / 4)) * g.N + n0 + 4 * (e % (NT / 4)));
-      else rb[r] = *(const f32x4t*)(g.B + (size_t)(n0 + e / (kBK / 4)) * g.K + k0 + 4 * (e % (kBK / 4)));
+      if (TB) rb[r] = *(const f32x4u*)(g.B + (size_t)(k0 + e / (NT / 4)) * g.N + n0 + 4 * (e % (NT / 4)));
+      else rb[r] = *(const f32x4u*)(g.B + (size_t)(n0 + e / (kBK / 4)) * g.K + k0 + 4 * (e % (kBK / 4)));
     }
   };
   auto store = [&]() {
@@ -195,6 +196,7 @@ template <int RM, int WAVES>
 __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* lds)
 {
   typedef float vec __attribute__((ext_vector_type(RM)));
+  typedef float vecu __attribute__((ext_vector_type(RM), aligned(4)));
   constexpr int U = WAVES > 8 ? 8 : 16;        // rows of 4 per batch of loads; two batches in flight
   const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, i = lane & 15, q = lane >> 4;
   const int tn = g.N / 16, m0 = (tile / tn) * 16 * RM, n0 = (tile % tn) * 16;
@@ -211,7 +213,7 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
   auto load = [&](vec (&va)[U], float (&vb)[U], int at) {
 #pragma unroll
     for (int u = 0; u < U; ++u) {
-      va[u] = *(const vec*)(a + (size_t)4 * (at + u) * g.M);
+      va[u] = *(const vecu*)(a + (size_t)4 * (at + u) * g.M);
       vb[u] = b[(size_t)4 * (at + u) * g.N];
     }
   };
@@ -235,7 +237,7 @@ __device__ __forceinline__ void grad_tile(const GradArgs& g, int tile, float* ld
   if (s + U <= steps) { products(va[0], vb[0]); s += U; }
   vec t0 = {}, t1 = {};                           // the rest of the rows: even and odd ones
   for (; s < steps; ++s) {
-    const vec ta = *(const vec*)(a + (size_t)4 * s * g.M);
+    const vec ta = *(const vecu*)(a + (size_t)4 * s * g.M);
     const float tb = b[(size_t)4 * s * g.N];
 #pragma unroll
     for (int e = 0; e < RM; ++e)

@@ -75,14 +75,13 @@ def test_forward_and_gradients_vs_oracle(L, case):
     assert abs(float(part.sum()) / (B * 55) - loss) <= 1e-5 * loss
 
 
-def backward(L, p, X, T):
-    """(gradients, work) of one batch: work holds dZ of layer 1, then of layer 2, at the end."""
+def backward(L, p, X, T, shift=0):
+    """(gradients, work) of one batch: work holds dZ of layer 1, then of layer 2, at the end. Every
+    array starts `shift` floats into its allocation."""
     B, H = X.shape[0], hidden_width()
-    dp, dX, dT = t32(p), t32(X), t32(T)
-    acts = torch.full((6 * B * H + B * IN,), np.nan, dtype=torch.float32, device=dev)
-    grads = torch.full_like(dp, np.nan)
-    work = torch.full((2 * B * H,), np.nan, dtype=torch.float32, device=dev)
-    part = torch.full(((B * IN + 255) // 256,), np.nan, dtype=torch.float32, device=dev)
+    nans = lambda n: torch.full((n + shift,), np.nan, dtype=torch.float32, device=dev)[shift:]
+    dp, dX, dT = (nans(a.size).copy_(t32(a).reshape(-1)) for a in (p, X, T))
+    acts, grads, work, part = (nans(n) for n in (6 * B * H + B * IN, p.size, 2 * B * H, (B * IN + 255) // 256))
     assert L.kx_mlp_forward(_p(dp), B, _p(dX), _p(acts), None) == 0
     assert L.kx_mlp_backward(_p(dp), B, _p(dX), _p(acts), _p(dT), _p(grads), _p(work), _p(part), None) == 0
     torch.cuda.synchronize()
@@ -94,6 +93,14 @@ def inputs(B, seed):
     X = rng.normal(size=(B, IN)).astype(np.float32)
     X[:, 55:] = 0.0
     return X, rng.normal(size=(B, IN)).astype(np.float32)
+
+
+@pytest.mark.parametrize('shift', [1, 2, 3])
+def test_arrays_need_no_more_than_float_alignment(L, case, shift):
+    p, _, _ = case
+    X, T = inputs(192, 14)
+    for a, b in zip(backward(L, p, X, T), backward(L, p, X, T, shift)):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
 
 
 @pytest.mark.parametrize('B', [64, 960, 8192, 8256])
