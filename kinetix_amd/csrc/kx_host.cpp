@@ -664,8 +664,9 @@ int kx_sur_transport(kx_mech_t h, int n, int offsetT, int offset, const double* 
   // 3. plain kernel over the audit samples + queued out-of-hull states, in place: it reads
   //    the queued states, compares mu, lambda and rho*D of the audit entries with the surrogate's,
   //    and overwrites the outputs with its own. The queue length is read on the device; the
-  //    grid covers the longest possible queue (n_audit + n), and the workgroups past the
-  //    actual end return at once, after the working ones (the first) were dispatched.
+  //    kernel strides over the queue on a grid capped at the workgroups resident at once. (A
+  //    queue kernel of one lane per state, in code objects generated before those that stride,
+  //    takes a grid over the longest possible queue, n_audit + n.)
   {
     long long oT = offsetT, o = offset;
     double Tref = m->ref_T;
@@ -674,8 +675,8 @@ int kx_sur_transport(kx_mech_t h, int n, int offsetT, int offset, const double* 
                     (void*)&d_state, &d_cond, &d_visc, &d_rhoD, &d_Dkm, &Tref};
     const long long longest = (long long)n_audit + n;
     if (m->queue_lanes > 1 && !m->group_states.count("kx_bk2_fp64_queue")) {
-      // the cooperative form strides over the queue: a grid of the workgroups resident at
-      // once, or fewer when even the longest possible queue needs fewer
+      // the cooperative form (16 lanes per state): fewer workgroups when even the longest
+      // possible queue needs fewer
       const long long per_wg = m->block.at("kx_bk2_fp64_queue") / m->queue_lanes;
       const long long grid = std::min((longest + per_wg - 1) / per_wg, m->queue_grid_cap);
       if ((rc = launch_grid(m, "kx_bk2_fp64_queue", grid, stream, args))) return rc;

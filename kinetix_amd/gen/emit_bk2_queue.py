@@ -1,7 +1,8 @@
-"""The surrogate's plain pass, cooperative: kx_bk2_fp64_queue with several lanes per state, for
-mechanisms whose plain transport kernel runs one state per lane (emit_bk2_quad.fits says which
-do not): the pass evaluates the same polynomials in ln T as that kernel, so that the states it
-recomputes equal the plain kernel's to rounding.
+"""The surrogate's plain pass, cooperative: kx_bk2_fp64_queue with 16 lanes per state, for
+mechanisms below 20 species, whose plain transport kernel runs one state per lane
+(emit_bk2_quad.fits; from 20 to the surrogate's 62 species the pass runs that module's routine):
+the pass evaluates the same polynomials in ln T as that kernel, so that the states it recomputes
+equal the plain kernel's to rounding.
 
 kx_sur_transport runs the plain FP64 transport kernel over a queue of state ids -- the 1 %
 audit samples, then the out-of-hull states -- reading each state in place and writing its
@@ -40,12 +41,10 @@ from __future__ import annotations
 
 import numpy as np
 
-from . import emit_bk2_quad
 from . import emit_hip as E
 from . import emit_rolled as RL
 
-LPS = emit_bk2_quad.LPS      # of the mechanisms whose transport runs four lanes per state
-COOP_LPS = 16                # of this module's kernel
+LPS = 16
 BLOCK = 1024
 
 
@@ -63,12 +62,12 @@ def tables(t):
     return tri, np.asarray(t['C1'], np.float64), np.asarray(t['C2'], np.float64), sp
 
 
-def lds_bytes(t, lps=COOP_LPS, block=BLOCK):
+def lds_bytes(t, lps=LPS, block=BLOCK):
     N = int(t['n_species'])
     return 8 * (5 * N * (N - 1) // 2 + 2 * N * N + 12 * N + 2 * N * (block // lps))
 
 
-def emit(t, info, lps=COOP_LPS, block=BLOCK, unroll=8):
+def emit(t, info, lps=LPS, block=BLOCK, unroll=8):
     N = int(t['n_species'])
     if block % lps or 64 % lps:
         raise ValueError('lanes per state must divide the wavefront and the workgroup')

@@ -943,67 +943,38 @@ def _emit_conductivity(S, t):
     S('const double lambda = sqrT * (0.5 * (sum1 + 1.0 / sum2));')
 
 
-def _emit_bk2_fp64(t, info, pstate=False, block=BLOCK, queue=False):
+def _emit_bk2_fp64(t, info, pstate=False, block=BLOCK):
     """pstate=False: kx_bk2_fp64, scalar p (the reference's transport kernel).
     pstate=True: kx_bk2_fp64_pstate, p [Pa] per state, also writes D_km.
-    queue=True: kx_bk2_fp64_queue, the plain kernel over a device queue of state ids (the
-    surrogate's audit samples, then its out-of-hull states), p per state, reading each state
-    and writing its outputs in place; audit entries first compare mu and lambda with the
-    surrogate values they replace.
     block: threads per workgroup (the host launches with the kernel's launch bound). The
     kernel's LDS constant pool (~85 KB for GRI-3.0) admits one workgroup per CU, so 512
     threads (8 waves) is what gives 2 waves/SIMD: 8.4 ms instead of 14.5 at 256 threads for
     4M states, despite ~160 VGPRs spilled to scratch; 768 and 1024 spill far more and are
-    2-3x slower. The queue form is latency-bound (a few 10^4 states): 256 threads, one wave per
-    SIMD on every CU, each wave free to use 372 of the 512 registers without a spill. It is
-    emitted only for a mechanism whose tables do not fit the cooperative queue kernel's LDS
-    (emit_bk2_queue, 16 lanes per state)."""
+    2-3x slower."""
     N = int(t['n_species'])
     S = _Src()
     S(f'extern "C" __global__ void __launch_bounds__({block})', 0)
-    if queue:
-        S('kx_bk2_fp64_queue(const int n_audit,', 0)
-        S('            const int* __restrict__ queue, int* __restrict__ counters,', 0)
-        S('            const int* __restrict__ flags, const double tol, const double tol_rhoD,', 0)
-        S('            const long long offsetT, const long long offset,', 0)
-        S('            const double* __restrict__ p_state,', 0)
-        S('            const double* __restrict__ state, double* __restrict__ conductivity,', 0)
-        S('            double* __restrict__ viscosity, double* __restrict__ rhoD,', 0)
-        S('            double* __restrict__ Dkm, const double Tref)', 0)
-        S('{', 0)
-        S('// queue entries [0, n_audit) are audit samples, then counters[0] out-of-hull states;')
-        S('// counters: [0] out-of-hull states queued, [1] failed audits. The grid covers the')
-        S('// longest possible queue (every state out of hull); workgroups past the actual end')
-        S('// return before staging the LDS table, after the working ones were dispatched.')
-        S('const long long valid = (long long)n_audit + max(counters[0], 0);')
-        S(f'if ((long long)blockIdx.x * {block} >= valid) return;   // whole workgroup past the queue')
-        S(POOL_MARK)
-        S(f'const long long slot = (long long)blockIdx.x * {block} + threadIdx.x;')
-        S('if (slot >= valid) return;')
-        S('const long long id = queue[slot];')
-        S('const double p = p_state[id];')
-    elif pstate:
+    if pstate:
         S('kx_bk2_fp64_pstate(const int n_states, const long long offsetT, const long long offset,', 0)
         S('            const double* __restrict__ p_state,', 0)
     else:
         S('kx_bk2_fp64(const int n_states, const long long offsetT, const long long offset,', 0)
         S('            const double pressure,', 0)
-    if not queue:
-        S('            const double* __restrict__ state, double* __restrict__ conductivity,', 0)
-        S('            double* __restrict__ viscosity, double* __restrict__ rhoD,', 0)
-        if pstate:
-            S('            double* __restrict__ Dkm, const double Tref,', 0)
-        else:
-            S('            const double Tref,', 0)
-        S('            const int* __restrict__ n_dev)', 0)
-        S('{', 0)
-        S('// n_dev (optional): a state count known only on the device; workgroups wholly past it')
-        S('// return before staging the LDS table')
-        S(f'if (n_dev && (long long)blockIdx.x * {block} >= *n_dev) return;')
-        S(POOL_MARK)
-        S(f'const long long id = (long long)blockIdx.x * {block} + threadIdx.x;')
-        S('if (id >= n_states || (n_dev && id >= *n_dev)) return;')
-        S('const double p = ' + ('p_state[id];' if pstate else 'pressure;'))
+    S('            const double* __restrict__ state, double* __restrict__ conductivity,', 0)
+    S('            double* __restrict__ viscosity, double* __restrict__ rhoD,', 0)
+    if pstate:
+        S('            double* __restrict__ Dkm, const double Tref,', 0)
+    else:
+        S('            const double Tref,', 0)
+    S('            const int* __restrict__ n_dev)', 0)
+    S('{', 0)
+    S('// n_dev (optional): a state count known only on the device; workgroups wholly past it')
+    S('// return before staging the LDS table')
+    S(f'if (n_dev && (long long)blockIdx.x * {block} >= *n_dev) return;')
+    S(POOL_MARK)
+    S(f'const long long id = (long long)blockIdx.x * {block} + threadIdx.x;')
+    S('if (id >= n_states || (n_dev && id >= *n_dev)) return;')
+    S('const double p = ' + ('p_state[id];' if pstate else 'pressure;'))
     _emit_bk2_prelude(S, t, 'id')
     rcpW, W = t['rcpW'], t['W']
     # diffusion first: x and the N row sums are live
@@ -1011,28 +982,9 @@ def _emit_bk2_fp64(t, info, pstate=False, block=BLOCK, queue=False):
     S('const double TsqrT = T * sqrT;')
     S(f'const double rho = p * {lit(1.0 / float(t["R"]))} * rcpT * Mbar;')
     S('const double pMbar = p * Mbar;')
-    def stores(with_dkm):
-        for k in range(N):
-            S(f'{{ const double D = TsqrT * (Mbar - {lit(W[k])} * x{k}) / (pMbar * s{k});')
-            if queue:
-                # audit of rho*D: the surrogate's value is read before it is overwritten (an
-                # unconditional load; the flag masks non-audit entries, no branch per store)
-                S(f'  const double v = rho * D; const double e = fabs(rhoD[{k} * offset + id] / v - 1.0);')
-                S(f'  bad_rhoD |= !(e <= tol_rhoD); rhoD[{k} * offset + id] = v;'
-                  + (f' Dkm[{k} * offset + id] = D; }}' if with_dkm else ' }'))
-            else:
-                S(f'  rhoD[{k} * offset + id] = rho * D;' + (f' Dkm[{k} * offset + id] = D; }}' if with_dkm else ' }'))
-    if queue:
-        S('bool bad_rhoD = false;   // max_k |rhoD_k(surrogate) / rhoD_k - 1| > tol_rhoD, or NaN')
-        # D_km optional: one uniform branch around the stores (a branch per store splits the
-        # kernel into ~10^2 blocks, and the scheduler then spills ~10^4 VGPRs)
-        S('if (Dkm) {')
-        stores(True)
-        S('} else {')
-        stores(False)
-        S('}')
-    else:
-        stores(pstate)
+    for k in range(N):
+        S(f'{{ const double D = TsqrT * (Mbar - {lit(W[k])} * x{k}) / (pMbar * s{k});')
+        S(f'  rhoD[{k} * offset + id] = rho * D;' + (f' Dkm[{k} * offset + id] = D; }}' if pstate else ' }'))
     # viscosity: Wilke, eta_k = poly, Phi^(1/2)_kj = C1 + C2 eta_k / eta_j
     S('__builtin_amdgcn_sched_barrier(0);')
     S('// ---- viscosity (Wilke)')
@@ -1051,16 +1003,8 @@ def _emit_bk2_fp64(t, info, pstate=False, block=BLOCK, queue=False):
         S('}')
     S('__builtin_amdgcn_sched_barrier(0);')
     S('const double mu = sqrT * vis;')
-    if not queue:
-        S('viscosity[id] = mu;')
+    S('viscosity[id] = mu;')
     _emit_conductivity(S, t)
-    if queue:
-        S('if (slot < n_audit && flags[id] == 0) {   // audit of a state the surrogate answered')
-        S('  const double ev = fabs(viscosity[id] / mu - 1.0);')
-        S('  const double ec = fabs(conductivity[id] / lambda - 1.0);')
-        S('  if (!(ev <= tol) || !(ec <= tol) || bad_rhoD) atomicAdd(counters + 1, 1);')
-        S('}')
-        S('viscosity[id] = mu;')
     S('conductivity[id] = lambda;')
     S('}', 0)
     return S.text()
@@ -1219,12 +1163,8 @@ def generate(tables, info, opts=None):
         parts.append(_with_pool('kx_bk2_fp64_pstate_k', _emit_bk2_fp64, tables, info, True, o['bk2_block'],
                                 lds=o['lds_pool'], block=o['bk2_block']))
         from . import emit_bk2_queue as BQ
-        if BQ.lds_bytes(tables) <= 160 * 1024:
-            # several lanes per state: the pass over a few 10^4 queued states is latency-bound
+        if BQ.lds_bytes(tables) <= 160 * 1024:      # every mechanism of this branch a surrogate can have
             parts.append(BQ.emit(tables, info))
-        else:
-            parts.append(_with_pool('kx_bk2_fp64_queue_k', _emit_bk2_fp64, tables, info, True,
-                                    256, True, lds=o['lds_pool'], block=256))
         from . import emit_bk2_mfma as BM
         # the constant pool goes to LDS only beside the Wilke tables within 160 KB per CU
         parts.append(_with_pool('kx_bk2_fp64_mfma_k', BM.emit, tables, info, lds=o['lds_pool'],

@@ -366,8 +366,6 @@ def test_cooperative_queue_kernel_arithmetic_vs_oracle(gri, oracle):
     from kinetix_amd.gen import emit_bk2_queue as BQ
     info, t = gri
     assert BQ.lds_bytes(t) <= 160 * 1024
-    src = open(os.path.join(MDIR, 'kernels.hip')).read()
-    assert f'kx_bk2q_lanes = {BQ.LPS};' in src
     s, p = states.sample_transport_set(64, info['species'], t['W'], seed=21)
     got = _queue_kernel_numpy(t, s, p)
     ref = oracle.transport(s, 1.0, 1.0, p_state=p)
@@ -377,6 +375,29 @@ def test_cooperative_queue_kernel_arithmetic_vs_oracle(gri, oracle):
     t2 = dict(t)
     t2['C1'] = np.asarray(t['C1']).T.copy()
     assert np.max(np.abs(_queue_kernel_numpy(t2, s, p)[1] / ref[1] - 1)) > 1e-6
+
+
+@pytest.mark.parametrize('mech,lanes,quad', [('LiDryer', 16, False), ('gri30', 4, True), ('NH3Konnov_edit', 4, True)])
+def test_queue_kernel_by_species_count(mech, lanes, quad):
+    """Below 20 species the queue kernel is the cooperative one (16 lanes per state), from 20 on the
+    plain kernel's routine (4 lanes, 16 states per group); the code objects say which."""
+    import re
+    src = open(os.path.join(os.path.dirname(MDIR), mech, 'kernels.hip')).read()
+    assert re.findall(r'kx_bk2q_lanes = (\d+);', src) == [str(lanes)]
+    assert src.count('kx_bk2_fp64_queue_states_per_group = 16;') == quad
+    assert src.count('kxquad::queued<') == quad and src.count('kx_bk2q_gsum(double') == (not quad)
+
+
+def test_every_surrogate_width_has_a_queue_kernel():
+    """Up to the surrogate's 62 species one of the two queue kernels fits the LDS, whatever the rank
+    of the Wilke factor (at most the species count)."""
+    from kinetix_amd.gen import emit_bk2_quad as Q
+    from kinetix_amd.gen import emit_bk2_queue as BQ
+    for N in range(1, 63):
+        if N < 20:
+            assert BQ.lds_bytes({'n_species': N}) <= 160 * 1024
+        else:
+            assert 8 * Q.table_doubles(N, (N + 3) // 4) <= Q.LDS_MAX
 
 
 def _tile_kernel_numpy(t, s, p, wil=None):

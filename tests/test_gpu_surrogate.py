@@ -441,3 +441,36 @@ def test_audit_sampling_edges(trained, gri, n, stride, offset):
         a_, b_ = a.view(-1, n)[:, aud], b.view(-1, n)[:, aud]
         assert same_as_plain(a_, b_)
         assert torch.all(torch.isfinite(a.view(-1, n)))
+
+
+@pytest.mark.parametrize('mech,n', [('LiDryer', 1), ('LiDryer', 1001), ('NH3Konnov_edit', 17), ('NH3Konnov_edit', 1001)])
+@pytest.mark.parametrize('dkm', [True, False])
+def test_queue_kernels_of_other_mechanisms(mech, n, dkm):
+    """Every state audited behind an untrained network, no whole-call fallback: each output then
+    comes from the queue kernel, 16 lanes per state (9 species) or the plain kernel's routine (36),
+    on a strided layout, and equals the plain kernel's to rounding; nothing else is written."""
+    from kinetix_amd.gen import tables as tb
+    kx = Kinetix(mech)
+    try:
+        info, t = tb.load(kx.dir)
+        N, ld = kx.nSpecies(), n + 7
+        kx.build(states.ONE_ATM, 1.0, states.reference_mass_fractions(info['species'], t['W']))
+        sur = Surrogate(kx)
+        norm = np.zeros((4, IN), np.float32)
+        norm[1], norm[2], norm[3] = 1.0, -np.inf, np.inf
+        sur.set_model(init_params(5), norm, np.stack([np.zeros(IN), np.ones(IN)]))
+        s, p = states.sample_any(ld, info['species'], t['W'], T_range=(300.0, 2500.0), seed=50 + n,
+                                 p_range_atm=(0.5, 40.0))
+        ds, dp = (torch.from_numpy(np.ascontiguousarray(a)).to(dev).reshape(-1) for a in (s, p))
+        z = lambda m: torch.full((m,), np.nan, dtype=torch.float64, device=dev)
+        got = [z(n), z(n), z(N * ld)] + ([z(N * ld)] if dkm else [])
+        res = sur.infer(n, ld, ld, dp, ds, *got, audit_stride=1, max_audit_fail=1.0)
+        ref = sur.plain(n, ld, ld, dp, ds)
+        torch.cuda.synchronize()
+        assert res['audited'] == n and res['out_of_hull'] == 0 and not res['whole_call_fallback']
+        for a, b in zip(got, ref):
+            a_, b_ = a.view(-1, n if a.numel() == n else ld), b.view(-1, n if b.numel() == n else ld)
+            assert same_as_plain(a_[:, :n], b_[:, :n])
+            assert bool(torch.isnan(a_[:, n:]).all())
+    finally:
+        kx.close()
