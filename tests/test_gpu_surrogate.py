@@ -95,6 +95,31 @@ def inputs(B, seed):
     return X, rng.normal(size=(B, IN)).astype(np.float32)
 
 
+@pytest.mark.parametrize('B', [64, 128, 512, 1024, 1536, 8192, 8256])
+def test_gradients_per_layer(L, case, B):
+    """Every layer's weight and bias gradient against the oracle, at batches that take each part of
+    the weight gradient's loop (per wavefront B / 32 rows of 4, in layer 1 B / 64; batches of 16,
+    there 8): the rest only (64, 128), one batch (512), one turn of two (1,024), a turn and one
+    (1,536), turns only (8,192), turns and a rest (8,256).
+
+    Tolerance on the 2-norms: a running FP32 sum of n terms of random sign is off by
+    2^-24 / sqrt(3) sqrt(n / 2) of its value in the root mean square; n is 256 in each of up to three
+    products before a gradient, and B / 8 + 32 in its own chains of rows. 1.5 for what is not
+    random."""
+    p, _, _ = case
+    X, T = inputs(B, 20 + B)
+    g, _ = backward(L, p, X, T)
+    ref = mo.loss_and_grad(p, X, T)[2]
+    tol = 1.5 * 2.0 ** -24 / np.sqrt(3.0) * np.sqrt((3 * 256 + B / 8 + 32) / 2)
+    o = 0
+    for rows, cols in mo.SHAPES:
+        for n in (rows * cols, rows):
+            e = np.linalg.norm(g[o:o + n] - ref[o:o + n]) / np.linalg.norm(ref[o:o + n])
+            assert e < tol, (rows, cols, n, e, tol)
+            o += n
+    assert o == g.size
+
+
 @pytest.mark.parametrize('shift', [1, 2, 3])
 def test_arrays_need_no_more_than_float_alignment(L, case, shift):
     p, _, _ = case
