@@ -175,9 +175,13 @@ int kx_selftest_mfma_layout(float *d_out, void *stream);
  * the lane layout the FP64-MFMA transport kernel assumes. */
 int kx_selftest_mfma_f64_layout(int mode, double *d_out, void *stream);
 
-/* Diagnostics (no reference counterpart): d_out[i] = the transport kernels' FP64 reciprocal
- * (v_rcp_f64 + two Newton steps, kinetix_amd/csrc/kx_rcp.h) of d_in[i], i < n. */
+/* Diagnostics (no reference counterpart): d_out[i] = the transport and rate kernels' FP64
+ * reciprocal (v_rcp_f64 and one third-order step, kinetix_amd/csrc/kx_rcp.h) of d_in[i], i < n. */
 int kx_selftest_rcp(int n, const double *d_in, double *d_out, void *stream);
+
+/* Diagnostics (no reference counterpart): d_out[i] = the rate kernels' kx_exp2 (which = 0), kx_exp (1)
+ * or kx_log2 (2), kinetix_amd/csrc/kx_exp.h, of d_in[i], i < n. */
+int kx_selftest_exp(int which, int n, const double *d_in, double *d_out, void *stream);
 
 /* Learned transport surrogate (no reference counterpart): see kinetix_mi_surrogate.h. */
 

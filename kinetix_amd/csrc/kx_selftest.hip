@@ -8,6 +8,7 @@
 #include <hip/hip_runtime.h>
 
 #include "../../include/kinetix_mi.h"
+#include "kx_exp.h"
 #include "kx_rcp.h"
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -65,7 +66,7 @@ extern "C" int kx_selftest_mfma_f64_layout(int mode, double* d_out, void* stream
   return hipGetLastError() == hipSuccess ? KX_OK : KX_ERR_HIP;
 }
 
-// kx_rcp (the transport kernels' reciprocal) on n inputs: out[i] = kx_rcp(in[i]).
+// kx_rcp (the transport and rate kernels' reciprocal) on n inputs: out[i] = kx_rcp(in[i]).
 __global__ void __launch_bounds__(256) kx_rcp_probe(int n, const double* __restrict__ in,
                                                     double* __restrict__ out)
 {
@@ -79,5 +80,24 @@ extern "C" int kx_selftest_rcp(int n, const double* d_in, double* d_out, void* s
   if (n == 0) return KX_OK;
   hipLaunchKernelGGL(kx_rcp_probe, dim3((n + 255) / 256), dim3(256), 0, (hipStream_t)stream, n,
                      d_in, d_out);
+  return hipGetLastError() == hipSuccess ? KX_OK : KX_ERR_HIP;
+}
+
+// The rate kernels' exponentials on n inputs: out[i] = kx_exp2 (which 0), kx_exp (1) or kx_log2 (2).
+__global__ void __launch_bounds__(256) kx_exp_probe(int which, int n, const double* __restrict__ in,
+                                                    double* __restrict__ out)
+{
+  const long long i = (long long)blockIdx.x * 256 + threadIdx.x;
+  if (i >= n) return;
+  const double x = in[i];
+  out[i] = which == 0 ? kx_exp2(x) : which == 1 ? kx_exp(x) : kx_log2(x);
+}
+
+extern "C" int kx_selftest_exp(int which, int n, const double* d_in, double* d_out, void* stream)
+{
+  if (which < 0 || which > 2 || n < 0 || (n > 0 && (!d_in || !d_out))) return KX_ERR_INVALID_ARG;
+  if (n == 0) return KX_OK;
+  hipLaunchKernelGGL(kx_exp_probe, dim3((unsigned)(((long long)n + 255) / 256)), dim3(256), 0, (hipStream_t)stream,
+                     which, n, d_in, d_out);
   return hipGetLastError() == hipSuccess ? KX_OK : KX_ERR_HIP;
 }
