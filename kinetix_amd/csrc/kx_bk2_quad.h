@@ -18,10 +18,11 @@
 // The Wilke rule uses that C1_kj + C2_kj eta_k / eta_j = (W_j / (8 (W_k + W_j)))^(1/4) (u_k + u_j) / u_j
 // with u = eta W^(-1/4): S_k = sum_j a_j M_kj (u_k + u_j)^2, a_j = x_j sqrt(W_j) / u_j^2, with the
 // positive definite matrix M_kj = (8 (W_k + W_j))^(-1/2), a smooth function of W_k + W_j: its
-// pivoted Cholesky factor L reaches FP64 rounding at rank 13-16 for every mechanism here
-// (entries of L L^T within 2.5e-16 of M; by Cauchy-Schwarz the products' magnitudes sum to at
-// most twice M_kj, so nothing cancels badly). S = u^2 L(L^T a) + 2 u L(L^T a u) + L(L^T a u^2) is
-// then six thin products per 16 states, all on MFMA.
+// pivoted Cholesky factor L reaches FP64 rounding at rank 13-16 for the combustion mechanisms here (up
+// to 93 g/mol; octane to dodecane 17-18), and at 21 of 22 where masses spread over a factor of 300
+// (ranks beyond 16 take a second block of z). Entries of L L^T are within 1e-15 of M; by
+// Cauchy-Schwarz the products' magnitudes sum to at most twice M_kj, so nothing cancels badly.
+// S = u^2 L(L^T a) + 2 u L(L^T a u) + L(L^T a u^2) is then six thin products per 16 states, all on MFMA.
 //
 // Bound: FP64 issue. v_mfma_f64 and FP64 VALU instructions do not overlap on this chip (32 v_fma
 // and 2 v_mfma take the sum of their times), so per 16 states the ~18k cycles of the pair blocks

@@ -45,7 +45,7 @@ def slots(N):
 def wilke_factor(W):
     """L (N x r) with (L L^T)_kj = (8 (W_k + W_j))^(-1/2) to FP64 rounding: pivoted Cholesky in 50
     digits until the residual is 1e-16 of every diagonal entry, rounded once at the end (the
-    entries of the rounded product are within 2.5e-16 of the matrix for the mechanisms here)."""
+    entries of the product are within 1e-15 of the matrix for the mechanisms here)."""
     prec, getcontext().prec = getcontext().prec, 50
     try:
         w = [Decimal(float(v)) for v in W]

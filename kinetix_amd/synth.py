@@ -18,6 +18,11 @@ irreversible elementary, three-body, Lindemann, Troe with and without T2, SRI wi
 parameters, falloff with an explicit collider species, and PLOG over 2-4 of {0.1, 1, 10,
 100} atm, a quarter of them with two summed rates at one pressure.
 
+heavy=True replaces the compositions (and so the molar masses): H_m with m from 1 to 300 in geometric
+steps, everything else the source's. Molar masses spread like this give the transport kernels'
+Wilke factor about the rank of the species count (21 of 22), where combustion mechanisms have 13
+to 18.
+
     python -m kinetix_amd.synth --source gri30.yaml --species 160 --reactions 1000 \
         --seed 20261205 --out kinetix_amd/mechs/synth160/synth160.yaml
 """
@@ -109,21 +114,25 @@ def _coverage_reaction(rng, names, reac, prod, kind):
     return out
 
 
-def write(source_yaml, n_species, n_reactions, seed, out_path, coverage=False):
+def write(source_yaml, n_species, n_reactions, seed, out_path, coverage=False, heavy=False):
     src = mechanism.load_yaml(source_yaml)
     pool = [s for s in src['species']]
     rng = np.random.default_rng(seed)
     pick = rng.integers(0, len(pool), size=n_species)
     names = [f'S{k:03d}' for k in range(n_species)]
+    species = [pool[i] for i in pick]
+    if heavy:
+        species = [dict(s, composition={'H': max(k + 1, round(300 ** (k / (n_species - 1))))})
+                   for k, s in enumerate(species)]
     lines = ['description: seeded synthetic mechanism (species resampled from '
              f'{os.path.basename(source_yaml)}, seed {seed})',
              'units: {length: cm, time: s, quantity: mol, activation-energy: cal/mol}',
              'phases:', f'- name: synth{n_species}', '  thermo: ideal-gas',
-             '  elements: [' + ', '.join(sorted({e for i in pick for e in pool[i]['composition']})) + ']',
+             '  elements: [' + ', '.join(sorted({e for s in species for e in s['composition']})) + ']',
              '  species: [' + ', '.join(names) + ']', '  kinetics: gas',
              '  transport: mixture-averaged', '  state: {T: 300.0, P: 1 atm}', '', 'species:']
-    for k, i in enumerate(pick):
-        lines += _species_block(names[k], pool[i])
+    for k, sp in enumerate(species):
+        lines += _species_block(names[k], sp)
     lines += ['', 'reactions:']
     if coverage:
         kinds = rng.choice(10, size=n_reactions, p=[0.3, 0.1, 0.12, 0.08, 0.08, 0.06, 0.06, 0.06, 0.06, 0.08])
@@ -190,8 +199,9 @@ def main(argv=None):
     ap.add_argument('--seed', type=int, default=SEED)
     ap.add_argument('--out', required=True)
     ap.add_argument('--coverage', action='store_true', help='every reaction form (see module doc)')
+    ap.add_argument('--heavy', action='store_true', help='widely spread molar masses (see module doc)')
     a = ap.parse_args(argv)
-    print(write(a.source, a.species, a.reactions, a.seed, a.out, coverage=a.coverage))
+    print(write(a.source, a.species, a.reactions, a.seed, a.out, coverage=a.coverage, heavy=a.heavy))
 
 
 if __name__ == '__main__':

@@ -103,7 +103,7 @@ def quad_numpy(t, s, p):
     return lam[:16], mu[:16], rows(D * rho), rows(D)
 
 
-@pytest.mark.parametrize('mech', MECHS + ['EtOHKonnov', 'synth160'])
+@pytest.mark.parametrize('mech', MECHS + ['EtOHKonnov', 'synth160', 'synth22heavy'])
 def test_quad_routine_vs_oracle(mech):
     info, t = load(mech)
     s, p = states.sample_any(16, info['species'], t['W'], T_range=(300.0, 2500.0), seed=31,
@@ -122,10 +122,24 @@ def test_quad_routine_vs_oracle(mech):
         assert np.max(np.abs(got / want - 1)) < 1e-12 + 2e-15 * kappa
 
 
+@pytest.mark.parametrize('mech,rank', [('gri30', 13), ('synth160', 13), ('synth22heavy', 21)])
+def test_wilke_factor_ranks(mech, rank):
+    """The factor reproduces its matrix to rounding at any rank; 22 molar masses spread over a factor of
+    300 in geometric steps have rank 21 and need a second block of 16 ranks."""
+    _, t = load(mech)
+    W = np.asarray(t['W'])
+    L = Q.wilke_factor(W)
+    assert L.shape[1] == rank
+    M = (8 * (W[:, None] + W)) ** -0.5
+    assert np.max(np.abs(L @ L.T / M - 1)) < 2e-15
+    assert np.max(np.abs(L) @ np.abs(L).T / M) < 2.0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize('mech,n', [('gri30', 1), ('gri30', 15), ('gri30', 2049), ('gri30', 33000),
                                     ('chempolimi_edit', 17), ('synth40cov', 4097),
-                                    ('EtOHKonnov', 1), ('EtOHKonnov', 2065), ('synth160', 33000)])
+                                    ('EtOHKonnov', 1), ('EtOHKonnov', 2065), ('synth160', 33000),
+                                    ('synth22heavy', 17), ('synth22heavy', 4097)])
 def test_quad_kernels_at_group_edges(mech, n):
     """Scalar, per-state-pressure and (straight-line mechanisms) MFMA entry points, the table
     resident in LDS and streamed (129 and 160 species), at state counts that end inside a 16-state group, fill every wavefront of the grid (256 x 8 x 16 states on a 256-CU GPU) and
