@@ -381,8 +381,9 @@ static int production_rates_impl(const char* kernel, kx_mech_t h, int n, int off
   double* r = d_rates;
   void* args[] = {&n, &oT, &o, &pressure_R, &pressure_, &s, &r, &Tref};
   // more states than a launch takes (8 lanes per state: 536,870,848) go in pieces: a state's
-  // rows lie at fixed distances from its first value, so a piece is the same call further on
-  const long long most = states_per_launch(m, kernel);
+  // rows lie at fixed distances from its first value, so a piece is the same call further on. Even
+  // with 1,024 lanes per state a launch takes 4,194,303, and most calls are spared the look-up.
+  const long long most = n <= 4194303 ? n : states_per_launch(m, kernel);
   long long left = n;
   do {
     n = (int)std::min(left, most);

@@ -41,7 +41,7 @@ def stub(tmp_path_factory):
     return out
 
 
-@pytest.mark.parametrize('n', [1, 1000, (1 << 29) - 8, 1 << 29, (1 << 30) + 7, (1 << 31) - 1])
+@pytest.mark.parametrize('n', [0, 1, 1000, 4194303, 4194304, (1 << 29) - 8, 1 << 29, (1 << 30) + 7, (1 << 31) - 1])
 @pytest.mark.parametrize('block,lanes', [(256, 0), (512, 8), (768, 12), (1024, 32)])
 def test_rates_of_any_state_count(stub, n, block, lanes):
     """Every state count an int holds is launched, whatever the kernel's lanes per state: pieces in
