@@ -1,6 +1,6 @@
 // Mixture-averaged transport (FP64), four lanes per state: the wave-level routine of
-// kx_bk2_fp64, kx_bk2_fp64_pstate and kx_bk2_fp64_queue for mechanisms whose pair tables fit the
-// LDS (kinetix/core/mix_transport.py:261-471; benchmark/okl/transportProps.okl:11-47).
+// kx_bk2_fp64, kx_bk2_fp64_pstate and kx_bk2_fp64_queue, with the pair tables in LDS or, beyond 72
+// species, their rows streamed through it (kinetix/core/mix_transport.py:261-471; benchmark/okl/transportProps.okl:11-47).
 //
 // A wavefront takes 16 states: lane l works on state l % 16, and lane group g = l / 16 owns the
 // species 4 m + g (slot m). Why this layout:

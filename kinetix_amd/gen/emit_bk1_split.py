@@ -249,12 +249,14 @@ def shape(t, info):
     not fit.
 
     Two workgroups of 8 per CU at 128 registers where the LDS holds two and a wavefront's sums
-    stay in registers (53 species / 325 reactions: 617 us for 1,048,576 states; one workgroup
-    per CU of 4 wavefronts with all registers 625). Larger mechanisms have one workgroup per CU:
-    12 wavefronts of 168 registers up to 52 sums (129 / 1,231, 100,003 states: 251 us; 8 of 256
-    registers 262, 16 of 128, which spill, 305), else 8 of 256 up to 112 sums, with values from LDS
-    kept for three reactions at a time instead of six (160 / 1,000, 524,288 states, 108 sums:
-    2,205 us against 2,258 with four; 12 wavefronts would have 99 sums for 168 registers)."""
+    stay in registers (53 species / 325 reactions: one workgroup per CU of 4 wavefronts with all
+    registers takes 1.3 % longer). Larger mechanisms have one workgroup per CU: 12 wavefronts of 168
+    registers up to 52 sums (129 / 1,231: 8 of 256 registers take 4 % longer, 16 of 128, which
+    spill, 22 %), else 8 of 256 up to 112 sums, with values from LDS kept for three reactions at a
+    time instead of six (160 / 1,000, 108 sums: with four 2.4 % longer; 12 wavefronts would have 99
+    sums for 168 registers; all before the order of the sums' rounds and the searched rows). The
+    limits of 112 sums and of 80 for the shorter segments are set by that one mechanism and have no
+    measurement on their far side; 100 species / 2,200 reactions (89 sums) takes the same shape."""
     fits = lambda p: lds_bytes(p['em'].N, p['rows'], p['waves'], p['tight']) <= LDS_MAX
     most = lambda p: max(len(s) for s in p['sums'])
     p8 = plan(t, info)
@@ -269,10 +271,12 @@ def shape(t, info):
 
 
 def pays(t, info):
-    """The shape if a mechanism's reactions are split, else None. A state's modelled load has to be worth the
-    barriers and the per-wavefront prologue: 9 species / 21 reactions (5,000 cycles) run
-    1,048,576 states in 56 us with one wavefront per 64 states and 132 split; 31 / 203
-    (41,000) in 1,234 and 423. The line lies between, at 16,000."""
+    """The shape if a mechanism's reactions are split, else None. A state's modelled load has to be
+    worth the barriers and the per-wavefront prologue. 1,048,576 states, one wavefront per 64 states
+    -> split, FP64 (mixed): load 7,000 (10 species / 15 reactions) 127 -> 191 us (77 -> 161), 8,700
+    (10 / 22) 191 -> 216 (124 -> 194), 12,300 (11 / 30) 226 -> 264 (122 -> 213), 17,100 (12 / 40) 284
+    -> 273 (223 -> 206), 24,000 (14 / 60) 457 -> 337 (478 -> 245), 42,100 (20 / 100) 2,061 -> 555
+    (1,826 -> 370). The line lies at 16,000."""
     em = E._RateEmitter(t, info)
     if sum(reaction_cost(em, r) for r in range(em.R)) < 16000:
         return None

@@ -1,8 +1,9 @@
 """FP64 transport with four lanes per state: kx_bk2_fp64, kx_bk2_fp64_pstate and the
 surrogate's kx_bk2_fp64_queue on the wave-level routine of csrc/kx_bk2_quad.h.
 
-This module builds the routine's table (one FP64 __device__ array per mechanism, staged in
-LDS by each workgroup) and emits the kernels around it. With NB = ceil(N / 4) slots of four
+This module builds the routine's table (one FP64 __device__ array per mechanism; each workgroup
+stages it in LDS, the whole of it up to 72 species, else the species part, with the pair rows
+streamed through two row buffers) and emits the kernels around it. With NB = ceil(N / 4) slots of four
 species and one block (m, j) per slot pair j <= m, the table holds, in this order:
 
   rows m = 0 .. NB - 1, each fitA then fitC of its m + 1 blocks:
@@ -163,10 +164,13 @@ def table(t):
 
 def fits(t):
     """Whether a mechanism takes this family, with its whole table in LDS. N >= 20: below, the
-    4-fold repeated per-state work (T powers, divides) outweighs the shared pairs -- 1,048,576
-    states of 9 species: 144 us against 69 for one state per lane, of 31 species: 422 against
-    598, of 53: 910 against 1,861; the two cost curves in N cross near 18. At the other end the
-    table has to fit the 160 KB of a CU's LDS (N <= 72)."""
+    4-fold repeated per-state work (T powers, divides) and padding species outweigh the shared
+    pairs. 1,048,576 states of subsets of GRI-3.0, one state per lane -> this: 16 species 208 -> 207
+    us, 18 249 -> 289, 19 269 -> 290, 20 313 -> 292, 21 (three padding species) 343 -> 355, 22 381 ->
+    345, 24 429 -> 347, 32 668 -> 483; 9 species 69 -> 144, 53 1,861 -> 910. Calls of 100,003 states
+    and fewer are faster from 16 species on (20: 41 -> 35 us, 1,000 states 34 -> 10), and a line by
+    calls would need both kernels in every code object. At the other end the table has to fit the 160
+    KB of a CU's LDS (N <= 72)."""
     return int(t['n_species']) >= 20 and lds_bytes(t) <= LDS_MAX
 
 

@@ -946,11 +946,10 @@ def _emit_conductivity(S, t):
 def _emit_bk2_fp64(t, info, pstate=False, block=BLOCK):
     """pstate=False: kx_bk2_fp64, scalar p (the reference's transport kernel).
     pstate=True: kx_bk2_fp64_pstate, p [Pa] per state, also writes D_km.
-    block: threads per workgroup (the host launches with the kernel's launch bound). The
-    kernel's LDS constant pool (~85 KB for GRI-3.0) admits one workgroup per CU, so 512
-    threads (8 waves) is what gives 2 waves/SIMD: 8.4 ms instead of 14.5 at 256 threads for
-    4M states, despite ~160 VGPRs spilled to scratch; 768 and 1024 spill far more and are
-    2-3x slower."""
+    One state per lane, straight-line: for mechanisms below 20 species (emit_bk2_quad.fits).
+    block: threads per workgroup (the host launches with the kernel's launch bound). Chosen at 53
+    species, where the LDS constant pool (85 KB) admits one workgroup per CU: 512 threads 8.4 ms
+    for 4,194,304 states, 256 14.5, 768 and 1,024 2-3x slower (spills)."""
     N = int(t['n_species'])
     S = _Src()
     S(f'extern "C" __global__ void __launch_bounds__({block})', 0)
@@ -1114,11 +1113,13 @@ def generate(tables, info, opts=None):
         # large mechanism: no code that unrolls the pairs or keeps a state's species in registers,
         # no MFMA-accumulation variant and no surrogate (its width is fixed at 64)
         # production rates: straight-line reactions split over a workgroup's wavefronts where the
-        # species' rows fit the LDS (129 species / 1,231 reactions, 100,003 states: 238 us against
+        # species' rows fit the LDS (129 species / 1,231 reactions, 100,003 states: 244 us against
         # 1,732 in loop form; 160 / 1,000, 524,288 states: 1,825 against 5,340); beyond that, or
-        # asked for (rolled), several lanes per state over a reaction loop (emit_coop). Code and
-        # compile time grow with the reactions (1,231: 0.5 MB, 29 s; 1,000 with fewer shared terms:
-        # 0.8 MB, 54 s): past 2,000 the loop stays
+        # asked for (rolled), several lanes per state over a reaction loop (emit_coop). The limit of
+        # 2,000 reactions is one of generation time, not of speed: 1,231 plan and compile in half a
+        # minute, 1,000 of 160 species in 21 + 48 s, 2,500 of 150 search for two minutes and find no
+        # shape; where one is found the split stays ahead (100 / 2,200, 100,003 states: 573 us
+        # against 2,899)
         from . import emit_bk1_split as SP
         from . import emit_coop
         split = None if o.get('rolled') or int(tables['n_reactions']) > 2000 else SP.pays(tables, info)
