@@ -124,10 +124,11 @@ int kx_mixture_avg_transport(kx_mech_t m, int n_states, int offsetT, int offset,
                              double *d_conductivity, double *d_rhoD, void *stream);
 
 /* Same arguments, outputs and FP64 arithmetic as kx_mixture_avg_transport, with the O(N^2)
- * Wilke viscosity sum (kinetix_viscosity, mix_transport.py:337-345) computed as three GEMMs
- * (C1^2, 2 C1 C2, C2^2 against x_j, x_j/eta_j, x_j/eta_j^2) on FP64 MFMA
- * (v_mfma_f64_16x16x4_f64) over the states of each wavefront. Straight-line mechanisms only
- * (KX_ERR_NO_KERNEL for the loop-form ones). */
+ * Wilke viscosity sum (kinetix_viscosity, mix_transport.py:337-345) on FP64 MFMA
+ * (v_mfma_f64_16x16x4_f64) over the states of each wavefront: from 20 species on the kernel of
+ * kx_mixture_avg_transport, which has it so; below, three GEMMs (C1^2, 2 C1 C2, C2^2 against
+ * x_j, x_j/eta_j, x_j/eta_j^2). Mechanisms up to 96 species, not in loop form
+ * (KX_ERR_NO_KERNEL for the others). */
 int kx_mixture_avg_transport_mfma(kx_mech_t m, int n_states, int offsetT, int offset,
                                   double pressure, const double *d_state, double *d_viscosity,
                                   double *d_conductivity, double *d_rhoD, void *stream);

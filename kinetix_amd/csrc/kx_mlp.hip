@@ -1,8 +1,9 @@
 // Hand-written kernels of the transport-surrogate MLP: 64 -> kH -> kH -> kH -> 64 (kH = 256)
 // (55 inputs / 55 outputs zero-padded to 64), GELU (tanh form) on the hidden layers.
 //
-// Training (FP32 master weights): tiled FP32 GEMM with either operand transposed, bias +
-// GELU forward, GELU backward, masked-MSE gradient, bias-gradient reduction, Adam.
+// Training (FP32 master weights): FP32-MFMA GEMMs with the bias, GELU and GELU's derivative in their
+// epilogues, weight and bias gradients of a layer in one launch with the gradient handed down,
+// masked-MSE gradient, Adam.
 // Inference: BF16 weights packed into MFMA fragment order (kx_mlp_wave.h) and the
 // wave-level forward pass of kx_mlp_wave.h, 64 states per wavefront.
 //

@@ -31,7 +31,7 @@ Large mechanisms (shape) have one workgroup per CU; where the rows fill the LDS 
 partial sums share them, the NASA-7 table stays in global memory and a third body's C_k is w_k
 rg_k. Before, a loop over reaction descriptors with a state's species shared by 32 lanes (LDS
 gathers and atomics, 160+ instructions a reaction; here 26 to 56, as constants are in the code and
-equal exponentials are shared): 129 species / 1,231 reactions, 100,003 states FP64 1,732 -> 244
+equal exponentials are shared): 129 species / 1,231 reactions, 100,003 states FP64 1,732 -> 246
 us, mixed 1,310 -> 211, 1,000 states 1,253 -> 30; 160 / 1,000, 524,288 states 5,340 -> 1,825,
 mixed 4,164 -> 1,469, 1,000 states 1,298 -> 50. Of a group's 133,000 cycles at 160 / 1,000,
 loading Y takes 13,000 (nothing beside it hides that), the species 20,000, the reactions

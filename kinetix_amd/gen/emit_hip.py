@@ -1113,7 +1113,7 @@ def generate(tables, info, opts=None):
         # large mechanism: no code that unrolls the pairs or keeps a state's species in registers,
         # no MFMA-accumulation variant and no surrogate (its width is fixed at 64)
         # production rates: straight-line reactions split over a workgroup's wavefronts where the
-        # species' rows fit the LDS (129 species / 1,231 reactions, 100,003 states: 244 us against
+        # species' rows fit the LDS (129 species / 1,231 reactions, 100,003 states: 246 us against
         # 1,732 in loop form; 160 / 1,000, 524,288 states: 1,825 against 5,340); beyond that, or
         # asked for (rolled), several lanes per state over a reaction loop (emit_coop). The limit of
         # 2,000 reactions is one of generation time, not of speed: 1,231 plan and compile in half a

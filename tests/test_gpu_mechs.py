@@ -1,7 +1,7 @@
 """The reference's other mechanisms on the GPU, through the C ABI, against the oracle:
 LiDryer (9 species), NH3Konnov_edit (36, 3 PLOG reactions), chempolimi_edit (31, 21 PLOG),
 both straight-line, NH3Konnov_edit in the loop form too, EtOHKonnov (129 species, 1,231
-reactions, loop form), and the seeded 40-species coverage mechanism (kinetix_amd/synth.py
+reactions: split straight-line rates, streamed transport), and the seeded 40-species coverage mechanism (kinetix_amd/synth.py
 --coverage: every reaction form, incl. SRI, Lindemann, explicit colliders, irreversible
 reactions and PLOG points with summed rates) in both forms. BK1 FP64 <= 1e-12 of the reaction flux each output sums (forward
 and reverse separately) at pressures below, on, between and above the PLOG points; BK1 mixed <= 1e-5 relative L2 per species; BK2 and the
