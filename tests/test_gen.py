@@ -359,16 +359,21 @@ def _queue_kernel_numpy(t, s, p):
     return cond, mu, rhoD, Dkm
 
 
-def test_cooperative_queue_kernel_arithmetic_vs_oracle(gri, oracle):
+@pytest.mark.parametrize('mech', ['LiDryer', 'gri30'])
+def test_cooperative_queue_kernel_arithmetic_vs_oracle(mech):
     """The queue kernel's table layout and formulas against the oracle's FP64 transport with
-    per-state pressure; a transposed Wilke table or a wrong pair index fails by far more."""
+    per-state pressure, for a mechanism that ships this kernel and on larger tables; a transposed
+    Wilke table or a wrong pair index fails by far more."""
     from kinetix_amd import states
     from kinetix_amd.gen import emit_bk2_queue as BQ
-    info, t = gri
+    from kinetix_amd.gen import tables as tb
+    from oracle import pyoracle as po
+    info, t = tb.load(os.path.join(os.path.dirname(MDIR), mech))
     assert BQ.lds_bytes(t) <= 160 * 1024
-    s, p = states.sample_transport_set(64, info['species'], t['W'], seed=21)
+    s, p = states.sample_any(64, info['species'], t['W'], T_range=(300.0, 2500.0), seed=21,
+                             p_range_atm=(0.5, 40.0))
     got = _queue_kernel_numpy(t, s, p)
-    ref = oracle.transport(s, 1.0, 1.0, p_state=p)
+    ref = po.Oracle(t).transport(s, 1.0, 1.0, p_state=p)
     for g, r in zip(got, ref):
         assert np.max(np.abs(g / r - 1)) < 1e-12
     # the check has teeth: C1 transposed moves mu by far more than the tolerance
